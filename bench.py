@@ -146,7 +146,7 @@ def operator_roofline(table, grid, traffic=None):
     nbytes = (KERNEL_BYTES["apply_w"] + KERNEL_BYTES["apply_self"]) * P
     achieved = nbytes / (t * 1e-3) / 1e9
     return {
-        "kernel": "k_apply<16, 16, 32, 1, false> + k_apply<16, 16, 32, 2, false> (the two operator launches "
+        "kernel": "k_apply<false, 1, false> + k_apply<false, 2, false> (the two operator launches "
                   "of a BiCGstab iteration)",
         "bound": "hbm",
         "achieved": achieved,

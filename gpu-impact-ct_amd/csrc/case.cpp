@@ -228,7 +228,25 @@ int upload_coeffs(ih_case *c) {
     // SoA layout: per direction 10 arrays of up to 7 taps plus cdg (3 taps) and coordinates
     std::vector<double> h;
     std::vector<int64_t> off_G(3), off_Ip(3), off_D(3), off_Iu(3), off_NpD(3), off_NpU(3), off_NuD(3), off_NuU(3),
-        off_p2(3), off_u2(3), off_dg(3), off_xp(3), off_xu(3);
+        off_p2(3), off_u2(3), off_dg(3), off_xp(3), off_xu(3), off_G6(3), off_D6(3);
+    // the taps of a position together, positions -COEF6_LEAD .. N + COEF6_TAIL
+    auto push6 = [&](const std::vector<double> &src, int d, int lo, int hi) -> int64_t {
+        const int64_t o = (int64_t)h.size();
+        const int N = g.N[d], P = g.Np[d] - g.Sp[d] + 1;
+        h.resize(h.size() + 6 * (size_t)(N + COEF6_LEAD + COEF6_TAIL + 1), 0.0);
+        for (int pos = -COEF6_LEAD; pos <= N + COEF6_TAIL; ++pos) {
+            int i = pos;
+            if (g.per[d]) {
+                while (i < g.Sp[d]) i += P;
+                while (i > g.Np[d]) i -= P;
+            } else if (pos < lo || pos > hi) {
+                continue;
+            }
+            for (int t = 0; t < 6; ++t)
+                h[(size_t)o + 6 * (size_t)(pos + COEF6_LEAD) + (size_t)t] = src[(size_t)t + 6 * (size_t)i];
+        }
+        return o;
+    };
     auto push = [&](const std::vector<double> &src, int taps, int cst, int N, bool is_dg) -> int64_t {
         const int64_t o = (int64_t)h.size();
         h.resize(h.size() + (size_t)taps * cst, 0.0);
@@ -255,6 +273,8 @@ int upload_coeffs(ih_case *c) {
         off_p2[d] = push(hc.p2[d], 7, cst, N, false);
         off_u2[d] = push(hc.u2[d], 7, cst, N, false);
         off_dg[d] = push(hc.dg[d], 3, cst, N, true);
+        off_G6[d] = push6(hc.G[d], d, 1, N - 1);
+        off_D6[d] = push6(hc.D[d], d, 1, N);
         off_xp[d] = (int64_t)h.size();
         h.insert(h.end(), c->hg.xp[d].begin(), c->hg.xp[d].end());
         off_xu[d] = (int64_t)h.size();
@@ -290,6 +310,8 @@ int upload_coeffs(ih_case *c) {
         c->c.u2[d] = c->dcoef + off_u2[d];
         c->c.dg[d] = c->dcoef + off_dg[d];
         c->c.dgf[d] = c->dcoef32 + off32[d];
+        c->c.G6[d] = c->dcoef + off_G6[d];
+        c->c.D6[d] = c->dcoef + off_D6[d];
         c->c.xp[d] = c->dcoef + off_xp[d];
         c->c.xu[d] = c->dcoef + off_xu[d];
     }

@@ -43,10 +43,17 @@ struct Coef {
     const double *u2[3];   // cu11..
     const double *dg[3];   // cdg: 3 taps (lo -1), index i = 1..N
     const float *dgf[3];   // cdg in FP32 for the mixed-precision sweep
+    // G and D once more, the six taps of a position together: entry t of position
+    // pos at [6*(pos + COEF6_LEAD) + t], pos from -COEF6_LEAD to N + COEF6_TAIL.
+    // Positions past a periodic pair hold the wrapped position's taps; G outside
+    // its wall range 1..N-1 and D outside 1..N hold zeros.
+    const double *G6[3], *D6[3];
     const double *xp[3];   // coordinates (-3:N+3) at [i+3]
     const double *xu[3];
     const double *zero;    // 64 doubles of 0.0, never written: the load source for positions outside the field
 };
+
+constexpr int COEF6_LEAD = 8, COEF6_TAIL = 40;
 
 // Reduction tree constants, shared with the oracle's restatement: blocks of
 // RED_TX x RED_TY threads over (i, j); along k the range is cut into

@@ -23,6 +23,7 @@
 #include "ih_krylov.h"
 #include "ih_mg.h"
 
+#include <type_traits>
 #include <utility>
 
 namespace ih {
@@ -88,27 +89,375 @@ __device__ inline bool wall_z(const Geo &g, int idx) {
 // dot modes of k_apply
 enum { DOT_NONE = 0, DOT_W = 1, DOT_SELF = 2, DOT_PAIR = 3 };
 
-// One thread per (x, y) column of a TX x TY tile, the planes of one z chunk
-// (balanced chunks of at most AZ planes, the reduction chunks).  Pressure cross
-// and gradient tiles are double buffered, and the divergence of plane k-1 is
-// formed after the gradients of plane k, so each plane costs one barrier.  The
-// halo of plane k+2, p(k+7) of the column queue and w(k+1) are loaded while
-// planes k and k+1 are computed (the plane loop is unrolled twice so that the
-// two register sets alternate).  The gradient coefficients of a thread's
-// positions stay in registers for the whole chunk; every thread forms one G_1,
-// one G_2 and at most one halo gradient per plane without divergent branches.
+// Two forms of the operator on a 16 x 16 column tile marching through a z chunk.
+//
+// Teams (apply_teams): two teams of 256 threads, one thread of each team per
+// (x, y) column:
+//   team 0 stages the halo of the pressure cross and forms the G_1 and G_2 values
+//   of the tile and its halo from the staged plane;
+//   team 1 stages the tile's own pressures, keeps p and G_3 of its column in
+//   register queues along z, and forms the divergence from the gradient tiles.
+// Cross and gradient tiles are double buffered: between two barriers team 0 forms
+// the gradients of plane k while team 1 forms the divergence of plane k-1, so a
+// plane costs one barrier and each team about half of its instructions.
+//
+// Column (apply_column): one thread per column does all of a plane.
+//
+// What bounds them: where the tiles do not fill the compute units (65^3 has 75) the
+// chain of one plane, barrier to barrier, which the teams halve; beyond two tiles a
+// compute unit LDS and FP64 issue, each about 40 % busy at 257x129x129, which the
+// waves' waits keep from overlapping further, and there two teams (8 wavefronts, two
+// blocks a compute unit) gain nothing over three blocks of 4 wavefronts.  Operator
+// with <Ap, w>, teams against column: 14.0 / 20.5 us at 33x17x17, 17.3 / 25.7 at
+// 65^3, 28.8 / 36.7 at 193x97x97; a whole BiCGstab iteration 108.7 / 122.2 us at
+// 193x97x97 (364 tiles), 177.8 / 177.3 at 257x129x129 (765), 603.5 / 596.7 at
+// 385x193x193 (2275): teams up to two tiles a compute unit, column beyond.
+// Measured and not taken: segments of four points a thread in each direction in
+// turn with all coefficients scalar (9/4 gradients a point, bound by VALU: 48 us
+// at 257x129x129 against 45); the teams at 80 VGPRs for three blocks (spills).
+constexpr int64_t APPLY_TEAM_TILES = 512;
+constexpr int APPLY_THREADS = 2 * RED_TX * RED_TY;
+
+// Keeps the compiler to the order written: nothing moves across.
+__device__ inline void pin() { __builtin_amdgcn_sched_barrier(0); }
+
+// Loaded values that a loop only reads: waited for here, before the loop.  (With
+// their loads possibly still in flight at its head, the first use in the loop
+// would wait, every trip, for everything in flight, the prefetches included.)
+template <int N>
+__device__ inline void arrive(double (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
+
+using cdbl = const __attribute__((address_space(4))) double;
+
+// the tables of direction d from position pos on (six taps a position)
+__device__ inline cdbl *row6(const double *t, int pos) { return (cdbl *)(t + 6 * (pos + COEF6_LEAD)); }
+
 // DM = DOT_W accumulates <Ap, w>, DOT_SELF <p, Ap> and <Ap, Ap>, DOT_PAIR
-// <w, Ap> and <Ap, Ap>, per
-// thread in plane order, then over the block with the fixed tree.
-// The bound asks for 3 wavefronts per SIMD (at most 168 VGPRs): the pair-dot
-// form otherwise takes 170, which the 8-register allocation rounds to 176, and
-// runs at 2 wavefronts per SIMD, 40% slower.
-// The block function of tile (bx, by, bz); k_apply and the batched operator
-// (k_apply_batch) both run it, so a batched case is bit-identical to its own launch.
-template <int TX, int TY, int AZ, int DM, bool PZ>
-__device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r, int nbx, int nby, int nbz, int bx,
-                                   int by, int bz, const double *__restrict__ src, double *__restrict__ dst,
+// <w, Ap> and <Ap, Ap>, per column in plane order over the planes kc0..kc1 (a
+// reduction chunk), then over the tile with the fixed tree into entry pi.
+// The block functions of one tile serve the single-case and the batched kernels, and
+// both forms give the same bits, so a batched case is bit-identical to its own launch.
+template <int DM, bool PZ>
+__device__ inline void apply_teams(const Geo &g, const Coef &c, const Range3 &r, int bx, int by, int kc0, int kc1,
+                                   int64_t pi, const double *__restrict__ src, double *__restrict__ dst,
                                    const double *__restrict__ w, double *part1, double *part2) {
+    constexpr int TX = RED_TX, TY = RED_TY, NT = TX * TY;
+    constexpr int PW = TX + 10, PH = TY + 10, PS = PW * PH;
+    constexpr int NHX = 10 * TY, NH = NHX + 10 * TX;  // halo positions of a plane
+    constexpr int NG1X = 5 * TY, NG2X = 5 * TX;
+    static_assert(NG1X + NG2X <= NT && NH - NT == 64 && NT == 256, "one halo gradient per thread, the last 64 halo loads");
+    constexpr int G1S = TX + 5;                  // row stride of the G_1 tile
+    constexpr int OG2 = TY * G1S;                // offset of the G_2 tile
+    constexpr int GS = OG2 + (TY + 5) * TX;
+    __shared__ double sP[2][PS];
+    __shared__ double sG[2][GS + 1];
+    __shared__ double sm[8];
+
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int tid = tx + TX * ty;
+    const int team = __builtin_amdgcn_readfirstlane((int)threadIdx.z);
+    const int x0 = r.lo0 + bx * TX, y0 = r.lo1 + by * TY;
+    const int x = x0 + tx, y = y0 + ty;
+    const int xe = r.lo0 + r.n0 - 1, ye = r.lo1 + r.n1 - 1;
+    const int64_t pxy = g.pxy;
+    // A load outside the field reads some element of its plane instead and its
+    // value is replaced by zero where it is used, planes later (a select at the load
+    // would make the wave wait for it at once).  Bases are uniform, offsets 32-bit.
+    const double *hb = src + gidx(g, -3, -3, 0);
+    double acc1 = 0.0, acc2 = 0.0;
+
+    if (team == 0) {
+        const int c0 = g.cst[0], c1 = g.cst[1];
+        const int b1 = (ty + 5) * PW + tx, w1 = ty * G1S + tx;     // G_1 at x0-3+tx, row ty
+        const int b2 = ty * PW + tx + 5, w2 = OG2 + ty * TX + tx;  // G_2 at y0-3+ty, column tx
+        int p1 = x0 - 3 + tx;
+        const bool v1 = p1 <= xe + 2 && g_src(g, 0, p1) && !wall_plane(g, 1, y);
+        int p2 = y0 - 3 + ty;
+        const bool v2 = p2 <= ye + 2 && g_src(g, 1, p2) && !wall_plane(g, 0, x);
+        double cg1[6], cg2[6];
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            cg1[s] = v1 ? c.G[0][s * c0 + p1] : 0.0;
+            cg2[s] = v2 ? c.G[1][s * c1 + p2] : 0.0;
+        }
+        arrive(cg1);
+        arrive(cg2);
+        // position e of the plane's halo: its place in the cross and in the field
+        auto halo_at = [&](int e, int &slot, unsigned &off) -> bool {
+            int hx, hy;
+            if (e < NHX) {
+                const int row = e / 10, cc = e % 10;
+                const int col = cc < 5 ? cc : TX + cc;
+                hx = x0 - 5 + col;
+                hy = y0 + row;
+                slot = (row + 5) * PW + col;
+            } else {
+                const int rr = (e - NHX) / TX, col = (e - NHX) % TX;
+                const int row = rr < 5 ? rr : TY + rr;
+                hx = x0 + col;
+                hy = y0 - 5 + row;
+                slot = row * PW + col + 5;
+            }
+            const bool v = hx <= xe + 5 && hy <= ye + 5 && p_src(g, 0, hx) && p_src(g, 1, hy);
+            off = v ? (unsigned)(gidx(g, hx, hy, 0) - gidx(g, -3, -3, 0)) : 0u;
+            return v;
+        };
+        // Three wavefronts form a halo gradient each thread (the last 32 threads of
+        // the third none), the fourth loads the 64 halo positions left over instead:
+        // a loop of its own for each, so that neither holds the other's registers.
+        auto march = [&](auto job_) {
+            constexpr bool JOB = decltype(job_)::value;
+            constexpr int NL = JOB ? 1 : 2;
+            unsigned hoff[NL];
+            int hslot[NL];
+            bool hval[NL];
+            hval[0] = halo_at(tid, hslot[0], hoff[0]);
+            if constexpr (!JOB) hval[1] = halo_at(NT + (tid & 63), hslot[1], hoff[1]);
+            auto load_halo = [&](int kk, double (&hv)[NL]) {
+                const double *b = hb + (int64_t)(kk <= kc1 ? kk : kc1) * pxy;  // planes past the chunk are not staged
+#pragma unroll
+                for (int h = 0; h < NL; ++h) hv[h] = b[hoff[h]];
+            };
+            auto stage_halo = [&](double *P, const double (&hv)[NL]) {
+#pragma unroll
+                for (int h = 0; h < NL; ++h) P[hslot[h]] = hval[h] ? hv[h] : 0.0;
+            };
+            // halo gradient: LDS base, stride, destination and coefficients
+            double cgx[6];
+            int bxj = 0, sxj = 1, wxj = GS;  // GS: a slot past the tiles for the threads without one
+            bool vx = false;
+            if constexpr (JOB) {
+                const double *cx = c.G[0];
+                int cix = 0, cstx = c0;
+                if (tid < NG2X) {
+                    const int c2x = tid % TX, v2r = TY + tid / TX;
+                    int py_ = y0 - 3 + v2r;
+                    vx = py_ <= ye + 2 && g_src(g, 1, py_) && !wall_plane(g, 0, x0 + c2x);
+                    cx = c.G[1];
+                    cix = py_;
+                    cstx = c1;
+                    bxj = v2r * PW + c2x + 5;
+                    sxj = PW;
+                    wxj = OG2 + v2r * TX + c2x;
+                } else if (tid < NG2X + NG1X) {
+                    const int e1 = tid - NG2X;
+                    const int r1x = e1 / 5, u1x = TX + e1 % 5;
+                    int px_ = x0 - 3 + u1x;
+                    vx = px_ <= xe + 2 && g_src(g, 0, px_) && !wall_plane(g, 1, y0 + r1x);
+                    cix = px_;
+                    bxj = (r1x + 5) * PW + u1x;
+                    wxj = r1x * G1S + u1x;
+                }
+#pragma unroll
+                for (int s = 0; s < 6; ++s) cgx[s] = vx ? cx[s * cstx + cix] : 0.0;
+                arrive(cgx);
+            }
+            double hvA[NL], hvB[NL];
+            load_halo(kc0, hvA);
+            pin();
+            load_halo(kc0 + 1, hvB);
+            // the gradients of plane k, then the halo of plane k+1 and the load of plane k+2's
+            auto body = [&](int k, int buf, double (&hv)[NL], double (&hnext)[NL]) {
+                __syncthreads();
+                load_halo(k + 2, hv);
+                const bool zk = wall_z<PZ>(g, k);
+                const double *P = sP[buf];
+                double *G = sG[buf];
+                double pa[6], pb[6], pe[6];
+#pragma unroll
+                for (int s = 0; s < 6; ++s) pa[s] = P[b1 + s];
+#pragma unroll
+                for (int s = 0; s < 6; ++s) pb[s] = P[b2 + s * PW];
+                if constexpr (JOB) {
+#pragma unroll
+                    for (int s = 0; s < 6; ++s) pe[s] = P[bxj + s * sxj];
+                }
+                pin();
+                double a = cg1[0] * pa[0], b = cg2[0] * pb[0], e = JOB ? cgx[0] * pe[0] : 0.0;
+#pragma unroll
+                for (int s = 1; s < 6; ++s) {
+                    a = a + cg1[s] * pa[s];
+                    b = b + cg2[s] * pb[s];
+                    if (JOB) e = e + cgx[s] * pe[s];
+                }
+                G[w1] = (v1 && !zk) ? a : 0.0;
+                G[w2] = (v2 && !zk) ? b : 0.0;
+                if constexpr (JOB) G[wxj] = (vx && !zk) ? e : 0.0;
+                stage_halo(sP[buf ^ 1], hnext);  // past the chunk: written and not read
+            };
+            stage_halo(sP[0], hvA);
+            for (int k = kc0;;) {
+                body(k, 0, hvA, hvB);
+                if (++k > kc1) break;
+                body(k, 1, hvB, hvA);
+                if (++k > kc1) break;
+            }
+        };
+        if (__builtin_amdgcn_readfirstlane(tid >> 6) < 3)
+            march(std::true_type{});
+        else
+            march(std::false_type{});
+        __syncthreads();
+    } else {
+        const bool own = (x <= xe) && (y <= ye);
+        int xs = x, ys = y;
+        const bool vcol = x <= xe + 5 && y <= ye + 5 && p_src(g, 0, xs) && p_src(g, 1, ys);
+        const unsigned colo = vcol ? (unsigned)(gidx(g, xs, ys, 0) - gidx(g, -3, -3, 0)) : 0u;
+        const unsigned selfo = own ? (unsigned)(gidx(g, x, y, 0) - gidx(g, -3, -3, 0)) : 0u;
+        double *const db = dst + gidx(g, -3, -3, 0);
+        const double *const wb = DM == DOT_W || DM == DOT_PAIR ? w + gidx(g, -3, -3, 0) : nullptr;
+        const bool g3on = own && !(wall_plane(g, 0, x) || wall_plane(g, 1, y));
+        const int gz_lo = PZ ? kc0 - 4 : 1, gz_hi = PZ ? kc1 + 4 : g.N[2] - 1;
+        // p of the own column at plane kk (at most kc1 + 5), and whether the field has it
+        auto col_ok = [&](int &kk) { return p_src_z<PZ>(g, kk); };
+        auto load_col = [&](int kk) -> double {
+            kk = kk <= kc1 + 5 ? kk : kc1 + 5;
+            return hb[(int64_t)(col_ok(kk) ? kk : kc1) * pxy + colo];
+        };
+        auto load_w = [&](int kk) -> double {
+            if (DM != DOT_W && DM != DOT_PAIR) return 0.0;  // w is only a valid pointer in these modes
+            return wb[(int64_t)(kk <= kc1 ? kk : kc1) * pxy + selfo];
+        };
+        // at the divergence of plane k: q = p(k .. k+5), g3 = G_3(k-3 .. k+2)
+        const int c0 = g.cst[0], c1 = g.cst[1];
+        double q[6], g3[6], cd1[6], cd2[6], pz[11];
+#pragma unroll
+        for (int s = 0; s < 11; ++s) pz[s] = load_col(kc0 - 5 + s);
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            cd1[s] = own ? c.D[0][s * c0 + x] : 0.0;
+            cd2[s] = own ? c.D[1][s * c1 + y] : 0.0;
+        }
+        {
+            cdbl *Gz = row6(c.G6[2], kc0 - 3);
+#pragma unroll
+            for (int s = 0; s < 11; ++s) {
+                int kk = kc0 - 5 + s;
+                pz[s] = vcol && col_ok(kk) ? pz[s] : 0.0;
+            }
+            sP[0][(ty + 5) * PW + tx + 5] = pz[5];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) {
+                double v = Gz[6 * t] * pz[t];
+#pragma unroll
+                for (int s = 1; s < 6; ++s) v = v + Gz[6 * t + s] * pz[t + s];
+                const int kk = kc0 - 3 + t;
+                g3[t] = (g3on && kk >= gz_lo && kk <= gz_hi) ? v : 0.0;
+            }
+#pragma unroll
+            for (int s = 0; s < 6; ++s) q[s] = pz[5 + s];
+        }
+        arrive(cd1);
+        arrive(cd2);
+        double pA = load_col(kc0 + 6), wA = load_w(kc0);
+        pin();
+        double pB = load_col(kc0 + 7), wB = load_w(kc0 + 1);
+        // the z coefficients of a plane: G_3 at k+3, then D_3 at k
+        double cz[12];
+        auto load_cz = [&](int k) {
+            cdbl *Gz = row6(c.G6[2], k + 3), *Dz = row6(c.D6[2], k);
+#pragma unroll
+            for (int s = 0; s < 6; ++s) {
+                cz[s] = Gz[s];
+                cz[6 + s] = Dz[s];
+            }
+        };
+        load_cz(kc0);
+        // the divergence of plane k (its gradients are in sG[buf]), staging p of plane k+2
+        auto body = [&](int k, int buf, double &pn, double &wv) {
+            __syncthreads();
+            double G1[6], G2[6];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) G1[t] = sG[buf][ty * G1S + tx + t];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) G2[t] = sG[buf][OG2 + (ty + t) * TX + tx];
+            sP[buf][(ty + 5) * PW + tx + 5] = q[2];  // past the chunk: written and not read
+            pin();
+            // what was loaded two planes ago is taken over before this plane's store
+            // is issued: a wait for it would then be a wait for the store as well
+            const double q0 = q[0], wk = wv;
+#pragma unroll
+            for (int s = 0; s < 5; ++s) q[s] = q[s + 1];
+            int kn = k + 6;
+            q[5] = vcol && col_ok(kn) ? pn : 0.0;
+            double v = cz[0] * q[0];
+#pragma unroll
+            for (int s = 1; s < 6; ++s) v = v + cz[s] * q[s];
+            pn = load_col(k + 8);
+            wv = load_w(k + 2);
+            double lap = cd1[0] * G1[0];
+#pragma unroll
+            for (int t = 1; t < 6; ++t) lap = lap + cd1[t] * G1[t];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) lap = lap + cd2[t] * G2[t];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) lap = lap + cz[6 + t] * g3[t];
+#pragma unroll
+            for (int t = 0; t < 5; ++t) g3[t] = g3[t + 1];
+            asm volatile("" : "+v"(v));  // a select, not a branch around the sum
+            g3[5] = (g3on && k + 3 >= gz_lo && k + 3 <= gz_hi) ? v : 0.0;
+            pin();
+            load_cz(k + 1);
+            pin();
+            if (DM == DOT_W) {
+                acc1 = acc1 + (own ? lap * wk : 0.0);
+            } else if (DM == DOT_SELF) {
+                acc1 = acc1 + (own ? q0 * lap : 0.0);
+                acc2 = acc2 + (own ? lap * lap : 0.0);
+            } else if (DM == DOT_PAIR) {
+                acc1 = acc1 + (own ? wk * lap : 0.0);
+                acc2 = acc2 + (own ? lap * lap : 0.0);
+            }
+            if (own) db[(int64_t)k * pxy + selfo] = lap;
+        };
+        __syncthreads();  // plane kc0 is staged
+        sP[1][(ty + 5) * PW + tx + 5] = q[1];
+        // the loop leaves from between its two halves: with a way around the second
+        // one the first half's wait for its loads would be a wait for all loads
+        for (int k = kc0;;) {
+            body(k, 0, pA, wA);
+            if (++k > kc1) break;
+            body(k, 1, pB, wB);
+            if (++k > kc1) break;
+        }
+    }
+    if (DM != DOT_NONE) {
+        // the fixed tree over the tile, the partial sums of team 1
+        if (team == 1) {
+            const double s1 = wave_sum(acc1);
+            const double s2 = DM == DOT_W ? 0.0 : wave_sum(acc2);
+            if ((tid & 63) == 0) {
+                sm[tid >> 6] = s1;
+                sm[4 + (tid >> 6)] = s2;
+            }
+        }
+        __syncthreads();
+        if (team == 1 && tid == 0) {
+            part1[pi] = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+            if (DM == DOT_SELF || DM == DOT_PAIR) part2[pi] = (sm[4] + sm[5]) + (sm[6] + sm[7]);
+        }
+    }
+}
+
+// The column form: one thread per (x, y) column.  Pressure cross and gradient
+// tiles are double buffered, and the divergence of plane k-1 is formed after the
+// gradients of plane k, so each plane costs one barrier.  The halo of plane k+2,
+// p(k+7) of the column queue and w(k+1) are loaded while planes k and k+1 are
+// computed (the plane loop is unrolled twice so that the two register sets
+// alternate).  The gradient coefficients of a thread's positions stay in registers
+// for the whole chunk, those in z are scalar loads a plane ahead (from LDS they were
+// 13 of a plane's 45 LDS accesses: 600.5 against 596.7 us an iteration at
+// 385x193x193, 177.9 against 177.3 at 257x129x129); every thread forms one G_1, one
+// G_2 and at most one halo gradient per plane without divergent branches.
+// 3 wavefronts per SIMD (at most 168 VGPRs).
+template <int DM, bool PZ>
+__device__ inline void apply_column(const Geo &g, const Coef &c, const Range3 &r, int bx, int by, int kc0, int kc1,
+                                    int64_t pi, const double *__restrict__ src, double *__restrict__ dst,
+                                    const double *__restrict__ w, double *part1, double *part2) {
+    constexpr int TX = RED_TX, TY = RED_TY;
     constexpr int NT = TX * TY;
     constexpr int PW = TX + 10, PH = TY + 10, PS = PW * PH;
     constexpr int NHX = 10 * TY;
@@ -119,12 +468,8 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
     constexpr int G1S = TX + 5;                 // row stride of the G_1 tile
     constexpr int OG2 = TY * G1S;               // offset of the G_2 tile
     constexpr int GS = OG2 + (TY + 5) * TX + 1; // + one dummy slot
-    constexpr int ZW = AZ + 7;                  // G_3 positions kc0-4 .. kc0+AZ+2
     __shared__ double sP[2][PS];
     __shared__ double sG[2][GS];
-    __shared__ double sCG3[6][ZW];
-    __shared__ double sCD3[6][AZ];
-    __shared__ int sVZ[ZW];
     __shared__ double sm[8];
 
     const int tx = threadIdx.x, ty = threadIdx.y;
@@ -133,25 +478,11 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
     const int x = x0 + tx, y = y0 + ty;
     const int xe = r.lo0 + r.n0 - 1, ye = r.lo1 + r.n1 - 1;
     const bool own = (x <= xe) && (y <= ye);
-    int kc0, kc1;
-    red_chunk(r, bz, nbz, kc0, kc1);
-    const int c0 = g.cst[0], c1 = g.cst[1], c2 = g.cst[2];
+    const int c0 = g.cst[0], c1 = g.cst[1];
     const int64_t pxy = g.pxy;
     // loads outside the field read c.zero, so no value is masked after its load
     // (a select on the loaded value would make the wave wait for it at once)
     const double *zero = c.zero;
-
-    for (int e = tid; e < 6 * ZW; e += NT) {
-        const int s = e / ZW, u = e % ZW;
-        int kk = kc0 - 4 + u;
-        const bool v = kk <= kc1 + 2 && g_src_z<PZ>(g, kk);
-        sCG3[s][u] = v ? c.G[2][s * c2 + kk] : 0.0;
-        if (s == 0) sVZ[u] = v ? 1 : 0;
-    }
-    for (int e = tid; e < 6 * AZ; e += NT) {
-        const int t = e / AZ, u = e % AZ;
-        sCD3[t][u] = (kc0 + u <= kc1) ? c.D[2][t * c2 + kc0 + u] : 0.0;
-    }
 
     const int64_t hbase = gidx(g, -3, -3, 0);  // a valid element; offsets below are >= 0 from it
     int xs = x, ys = y;
@@ -227,7 +558,7 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
         }
     }
     const bool g3on = own && !(wall_plane(g, 0, x) || wall_plane(g, 1, y));
-    __syncthreads();
+    const int gz_lo = PZ ? kc0 - 8 : 1, gz_hi = PZ ? kc1 + 8 : g.N[2] - 1;
 
     // queue at iteration k: q = p(k-1 .. k+4), g3 = G_3(k-4 .. k+1)
     double q[6], g3[6];
@@ -239,12 +570,14 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
             const bool v = vcol && p_src_z<PZ>(g, kk);
             pz[s] = *(v ? src + colb + (int64_t)kk * pxy : zero);
         }
+        cdbl *Gz = row6(c.G6[2], kc0 - 4);
 #pragma unroll
         for (int t = 0; t < 6; ++t) {
-            double v = sCG3[0][t] * pz[t];
+            double v = Gz[6 * t] * pz[t];
 #pragma unroll
-            for (int s = 1; s < 6; ++s) v = v + sCG3[s][t] * pz[t + s];
-            g3[t] = (g3on && sVZ[t]) ? v : 0.0;
+            for (int s = 1; s < 6; ++s) v = v + Gz[6 * t + s] * pz[t + s];
+            const int kk = kc0 - 4 + t;
+            g3[t] = (g3on && kk >= gz_lo && kk <= gz_hi) ? v : 0.0;
         }
 #pragma unroll
         for (int s = 0; s < 6; ++s) q[s] = pz[5 + s];
@@ -272,6 +605,18 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
     double pA = load_col(kc0 + 5), pB = load_col(kc0 + 6);
     double wA = load_w(kc0), wB = load_w(kc0 + 1);
     double acc1 = 0.0, acc2 = 0.0;
+    // z coefficients of plane k's step, scalar operands loaded a plane ahead: G_3 at
+    // k+2, D_3 at k-1
+    double cz[12];
+    auto load_cz = [&](int k) {
+        cdbl *Gz = row6(c.G6[2], k + 2), *Dz = row6(c.D6[2], k - 1);
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            cz[s] = Gz[s];
+            cz[6 + s] = Dz[s];
+        }
+    };
+    load_cz(kc0);
 
     auto divergence = [&](int k, const double *G, double wv) {
         // plane k from the gradient tile G, g3 = G_3(k-3 .. k+2), q[0] = p(k)
@@ -280,9 +625,8 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
         for (int t = 1; t < 6; ++t) lap = lap + cd1[t] * G[ty * G1S + tx + t];
 #pragma unroll
         for (int t = 0; t < 6; ++t) lap = lap + cd2[t] * G[OG2 + (ty + t) * TX + tx];
-        const int kz = k - kc0;
 #pragma unroll
-        for (int t = 0; t < 6; ++t) lap = lap + sCD3[t][kz] * g3[t];
+        for (int t = 0; t < 6; ++t) lap = lap + cz[6 + t] * g3[t];
         if (own) dst[selfb + (int64_t)k * pxy] = lap;
         if (DM == DOT_W) {
             acc1 = acc1 + (own ? lap * wv : 0.0);
@@ -334,11 +678,13 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
         pn = load_col(k + 7);
 #pragma unroll
         for (int t = 0; t < 5; ++t) g3[t] = g3[t + 1];
-        const int u = k - kc0 + 6;  // G_3 position k+2
-        double v = sCG3[0][u] * q[0];
+        double v = cz[0] * q[0];
 #pragma unroll
-        for (int s = 1; s < 6; ++s) v = v + sCG3[s][u] * q[s];
-        g3[5] = (g3on && sVZ[u]) ? v : 0.0;
+        for (int s = 1; s < 6; ++s) v = v + cz[s] * q[s];
+        g3[5] = (g3on && k + 2 >= gz_lo && k + 2 <= gz_hi) ? v : 0.0;
+        pin();
+        load_cz(k + 1);
+        pin();
         (void)wcur;
     };
     // w(k-1) is consumed in iteration k: the A set serves even offsets k-kc0, the B set odd ones
@@ -353,7 +699,6 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
         divergence(kc1, sG[buf], buf == 0 ? wA : wB);
     }
     if (DM != DOT_NONE) {
-        const int64_t pi = (int64_t)bx + (int64_t)nbx * ((int64_t)by + (int64_t)nby * bz);
         const double s1 = block_sum(acc1, sm);
         __syncthreads();
         if (tid == 0) part1[pi] = s1;
@@ -364,14 +709,30 @@ __device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r,
     }
 }
 
-template <int TX, int TY, int AZ, int DM, bool PZ>
-__global__ __launch_bounds__(TX *TY, 3) void k_apply(
+template <bool TEAMS, int DM, bool PZ>
+__device__ inline void apply_block(const Geo &g, const Coef &c, const Range3 &r, int bx, int by, int bz, int nbz,
+                                   int64_t pi, const double *src, double *dst, const double *w, double *part1,
+                                   double *part2) {
+    int kc0, kc1;
+    red_chunk(r, bz, nbz, kc0, kc1);
+    if constexpr (TEAMS)
+        apply_teams<DM, PZ>(g, c, r, bx, by, kc0, kc1, pi, src, dst, w, part1, part2);
+    else
+        apply_column<DM, PZ>(g, c, r, bx, by, kc0, kc1, pi, src, dst, w, part1, part2);
+}
+
+constexpr int apply_threads(bool teams) { return teams ? APPLY_THREADS : RED_THREADS; }
+constexpr int apply_waves(bool teams) { return teams ? 4 : 3; }  // wavefronts per SIMD
+
+template <bool TEAMS, int DM, bool PZ>
+__global__ __launch_bounds__(apply_threads(TEAMS), apply_waves(TEAMS)) void k_apply(
     Geo g, Coef c, Range3 r, int nbx, int nby, int nbz, const double *__restrict__ src, double *__restrict__ dst,
     const double *__restrict__ w, double *part1, double *part2, const int *active) {
     if (active && !*active) return;
     int bx, by, bz;
     if (!xcd_tile(nbx, nby, nbz, bx, by, bz)) return;
-    apply_block<TX, TY, AZ, DM, PZ>(g, c, r, nbx, nby, nbz, bx, by, bz, src, dst, w, part1, part2);
+    const int64_t pi = (int64_t)bx + (int64_t)nbx * ((int64_t)by + (int64_t)nby * bz);
+    apply_block<TEAMS, DM, PZ>(g, c, r, bx, by, bz, nbz, pi, src, dst, w, part1, part2);
 }
 
 // ---------------------------------------------------------------------------
@@ -766,10 +1127,9 @@ __device__ inline int batch_tile(const KBatchCase *cases, const int *tile_case, 
     return q;
 }
 
-template <int DM, bool PZ>
-__global__ __launch_bounds__(RED_TX *RED_TY, 3) void k_apply_batch(const KBatchCase *__restrict__ cases,
-                                                                   const int *__restrict__ tile_case, int ntiles,
-                                                                   int form, int pre) {
+template <bool TEAMS, int DM, bool PZ>
+__global__ __launch_bounds__(apply_threads(TEAMS), apply_waves(TEAMS)) void k_apply_batch(
+    const KBatchCase *__restrict__ cases, const int *__restrict__ tile_case, int ntiles, int form, int pre) {
     int bx, by, bz;
     int64_t pi;
     const int q = batch_tile(cases, tile_case, ntiles, bx, by, bz, pi);
@@ -791,8 +1151,7 @@ __global__ __launch_bounds__(RED_TX *RED_TY, 3) void k_apply_batch(const KBatchC
         dst = K.Ar;
         w = K.rr;
     }
-    apply_block<RED_TX, RED_TY, RED_KC, DM, PZ>(K.g, K.c, K.r, K.nbx, K.nby, K.nbz, bx, by, bz, src, dst, w, K.part1,
-                                                K.part2);
+    apply_block<TEAMS, DM, PZ>(K.g, K.c, K.r, bx, by, bz, K.nbz, pi, src, dst, w, K.part1, K.part2);
 }
 
 // the first-sweep operands of a batched case
@@ -946,15 +1305,22 @@ void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, c
     if (empty(r)) return;
     // the operator tile is the reduction tile, so the fused dot partials follow the fixed tree
     const int nbx = (r.n0 + RED_TX - 1) / RED_TX, nby = (r.n1 + RED_TY - 1) / RED_TY, nbz = (r.n2 + RED_KC - 1) / RED_KC;
-    const dim3 grid(xcd_grid((int64_t)nbx * nby * nbz)), block(RED_TX, RED_TY, 1);
-#define IH_APPLY(DMV)                                                                                           \
-    do {                                                                                                        \
-        if (g.per[2])                                                                                           \
-            hipLaunchKernelGGL((k_apply<RED_TX, RED_TY, RED_KC, DMV, true>), grid, block, 0, s, g, c, r, nbx, nby, \
-                               nbz, src, dst, w, part1, part2, active);                                         \
-        else                                                                                                    \
-            hipLaunchKernelGGL((k_apply<RED_TX, RED_TY, RED_KC, DMV, false>), grid, block, 0, s, g, c, r, nbx,     \
-                               nby, nbz, src, dst, w, part1, part2, active);                                    \
+    const int64_t tiles = (int64_t)nbx * nby * nbz;
+    const bool teams = tiles <= APPLY_TEAM_TILES;
+    const dim3 grid(xcd_grid(tiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
+#define IH_APPLY_AS(T, DMV, PZV)                                                                               \
+    hipLaunchKernelGGL((k_apply<T, DMV, PZV>), grid, block, 0, s, g, c, r, nbx, nby, nbz, src, dst, w, part1, part2, \
+                       active)
+#define IH_APPLY(DMV)                         \
+    do {                                      \
+        if (teams && g.per[2])                \
+            IH_APPLY_AS(true, DMV, true);     \
+        else if (teams)                       \
+            IH_APPLY_AS(true, DMV, false);    \
+        else if (g.per[2])                    \
+            IH_APPLY_AS(false, DMV, true);    \
+        else                                  \
+            IH_APPLY_AS(false, DMV, false);   \
     } while (0)
     if (dot_mode == DOT_W)
         IH_APPLY(DOT_W);
@@ -965,6 +1331,7 @@ void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, c
     else
         IH_APPLY(DOT_NONE);
 #undef IH_APPLY
+#undef IH_APPLY_AS
 }
 
 void launch_krylov_init(hipStream_t s, const Geo &g, const Box &b, const double *bb, double *rr, double *rh,
@@ -1077,15 +1444,20 @@ void launch_krylov_part(hipStream_t s, const Geo &g, const Coef &c, const Box &b
 void launch_apply_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, int form, bool pre,
                         bool any_pz, bool any_nonpz) {
     if (ntiles <= 0) return;
-    const dim3 grid(xcd_grid(ntiles)), block(RED_TX, RED_TY, 1);
-#define IH_APB(DMV)                                                                                               \
-    do {                                                                                                          \
-        if (any_nonpz)                                                                                            \
-            hipLaunchKernelGGL((k_apply_batch<DMV, false>), grid, block, 0, s, cases, tile_case, ntiles, form,      \
-                               (int)pre);                                                                         \
-        if (any_pz)                                                                                               \
-            hipLaunchKernelGGL((k_apply_batch<DMV, true>), grid, block, 0, s, cases, tile_case, ntiles, form,       \
-                               (int)pre);                                                                         \
+    const bool teams = ntiles <= APPLY_TEAM_TILES;
+    const dim3 grid(xcd_grid(ntiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
+#define IH_APB_AS(T, DMV, PZV)                                                                                    \
+    hipLaunchKernelGGL((k_apply_batch<T, DMV, PZV>), grid, block, 0, s, cases, tile_case, ntiles, form, (int)pre)
+#define IH_APB(DMV)                               \
+    do {                                          \
+        if (any_nonpz && teams)                   \
+            IH_APB_AS(true, DMV, false);          \
+        else if (any_nonpz)                       \
+            IH_APB_AS(false, DMV, false);         \
+        if (any_pz && teams)                      \
+            IH_APB_AS(true, DMV, true);           \
+        else if (any_pz)                          \
+            IH_APB_AS(false, DMV, true);          \
     } while (0)
     if (form == KB_APPLY_W)
         IH_APB(DOT_W);
@@ -1096,6 +1468,7 @@ void launch_apply_batch(hipStream_t s, const KBatchCase *cases, const int *tile_
     else
         IH_APB(DOT_NONE);
 #undef IH_APB
+#undef IH_APB_AS
 }
 
 void launch_krylov_init_batch(hipStream_t s, const KBatchCase *cases, int ncases, const int *tile_case, int ntiles,

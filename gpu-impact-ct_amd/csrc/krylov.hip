@@ -936,49 +936,84 @@ __device__ inline void breakdown(int *fl) {
     fl[KF_DONE] = 1;
 }
 
+// The planes of a reduction chunk (at most 32) on UPD_ZG groups of 256 threads, at
+// most UPD_KP planes each: all of a thread's loads are in flight before the scalar
+// of the step is reduced from the operator's partials.
+constexpr int UPD_ZG = 4, UPD_KP = RED_KC / UPD_ZG;
+
+// the planes k0 .. k0 + cnt - 1 of group zg out of the chunk kc0..kc1
+__device__ inline void split_planes(int zg, int kc0, int kc1, int &k0, int &cnt) {
+    const int per = (kc1 - kc0 + UPD_ZG) / UPD_ZG;
+    k0 = kc0 + zg * per;
+    cnt = kc1 - k0 + 1 < per ? kc1 - k0 + 1 : per;
+}
+
+// the sum of the partials by the 256 threads of a group, as wave sums sm[0..3]
+__device__ inline void split_sum_parts(const double *part, int64_t nb, int tid, double *sm) {
+    const double v = wave_sum(thread_sum_parts(part, nb, tid));
+    if ((tid & 63) == 0) sm[tid >> 6] = v;
+}
+
 // alpha = rhr/<rh, Ap> (a vanishing <rh, Ap> is a breakdown), then rr = rr - alpha*Ap
-// (src/mod_solvers.f90:1709-1740)
+// (src/mod_solvers.f90:1709-1740).  Bound by HBM from 257x129x129 on, below by latency:
+// a thread that walks its chunk's planes one by one waits once a plane.  Four groups
+// of planes against one: 5.4 -> 3.7 us at 33x17x17, 6.6 -> 4.4 at 65^3, 12.3 -> 8.1 at
+// 193x97x97, 18.9 -> 18.0 at 257x129x129 (5.7 TB/s), 58.2 -> 54.6 at 385x193x193.
 template <bool FIRST = false>
 __device__ inline void s_update_block(const Geo &g, const Range3 &r, int bx, int by, int bz, int nbz, int64_t pi,
                                       double *rr, const double *Ap, const double *part, int64_t nb, double *sc,
                                       int *fl, const FirstSweep &fs = FirstSweep{}) {
     __shared__ double sm[4];
-    __shared__ double s_alpha;
     __shared__ int s_go;
-    if (!wg_active(fl, &s_go)) return;
-    const double rhAp = reduce_sum_parts(part, nb, sm);
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        const bool ok = !(fabs(rhAp) == 0.0);
-        const double alpha = ok ? sc[KS_RHR] / rhAp : 0.0;
-        s_alpha = alpha;
-        s_go = ok;
-        if (pi == 0) {
-            if (ok)
-                sc[KS_ALPHA] = alpha;
-            else
-                breakdown(fl);
-        }
-    }
-    __syncthreads();
-    if (!s_go) return;
-    const double alpha = s_alpha;
+    const int tid = (int)(threadIdx.x + RED_TX * threadIdx.y);
+    const int zg = __builtin_amdgcn_readfirstlane((int)threadIdx.z);
+    if (tid == 0 && zg == 0) s_go = fl[KF_ACTIVE];
     const int i = r.lo0 + bx * RED_TX + (int)threadIdx.x;
     const int j = r.lo1 + by * RED_TY + (int)threadIdx.y;
-    if (i >= r.lo0 + r.n0 || j >= r.lo1 + r.n1) return;
+    const bool own = i < r.lo0 + r.n0 && j < r.lo1 + r.n1;
     int kc0, kc1;
     red_chunk(r, bz, nbz, kc0, kc1);
-    for (int k = kc0; k <= kc1; ++k) {
-        const int64_t x = gidx(g, i, j, k);
-        const double v = rr[x] - alpha * Ap[x];
-        rr[x] = v;
-        if (FIRST) first_sweep_point(g, fs, i, j, k, x, v);
+    int k0, cnt;
+    split_planes(zg, kc0, kc1, k0, cnt);
+    const int64_t x0 = gidx(g, own ? i : r.lo0, own ? j : r.lo1, 0);
+    double v[UPD_KP], a[UPD_KP];
+#pragma unroll
+    for (int u = 0; u < UPD_KP; ++u) {
+        v[u] = a[u] = 0.0;
+        if (u < cnt) {
+            const int64_t x = x0 + (int64_t)(k0 + u) * g.pxy;
+            v[u] = rr[x];
+            a[u] = Ap[x];
+        }
+    }
+    if (zg == 0) split_sum_parts(part, nb, tid, sm);
+    __syncthreads();
+    if (!s_go) return;
+    const double rhAp = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+    const bool ok = !(fabs(rhAp) == 0.0);
+    const double alpha = ok ? sc[KS_RHR] / rhAp : 0.0;
+    if (tid == 0 && zg == 0 && pi == 0) {
+        if (ok)
+            sc[KS_ALPHA] = alpha;
+        else
+            breakdown(fl);
+    }
+    if (!ok || !own) return;
+#pragma unroll
+    for (int u = 0; u < UPD_KP; ++u) {
+        if (u >= cnt) break;
+        const int k = k0 + u;
+        const int64_t x = x0 + (int64_t)k * g.pxy;
+        const double w = v[u] - alpha * a[u];
+        rr[x] = w;
+        if (FIRST) first_sweep_point(g, fs, i, j, k, x, w);
     }
 }
 
 template <bool FIRST>
-__global__ __launch_bounds__(256) void k_s_update_alpha(Geo g, Range3 r, double *rr, const double *Ap,
-                                                        const double *part, int64_t nb, double *sc, int *fl,
-                                                        FirstSweep fs) {
+__global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_s_update_alpha(Geo g, Range3 r, double *rr, const double *Ap,
+                                                                        const double *part, int64_t nb, double *sc,
+                                                                        int *fl, FirstSweep fs) {
     s_update_block<FIRST>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(), rr,
                           Ap, part, nb, sc, fl, fs);
 }
@@ -1078,6 +1113,116 @@ __global__ __launch_bounds__(256) void k_x_update_omega(Geo g, Range3 r, double 
                                                         int *fl, double *pmax, double *pdot) {
     x_update_block(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(), phi, rr,
                    ra, pa, Ar, rh, p1, p2, nb, sc, fl, pmax, pdot);
+}
+
+// The same update with the chunk's planes on UPD_ZG groups.  The chunk's sum is still
+// formed in plane order: the groups take turns, each adding its products to what the
+// group below passes on, so the partials are the same bits.  PRE: ra is another
+// field than rr (the preconditioned direction).  8.3 -> 7.1 us at 33x17x17, 11.0 ->
+// 9.2 at 65^3, 16.9 -> 11.7 at 118x71x91, 17.0 -> 14.5 at 129x97x97.
+template <bool PRE>
+__device__ inline void x_update_split_block(const Geo &g, const Range3 &r, int bx, int by, int bz, int nbz, int64_t pi,
+                                            double *phi, double *rr, const double *ra, const double *pa,
+                                            const double *Ar, const double *rh, const double *p1, const double *p2,
+                                            int64_t nb, double *sc, int *fl, double *pmax, double *pdot) {
+    __shared__ double sm[8], smax[4 * UPD_ZG], carry[RED_THREADS];
+    __shared__ int s_go;
+    const int tid = (int)(threadIdx.x + RED_TX * threadIdx.y);
+    const int zg = __builtin_amdgcn_readfirstlane((int)threadIdx.z);
+    if (tid == 0 && zg == 0) s_go = fl[KF_ACTIVE];
+    const int i = r.lo0 + bx * RED_TX + (int)threadIdx.x;
+    const int j = r.lo1 + by * RED_TY + (int)threadIdx.y;
+    const bool own = i < r.lo0 + r.n0 && j < r.lo1 + r.n1;
+    int kc0, kc1;
+    red_chunk(r, bz, nbz, kc0, kc1);
+    int k0, cnt;
+    split_planes(zg, kc0, kc1, k0, cnt);
+    const int64_t x0 = gidx(g, own ? i : r.lo0, own ? j : r.lo1, 0);
+    double vph[UPD_KP], vra[UPD_KP], vpa[UPD_KP], vrr[UPD_KP], vAr[UPD_KP], vrh[UPD_KP];
+#pragma unroll
+    for (int u = 0; u < UPD_KP; ++u) {
+        vph[u] = vra[u] = vpa[u] = vrr[u] = vAr[u] = vrh[u] = 0.0;
+        if (u < cnt) {
+            const int64_t x = x0 + (int64_t)(k0 + u) * g.pxy;
+            vph[u] = phi[x];
+            vpa[u] = pa[x];
+            vrr[u] = rr[x];
+            vra[u] = PRE ? ra[x] : vrr[u];
+            vAr[u] = Ar[x];
+            vrh[u] = rh[x];
+        }
+    }
+    const double alpha = sc[KS_ALPHA];
+    if (zg == 0) split_sum_parts(p1, nb, tid, sm);
+    if (zg == 1) split_sum_parts(p2, nb, tid, sm + 4);
+    __syncthreads();
+    if (!s_go) return;
+    const double rAr = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+    const double ArAr = (sm[4] + sm[5]) + (sm[6] + sm[7]);
+    const bool ok = !(fabs(ArAr) == 0.0);
+    const double om = ok ? rAr / ArAr : 0.0;
+    if (tid == 0 && zg == 0 && pi == 0) {
+        if (ok)
+            sc[KS_OMEGA] = om;
+        else
+            breakdown(fl);
+    }
+    if (!ok) return;
+    double m = 0.0;
+#pragma unroll
+    for (int u = 0; u < UPD_KP; ++u) {
+        const int64_t x = x0 + (int64_t)(k0 + u) * g.pxy;
+        const double w = vrr[u] - om * vAr[u];
+        const bool in = own && u < cnt;
+        if (in) {
+            phi[x] = vph[u] + om * vra[u] + alpha * vpa[u];
+            rr[x] = w;
+        }
+        m = in ? max_nan(fabs(w), m) : m;
+        vrh[u] = w * vrh[u];
+    }
+    m = wave_max(m);
+    if ((tid & 63) == 0) smax[zg * 4 + (tid >> 6)] = m;
+#pragma unroll
+    for (int z = 0; z < UPD_ZG; ++z) {
+        if (z > 0) __syncthreads();
+        if (zg == z) {
+            double d = z == 0 ? 0.0 : carry[tid];
+#pragma unroll
+            for (int u = 0; u < UPD_KP; ++u) d = own && u < cnt ? d + vrh[u] : d;
+            if (z < UPD_ZG - 1) {
+                carry[tid] = d;
+            } else {
+                const double s = wave_sum(d);
+                if ((tid & 63) == 0) sm[tid >> 6] = s;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0 && zg == 0) {
+        m = smax[0];
+        for (int q = 1; q < 4 * UPD_ZG; ++q) m = max_nan(smax[q], m);
+        pmax[pi] = m;
+        pdot[pi] = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+    }
+}
+
+// One block of it fills a compute unit (1024 threads of 104 or 120 VGPRs), so it is
+// taken where its blocks fill their rounds over the device: up to one round, or with
+// the last round at most an eighth of all empty.  A BiCGstab iteration with it and
+// without: 118x71x91 (120 tiles) 78.1 / 82 us, 193x97x97 (364, the second round 42 %
+// full) 105.3 / 104.7, 257x129x129 (765) 175.1 / 175.1, 385x193x193 (2275) 584 / 589.
+static bool x_split(int64_t tiles) {
+    const int64_t cus = 256, rounds = (tiles + cus - 1) / cus;
+    return rounds <= 1 || 8 * tiles >= 7 * rounds * cus;
+}
+
+template <bool PRE>
+__global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_x_update_split(
+    Geo g, Range3 r, double *phi, double *rr, const double *ra, const double *pa, const double *Ar, const double *rh,
+    const double *p1, const double *p2, int64_t nb, double *sc, int *fl, double *pmax, double *pdot) {
+    x_update_split_block<PRE>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(),
+                              phi, rr, ra, pa, Ar, rh, p1, p2, nb, sc, fl, pmax, pdot);
 }
 
 __global__ __launch_bounds__(256) void k_ctl_end(const double *pmax, const double *pdot, int64_t nb, double *sc,
@@ -1188,26 +1333,34 @@ __global__ __launch_bounds__(256) void k_p_update_batch(const KBatchCase *__rest
 }
 
 template <bool FIRST>
-__global__ __launch_bounds__(256) void k_s_update_batch(const KBatchCase *__restrict__ cases,
+__global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_s_update_batch(const KBatchCase *__restrict__ cases,
                                                         const int *__restrict__ tile_case, int ntiles, float omega) {
     int bx, by, bz;
     int64_t pi;
     const int q = batch_tile(cases, tile_case, ntiles, bx, by, bz, pi);
     if (q < 0) return;
     const KBatchCase &K = cases[q];
+    if (!K.fl[KF_ACTIVE]) return;  // a stopped case loads nothing
     s_update_block<FIRST>(K.g, K.r, bx, by, bz, K.nbz, pi, K.rr, K.Ap, K.part1, K.nb, K.sc, K.fl,
                           batch_first(K, omega));
 }
 
-__global__ __launch_bounds__(256) void k_x_update_batch(const KBatchCase *__restrict__ cases,
-                                                        const int *__restrict__ tile_case, int ntiles, int pre) {
+template <bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? RED_THREADS * UPD_ZG : RED_THREADS) void k_x_update_batch(
+    const KBatchCase *__restrict__ cases, const int *__restrict__ tile_case, int ntiles, int pre) {
     int bx, by, bz;
     int64_t pi;
     const int q = batch_tile(cases, tile_case, ntiles, bx, by, bz, pi);
     if (q < 0) return;
     const KBatchCase &K = cases[q];
-    x_update_block(K.g, K.r, bx, by, bz, K.nbz, pi, K.phi, K.rr, pre ? K.z2 : K.rr, pre ? K.z1 : K.pk, K.Ar, K.rh,
-                   K.part1, K.part2, K.nb, K.sc, K.fl, K.part3, K.part4);
+    if (!K.fl[KF_ACTIVE]) return;
+    const double *ra = pre ? K.z2 : K.rr, *pa = pre ? K.z1 : K.pk;
+    if constexpr (SPLIT)
+        x_update_split_block<true>(K.g, K.r, bx, by, bz, K.nbz, pi, K.phi, K.rr, ra, pa, K.Ar, K.rh, K.part1, K.part2,
+                                   K.nb, K.sc, K.fl, K.part3, K.part4);
+    else
+        x_update_block(K.g, K.r, bx, by, bz, K.nbz, pi, K.phi, K.rr, ra, pa, K.Ar, K.rh, K.part1, K.part2, K.nb, K.sc,
+                       K.fl, K.part3, K.part4);
 }
 
 // one workgroup per case
@@ -1381,6 +1534,29 @@ static void launch_precond(hipStream_t s, const Geo &g, const Coef &c, const Box
     launch_jor_f32_to64(s, g, c, b, k.omega, x, k.b32, z, act, k.shape);
 }
 
+static void launch_s_update(hipStream_t s, const Geo &g, const Range3 &r, int64_t nb, const KrylovPtrs &k, bool first,
+                            const FirstSweep &fs) {
+    if (first)
+        hipLaunchKernelGGL(k_s_update_alpha<true>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.rr, k.Ap,
+                           k.part1, nb, k.sc, k.fl, fs);
+    else
+        hipLaunchKernelGGL(k_s_update_alpha<false>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.rr, k.Ap,
+                           k.part1, nb, k.sc, k.fl, fs);
+}
+
+static void launch_x_update(hipStream_t s, const Geo &g, const Range3 &r, int64_t nb, const KrylovPtrs &k, bool pre) {
+    const double *ra = pre ? k.z2 : k.rr, *pa = pre ? k.z1 : k.pk;
+    if (x_split(nb) && pre)
+        hipLaunchKernelGGL(k_x_update_split<true>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.phi, k.rr,
+                           ra, pa, k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
+    else if (x_split(nb))
+        hipLaunchKernelGGL(k_x_update_split<false>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.phi, k.rr,
+                           ra, pa, k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
+    else
+        hipLaunchKernelGGL(k_x_update_omega, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.phi, k.rr, ra, pa,
+                           k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
+}
+
 void launch_krylov_iteration(hipStream_t s, const Geo &g, const Coef &c, const Box &b, const KrylovPtrs &k) {
     Range3 r = Rk(b);
     const int64_t nb = red_blocks(b);
@@ -1396,21 +1572,14 @@ void launch_krylov_iteration(hipStream_t s, const Geo &g, const Coef &c, const B
                            FirstSweep{});
     if (pre) launch_precond(s, g, c, b, k.pk, k.z1, k, fuse);
     launch_apply_A(s, g, c, b, pre ? k.z1 : k.pk, k.Ap, k.rh, DOT_W, k.part1, nullptr, k.fl + KF_ACTIVE);
-    if (fuse)
-        hipLaunchKernelGGL(k_s_update_alpha<true>, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.rr, k.Ap,
-                           k.part1, nb, k.sc, k.fl, fs);
-    else
-        hipLaunchKernelGGL(k_s_update_alpha<false>, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.rr, k.Ap,
-                           k.part1, nb, k.sc, k.fl, FirstSweep{});
+    launch_s_update(s, g, r, nb, k, fuse, fs);
     if (pre) {
         launch_precond(s, g, c, b, k.rr, k.z2, k, fuse);
         launch_apply_A(s, g, c, b, k.z2, k.Ar, k.rr, DOT_PAIR, k.part1, k.part2, k.fl + KF_ACTIVE);
     } else {
         launch_apply_A(s, g, c, b, k.rr, k.Ar, nullptr, DOT_SELF, k.part1, k.part2, k.fl + KF_ACTIVE);
     }
-    hipLaunchKernelGGL(k_x_update_omega, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.phi, k.rr,
-                       pre ? k.z2 : k.rr, pre ? k.z1 : k.pk, k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3,
-                       k.part4);
+    launch_x_update(s, g, r, nb, k, pre);
     hipLaunchKernelGGL(k_ctl_end, dim3(1), dim3(RED_TX, RED_TY, 1), 0, s, k.part3, k.part4, nb, k.sc, k.fl);
 }
 
@@ -1426,15 +1595,13 @@ void launch_krylov_part(hipStream_t s, const Geo &g, const Coef &c, const Box &b
         launch_apply_A(s, g, c, b, k.pk, k.Ap, k.rh, DOT_W, k.part1, nullptr, k.fl + KF_ACTIVE);
         break;
     case KPART_S_UPDATE:
-        hipLaunchKernelGGL(k_s_update_alpha<false>, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.rr, k.Ap,
-                           k.part1, nb, k.sc, k.fl, FirstSweep{});
+        launch_s_update(s, g, r, nb, k, false, FirstSweep{});
         break;
     case KPART_APPLY_SELF:
         launch_apply_A(s, g, c, b, k.rr, k.Ar, nullptr, DOT_SELF, k.part1, k.part2, k.fl + KF_ACTIVE);
         break;
     case KPART_X_UPDATE:
-        hipLaunchKernelGGL(k_x_update_omega, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.phi, k.rr, k.rr,
-                           k.pk, k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
+        launch_x_update(s, g, r, nb, k, false);
         break;
     default:
         break;
@@ -1494,17 +1661,21 @@ void launch_s_update_batch(hipStream_t s, const KBatchCase *cases, const int *ti
                            float omega) {
     if (ntiles <= 0) return;
     if (first)
-        hipLaunchKernelGGL(k_s_update_batch<true>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, 1), 0, s, cases,
+        hipLaunchKernelGGL(k_s_update_batch<true>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, cases,
                            tile_case, ntiles, omega);
     else
-        hipLaunchKernelGGL(k_s_update_batch<false>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, 1), 0, s, cases,
+        hipLaunchKernelGGL(k_s_update_batch<false>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, cases,
                            tile_case, ntiles, omega);
 }
 
 void launch_x_update_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, bool pre) {
-    if (ntiles > 0)
-        hipLaunchKernelGGL(k_x_update_batch, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, 1), 0, s, cases, tile_case,
-                           ntiles, (int)pre);
+    if (ntiles <= 0) return;
+    if (x_split(ntiles))
+        hipLaunchKernelGGL(k_x_update_batch<true>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, cases,
+                           tile_case, ntiles, (int)pre);
+    else
+        hipLaunchKernelGGL(k_x_update_batch<false>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, 1), 0, s, cases,
+                           tile_case, ntiles, (int)pre);
 }
 
 void launch_gather_batch(hipStream_t s, const KBatchCase *cases, int ncases, int *fl_out, double *sc_out) {

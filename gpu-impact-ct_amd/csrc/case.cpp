@@ -280,6 +280,7 @@ int upload_coeffs(ih_case *c) {
         off_xu[d] = (int64_t)h.size();
         h.insert(h.end(), c->hg.xu[d].begin(), c->hg.xu[d].end());
     }
+    h.resize((h.size() + 1) / 2 * 2, 0.0);  // 16-byte loads read it
     const int64_t off_zero = (int64_t)h.size();
     h.resize(h.size() + 64, 0.0);
     if (c->dcoef) (void)hipFree(c->dcoef);
@@ -297,6 +298,9 @@ int upload_coeffs(ih_case *c) {
     HIPCHK(hipMalloc(&c->dcoef32, sizeof(float) * h32.size()));
     HIPCHK(hipMemcpy(c->dcoef32, h32.data(), sizeof(float) * h32.size(), hipMemcpyHostToDevice));
     c->c.zero = c->dcoef + off_zero;
+    c->c.dg_walls0 = 1;
+    for (int d = 0; d < 3; ++d)
+        if (!g.per[d] && (hc.dg[d][0] != 0.0 || hc.dg[d][2 + 3 * (size_t)(g.N[d] - 1)] != 0.0)) c->c.dg_walls0 = 0;
     for (int d = 0; d < 3; ++d) {
         c->c.G[d] = c->dcoef + off_G[d];
         c->c.Ip[d] = c->dcoef + off_Ip[d];
@@ -1013,9 +1017,16 @@ static int jor_run(ih_case *c, int n_sweeps, double omega, const Box &b, ih_fiel
     const bool with_bc = pbc_substep == 3 && c->ctlab;
     int rc;
     PhaseTimer pt(c, "jor");
-    for (int s = 0; s < n_sweeps; ++s) {
+    const bool pairs = whole && !with_bc && jor_pair_ok(c->g, c->c, b, false);
+    for (int s = 0; s < n_sweeps;) {
         if (with_bc && (rc = jacobi_pressure_bc(c, x, pbc_substep, pbc_dtime))) return rc;
-        launch_jor(c->stream, c->g, c->c, b, omega, x, B, y, sh);
+        if (pairs && n_sweeps - s >= 2) {
+            launch_jor_pair(c->stream, c->g, c->c, b, omega, x, B, y, nullptr);
+            s += 2;
+        } else {
+            launch_jor(c->stream, c->g, c->c, b, omega, x, B, y, sh);
+            s += 1;
+        }
         std::swap(x, y);
     }
     pt.done(n_sweeps);
@@ -1280,6 +1291,7 @@ static int mg_setup(ih_case *c) {
             offR[g][d] = put(h.cR[d], 3);
             offI[g][d] = put(h.cI[d], 2);
         }
+    tab.resize((tab.size() + 1) / 2 * 2, 0.0);  // 16-byte loads read it (arr is even)
     const int64_t offZ = (int64_t)tab.size();
     tab.resize(tab.size() + 64, 0.0);
     const int64_t total = arr + (int64_t)tab.size();
@@ -1300,6 +1312,12 @@ static int mg_setup(ih_case *c) {
             L.c = Coef{};
             for (int d = 0; d < 3; ++d) L.c.dg[d] = tb + offdg[g][d];
             L.c.zero = tb + offZ;
+            L.c.dg_walls0 = 1;
+            for (int d = 0; d < 3; ++d) {
+                const HostMgLevel &h = c->mgh[g - 1];
+                if (!L.g.per[d] && (h.dg[d][0] != 0.0 || h.dg[d][2 + 3 * (size_t)(h.N[d] - 1)] != 0.0))
+                    L.c.dg_walls0 = 0;
+            }
             L.A = base + offA[g];
             L.B = base + offB[g];
         }
@@ -1822,8 +1840,15 @@ static int poisson_solve(ih_case *c, const ih_step_params *p, const Box &b, int 
                 launch_jor_f32(c->stream, g, c->c, b, (float)p->jor_omega, x, c->f32[1], y, nullptr, l);
             });
             PhaseTimer pt(c, "jor_f32");
-            for (int s = 0; s < p->jor_sweeps; ++s) {
-                launch_jor_f32(c->stream, g, c->c, b, (float)p->jor_omega, x, c->f32[1], y, nullptr, sh);
+            const bool pairs = jor_pair_ok(g, c->c, b, true);
+            for (int s = 0; s < p->jor_sweeps;) {
+                if (pairs && p->jor_sweeps - s >= 2) {
+                    launch_jor_pair(c->stream, g, c->c, b, (float)p->jor_omega, x, c->f32[1], y, nullptr);
+                    s += 2;
+                } else {
+                    launch_jor_f32(c->stream, g, c->c, b, (float)p->jor_omega, x, c->f32[1], y, nullptr, sh);
+                    s += 1;
+                }
                 std::swap(x, y);
             }
             pt.done(p->jor_sweeps);
@@ -2296,6 +2321,14 @@ int ih_bench_kernel(ih_case *c, const char *name, int launches, double *ms_per_l
             launch_jor_f32(s, c->g, c->c, b, 0.8f, c->f32[0], c->f32[1], c->f32[2], nullptr, l);
         });
         one = [&]() { launch_jor_f32(s, c->g, c->c, b, 0.8f, c->f32[0], c->f32[1], c->f32[2], nullptr, sh); };
+    } else if ((n == "jor_pair" || n == "jor_pair_f32") && jor_pair_ok(c->g, c->c, b, n == "jor_pair_f32")) {
+        // two sweeps in one launch
+        if (n == "jor_pair")
+            one = [&]() {
+                launch_jor_pair(s, c->g, c->c, b, 0.8, F(c, IH_PRE), F(c, IH_RES), F(c, IH_COMP), nullptr);
+            };
+        else
+            one = [&]() { launch_jor_pair(s, c->g, c->c, b, 0.8f, c->f32[0], c->f32[1], c->f32[2], nullptr); };
     } else if (n == "apply") {
         one = [&]() {
             launch_apply_A(s, c->g, c->c, b, F(c, IH_PK), F(c, IH_AP), nullptr, KDOT_NONE, nullptr, nullptr, nullptr);

@@ -50,6 +50,7 @@ struct Coef {
     const double *G6[3], *D6[3];
     const double *xp[3];   // coordinates (-3:N+3) at [i+3]
     const double *xu[3];
+    int dg_walls0 = 0;     // cdg couples nothing past a wall (0 at -1 of the first, 0 at +1 of the last point)
     const double *zero;    // 64 doubles of 0.0, never written: the load source for positions outside the field
 };
 
@@ -110,6 +111,16 @@ void launch_jor(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double
                 const double *bb, double *out, const int *active, JorLaunch shape);
 void launch_jor_f32(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
                     const float *bb, float *out, const int *active = nullptr, JorLaunch shape = JorLaunch());
+// Two JOR sweeps in one launch, out = sweep(sweep(rel)), the bits of two single
+// ones.  jor_pair_ok: whether box b takes it (the whole pressure range, x not
+// periodic, no coupling past a wall, rows short enough for a block).
+bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32);
+void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double omega, const double *rel,
+                     const double *bb, double *out, const int *active);
+void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
+                     const float *bb, float *out, const int *active);
+void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
+                     const float *bb, double *out, const int *active);
 void launch_residual_cdg(hipStream_t s, const Geo &g, const Coef &c, const Box &b, const double *rel,
                          const double *bb, double *out_res /* may be null */, double *partial_max);
 void launch_copy_box(hipStream_t s, const Geo &g, const Box &b, const double *src, double *dst);

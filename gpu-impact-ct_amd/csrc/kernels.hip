@@ -926,6 +926,215 @@ __global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, Coef c, Range3 r, JorVec
     jor_vec_block<T, T, TPB, PXM, const T *, T *, true>(g, r, sh, tw, bz, nbz, T(0), x, x, lap, g1, g2, g3);
 }
 
+// Two sweeps in one launch: out = sweep(sweep(rel)), each value formed with the
+// operands and order of the single sweep, so the result is its bits.  The first
+// sweep's iterate lives on chip.  The entries of a plane (rows of aligned vectors
+// with a halo vector at either end, one flat sequence as above) are cut into
+// stretches; a block takes TPB consecutive entries, one a thread, and marches z:
+//   - plane k of rel goes through LDS, where a thread finds its y neighbours nent
+//     entries away and the x neighbours of a wavefront's edge lanes; the threads
+//     within a row of the stretch's ends load their outer y neighbour instead;
+//   - the first iterate of plane k goes through LDS the same way, a plane later, for
+//     the second sweep of plane k-1 (one barrier a plane, both double buffered);
+//   - z neighbours of both sweeps are register queues.
+// The first iterate is right on all TPB entries, the second on those a row and an
+// entry or more from the ends, so consecutive stretches overlap by 2 (nent + 1)
+// entries, and z chunks by one plane at either end.
+// Points outside the range enter the second sweep as zeros; their coefficients are
+// zero (the rule for taking this kernel checks it), as is what dead entries load.
+// A single sweep moves 24 (FP32: 12) bytes a point for 27 operations and runs at the
+// rate of the last-level cache or of the launches; a pair moves them once, and the
+// vector ALU bounds it (about 30 instructions a point and sweep, 13 of them the
+// IEEE division).  Measured, microseconds for two sweeps, two launches -> a pair:
+//               33x17x17    65^3       97^3       193x97x97  257x129x129 385x193x193
+//   FP64        7.0 ->  4.9 8.8 -> 7.8 12.6 -> 12.3 19.4 -> 16.5 38.4 -> 30.9 164 -> 93.5
+//   FP32        7.8 ->  5.4 8.4 -> 6.5 12.6 -> 10.7 14.4 -> 13.9 24.0 -> 22.4 55.2 -> 51.2
+// A reciprocal shared by the two sweeps with the quotient corrected to the IEEE
+// one costs, with the range checks, as many instructions as it saves.
+template <typename T, typename TO, int TPB, bool PZ>
+__global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVecShape sh, int nt, int nbz, T omega,
+                                                  const T *__restrict__ rel, const T *__restrict__ bb,
+                                                  TO *__restrict__ out, const int *active) {
+    if (active && !*active) return;
+    int tw, dummy, bz;
+    if (!xcd_tile(nt, 1, nbz, tw, dummy, bz)) return;
+    constexpr int V = 16 / sizeof(T);
+    typedef typename VecOf<T>::type VT;
+    typedef TO VO __attribute__((ext_vector_type(V)));
+    __shared__ VT s0[2][TPB], s1[2][TPB];
+    const T *const g1 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[0] : (const void *)c.dgf[0]);
+    const T *const g2 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[1] : (const void *)c.dgf[1]);
+    // scalar loads: a vector load of a uniform value would be waited for together with
+    // the plane's prefetches
+    typedef const __attribute__((address_space(4))) T *CP;
+    const CP g3 = (CP)(sizeof(T) == 8 ? (const void *)c.dg[2] : (const void *)c.dgf[2]);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int nent = sh.nent, H = nent + 1;
+    const int q = tw * (TPB - 2 * H) - H + tid;
+    // past the first or the last row: the opposite row of a periodic y, else dead
+    const bool inside = q >= 0 && q < sh.nent_all;
+    // (from one row below, where the outer neighbours are loads, to two above: nothing
+    // further out is used)
+    const bool live = inside || (g.per[1] && q < sh.nent_all + 2 * H);
+    int qm = q < 0 ? q + sh.nent_all : (q >= sh.nent_all ? q - sh.nent_all : q);
+    if (!live) qm = 0;
+    const int jj = qm / nent, e = qm - jj * nent;
+    const int j = r.lo1 + jj;
+    const int is = sh.i0 + V * (e - 1);
+    const int hi0 = r.lo0 + r.n0 - 1;
+    const bool row = live && e >= 1 && e <= sh.nv;  // a vector with points of the range
+    const bool full = row && is >= r.lo0 && is + V - 1 <= hi0;
+    const bool store = inside && row && tid >= H && tid < TPB - H;
+    const int c0 = g.cst[0], c1 = g.cst[1], c2 = g.cst[2];
+    T a1m[V], a1p[V], a1d[V];
+#pragma unroll
+    for (int t = 0; t < V; ++t) {
+        int ic = is + t;
+        ic = ic < r.lo0 ? r.lo0 : (ic > hi0 ? hi0 : ic);
+        a1m[t] = g1[0 * c0 + ic];
+        a1p[t] = g1[2 * c0 + ic];
+        a1d[t] = g1[1 * c0 + ic];
+    }
+    const T a2m = g2[0 * c1 + j], a2p = g2[2 * c1 + j], a2d = g2[1 * c1 + j];
+    int kc0, kc1;
+    red_chunk(r, bz, nbz, kc0, kc1);
+    const int lo2 = r.lo2, hi2 = r.lo2 + r.n2 - 1;
+    // plane index in memory: wrapped, or held to the range and m ghost planes
+    auto plane = [&](int k, int m) {
+        if constexpr (PZ) return k < lo2 ? k + r.n2 : (k > hi2 ? k - r.n2 : k);
+        k = k < lo2 - m ? lo2 - m : k;
+        return k > hi2 + m ? hi2 + m : k;
+    };
+    const int64_t xy = gidx(g, is, j, 0) - 3 * g.pxy;
+    // dead entries read zeros, whatever the plane
+    const T *const xp = live ? rel + xy + 3 * g.pxy : (const T *)c.zero;
+    const T *const bp = live ? bb + xy + 3 * g.pxy : (const T *)c.zero;
+    // outer y neighbour of the stretch's first and last row
+    const bool lowe = tid < nent, highe = tid >= TPB - nent;
+    int64_t dye = lowe ? -(int64_t)g.px : (int64_t)g.px;
+    if (g.per[1]) {
+        if (lowe && j == g.Sp[1]) dye = (int64_t)(g.Np[1] - g.Sp[1]) * g.px;
+        if (highe && j == g.Np[1]) dye = -(int64_t)(g.Np[1] - g.Sp[1]) * g.px;
+    }
+    const T *const ep = live ? xp + dye : xp;
+    const bool edge_wave = __builtin_amdgcn_readfirstlane(tid & ~63) < nent ||
+                           __builtin_amdgcn_readfirstlane(tid | 63) >= TPB - nent;
+    auto ld = [&](const T *p, int k, int m) {
+        const int64_t o = (int64_t)plane(k, m) * g.pxy;
+        return vload<VT>(p + (live ? o : 0));
+    };
+
+    struct Zc {  // z coefficients of a plane
+        T m, p, d;
+    };
+    auto zcoef = [&](int k) {
+        const int kg = plane(k, 0);
+        return Zc{g3[kg], g3[2 * c2 + kg], g3[c2 + kg]};
+    };
+    // one sweep of this thread's vector x on the right-hand side b
+    auto relax = [&](const VT &b, const VT &x, const VT &ym, const VT &yp, const VT &zlo, const VT &zhi, T xl, T xr,
+                     const Zc &z, VT &res) {
+#pragma unroll
+        for (int t = 0; t < V; ++t) {
+            T s = b[t];
+            s = s - a1m[t] * (t == 0 ? xl : x[t > 0 ? t - 1 : 0]);
+            s = s - a1p[t] * (t == V - 1 ? xr : x[t < V - 1 ? t + 1 : V - 1]);
+            s = s - a2m * ym[t];
+            s = s - a2p * yp[t];
+            s = s - z.m * zlo[t];
+            s = s - z.p * zhi[t];
+            const T diag = (a1d[t] + a2d) + z.d;
+            res[t] = omega * s / diag + (T(1) - omega) * x[t];
+        }
+    };
+    // x neighbours: the adjacent lanes', at a wavefront's edges from LDS
+    const bool elane = lane == 0 || lane == 63;
+    const int eidx = lane == 0 ? (tid > 0 ? V * tid - 1 : 0) : (tid < TPB - 1 ? V * (tid + 1) : 0);
+    auto x_neighbours = [&](const VT *buf, const VT &x, T &xl, T &xr) {
+        xl = lane_prev(x[V - 1]);
+        xr = lane_next(x[0]);
+        if (elane) {
+            const T v = ((const T *)buf)[eidx];
+            if (lane == 0)
+                xl = v;
+            else
+                xr = v;
+        }
+    };
+    const int im = tid >= nent ? tid - nent : tid, ip = tid < TPB - nent ? tid + nent : tid;
+    bool real[V];  // points of the range
+#pragma unroll
+    for (int t = 0; t < V; ++t) real[t] = row && is + t >= r.lo0 && is + t <= hi0;
+
+    const VT zero{};
+    VT zm = ld(xp, kc0 - 2, 1), zc = ld(xp, kc0 - 1, 1);
+    VT bm = zero, um = zero, uc = zero;  // b at k-1, first iterate at k-2 and k-1
+    Zc gm{}, gc = zcoef(kc0 - 1);
+    // what a plane needs from memory: rel at k+1, b and the edge rows at k; loaded a
+    // plane ahead, into two sets by turns
+    struct Plane {
+        VT zp, b, ye;
+    };
+    auto fetch = [&](int k, Plane &P) {
+        P.zp = ld(xp, k + 1, 1);
+        P.b = ld(bp, k, 0);
+        if (edge_wave) P.ye = ld(ep, k, 1);
+    };
+    Plane A, B;
+    A.ye = B.ye = zero;
+    fetch(kc0 - 1, A);
+    s0[0][tid] = zc;
+    auto step = [&](int k, int buf, Plane &P, Plane &next) {
+        __syncthreads();
+        fetch(k + 1, next);
+        const Zc gn = zcoef(k + 1);
+        VT ym = s0[buf][im], yp = s0[buf][ip];
+        VT vm = s1[buf ^ 1][im], vp = s1[buf ^ 1][ip];
+        T xl, xr, vl, vr;
+        x_neighbours(s0[buf], zc, xl, xr);
+        x_neighbours(s1[buf ^ 1], uc, vl, vr);
+        if (lowe) ym = P.ye;
+        if (highe) yp = P.ye;
+        VT u;
+        relax(P.b, zc, ym, yp, zm, P.zp, xl, xr, gc, u);
+        const bool in_z = PZ || (k >= lo2 && k <= hi2);
+#pragma unroll
+        for (int t = 0; t < V; ++t) u[t] = real[t] && in_z ? u[t] : T(0);
+        s1[buf][tid] = u;
+        s0[buf ^ 1][tid] = P.zp;
+        VT w;  // the second sweep of plane k-1 (from k = kc0 + 1 on)
+        relax(bm, uc, vm, vp, um, u, vl, vr, gm, w);
+        if (store && k > kc0) {
+            TO *const o = out + xy + (int64_t)(k - 1 + 3) * g.pxy;
+            if (full) {
+                VO v;
+#pragma unroll
+                for (int t = 0; t < V; ++t) v[t] = (TO)w[t];
+                vstore<VO>(o, v);
+            } else {
+#pragma unroll
+                for (int t = 0; t < V; ++t)
+                    if (real[t]) o[t] = (TO)w[t];
+            }
+        }
+        um = uc;
+        uc = u;
+        bm = P.b;
+        zm = zc;
+        zc = P.zp;
+        gm = gc;
+        gc = gn;
+    };
+    // leaves from between its halves (with a way around one of them, the other's wait
+    // for its loads would be a wait for all loads)
+    for (int k = kc0 - 1;;) {
+        step(k, 0, A, B);
+        if (++k > kc1 + 1) break;
+        step(k, 1, B, A);
+        if (++k > kc1 + 1) break;
+    }
+}
+
 // First FP32 sweep from e = 0 on A e = (float)v: b32 = (float)v is stored for
 // the later sweeps; every neighbour term is the product with 0 that the
 // generic sweep would form, so the result is that sweep's bit for bit.  A
@@ -1562,6 +1771,86 @@ void launch_jor_f32(hipStream_t s, const Geo &g, const Coef &c, const Box &b, fl
 void launch_jor_f32_to64(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
                          const float *bb, double *out, const int *active, JorLaunch shape) {
     launch_jor_vec<float, double>(s, g, c, b, omega, rel, bb, out, active, shape);
+}
+
+// Launch of a sweep pair: threads a block and z chunk by the estimated time of the
+// most loaded compute unit.  A block's plane costs its two sweeps' instructions
+// (about 1000 clocks a wavefront of 4 FP32 points or 2 FP64 ones, shared by the
+// wavefronts of a SIMD) or, where few wavefronts are resident, the latency of the
+// chain barrier to barrier; starting a block costs about five planes of latency.
+template <typename T, typename TO>
+static bool launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, T omega, const T *rel, const T *bb,
+                        TO *out, const int *active) {
+    const Range3 r = R(b);
+    int best_t = 0, best_nbz = 0, best_nt = 0;
+    double best = 0.0;
+    JorVecShape sh;
+    for (int tpb : {256, 512, 1024}) {
+        int nbw, nbz0;
+        sh = jor_vec_shape(g, r, 16 / (int)sizeof(T), 256, 0, nbw, nbz0);
+        const int span = tpb - 2 * (sh.nent + 1);
+        if (4 * (sh.nent + 1) > tpb) continue;
+        const int nt = (sh.nent_all + span - 1) / span;
+        for (int nbz = 1, kc; nbz <= r.n2; nbz = kc > 1 ? (r.n2 + kc - 2) / (kc - 1) : r.n2 + 1) {
+            kc = (r.n2 + nbz - 1) / nbz;  // the fewest chunks of each length
+            const double blocks = std::ceil((double)nt * nbz / 256.0);  // on the most loaded compute unit
+            const double resident = std::min(blocks, 1024.0 / tpb);
+            const double plane = std::max(1200.0, resident * tpb / 256.0 * 1000.0);
+            const double t = blocks / resident * (6000.0 + (kc + 2) * plane);
+            if (!best_t || t < best) {
+                best = t;
+                best_t = tpb;
+                best_nbz = nbz;
+                best_nt = nt;
+            }
+        }
+    }
+    if (!best_t) return false;
+    const dim3 grid(xcd_grid((int64_t)best_nt * best_nbz));
+#define IH_JP(TPBV)                                                                                               \
+    do {                                                                                                          \
+        if (g.per[2])                                                                                             \
+            hipLaunchKernelGGL((k_jor_pair<T, TO, TPBV, true>), grid, dim3(TPBV), 0, s, g, c, r, sh, best_nt,        \
+                               best_nbz, omega, rel, bb, out, active);                                            \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_jor_pair<T, TO, TPBV, false>), grid, dim3(TPBV), 0, s, g, c, r, sh, best_nt,       \
+                               best_nbz, omega, rel, bb, out, active);                                            \
+    } while (0)
+    if (best_t == 256)
+        IH_JP(256);
+    else if (best_t == 512)
+        IH_JP(512);
+    else
+        IH_JP(1024);
+#undef IH_JP
+    return true;
+}
+
+// The pair is the faster form at every size it fits (figures above k_jor_pair), so
+// the rule is what it can do: rows of which four fit a block (half of its entries
+// are then stored: FP64 rows to 506 points, FP32 to 1012), at least two rows' worth
+// of entries to wrap a periodic y by, nothing that the second sweep would read
+// from a ghost point that is not there.
+bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32) {
+    if (!c.dg_walls0 || g.per[0]) return false;
+    for (int d = 0; d < 3; ++d)
+        if (b.lo[d] != g.Sp[d] || b.hi[d] != g.Np[d]) return false;
+    int nbw, nbz;
+    const JorVecShape sh = jor_vec_shape(g, R(b), fp32 ? 4 : 2, 256, 0, nbw, nbz);
+    return 4 * (sh.nent + 1) <= 1024 && 2 * (sh.nent + 1) <= sh.nent_all && b.hi[2] > b.lo[2];
+}
+
+void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double omega, const double *rel,
+                     const double *bb, double *out, const int *active) {
+    launch_pair<double, double>(s, g, c, b, omega, rel, bb, out, active);
+}
+void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
+                     const float *bb, float *out, const int *active) {
+    launch_pair<float, float>(s, g, c, b, omega, rel, bb, out, active);
+}
+void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
+                     const float *bb, double *out, const int *active) {
+    launch_pair<float, double>(s, g, c, b, omega, rel, bb, out, active);
 }
 
 // the residual product of a multigrid level with the sweep's vector lanes and launch shape

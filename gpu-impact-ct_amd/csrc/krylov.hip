@@ -1513,10 +1513,17 @@ static void launch_precond(hipStream_t s, const Geo &g, const Coef &c, const Box
     if (k.sweeps64 > 0) {
         // FP64 sweeps on A e = v from e = 0 (the like-for-like FP64 form of the FP32 M):
         // the first reads the zero field, the last writes z
+        const bool pairs = jor_pair_ok(g, c, b, false);
         const double *x = k.zero64;
-        for (int q = 0; q < k.sweeps64; ++q) {
-            double *y = q == k.sweeps64 - 1 ? z : (q % 2 == 0 ? k.e64a : k.e64b);
-            launch_jor(s, g, c, b, k.omega64, x, v, y, act, k.shape64);
+        for (int q = 0; q < k.sweeps64;) {
+            // an odd count's single sweep comes first
+            const int n = pairs && (k.sweeps64 - q) % 2 == 0 ? 2 : 1;
+            q += n;
+            double *y = q == k.sweeps64 ? z : (x == k.e64a ? k.e64b : k.e64a);
+            if (n == 2)
+                launch_jor_pair(s, g, c, b, k.omega64, x, v, y, act);
+            else
+                launch_jor(s, g, c, b, k.omega64, x, v, y, act, k.shape64);
             x = y;
         }
         return;
@@ -1526,12 +1533,22 @@ static void launch_precond(hipStream_t s, const Geo &g, const Coef &c, const Box
         return;
     }
     if (!first_done) launch_jor_f32_first(s, g, c, b, k.omega, v, k.b32, k.e0, nullptr, act);
+    // the sweeps after the first, two a launch where the box takes pairs
+    const bool pairs = jor_pair_ok(g, c, b, true);
     float *x = k.e0, *y = k.e1;
-    for (int q = 1; q < k.sweeps - 1; ++q) {
-        launch_jor_f32(s, g, c, b, k.omega, x, k.b32, y, act, k.shape);
+    for (int left = k.sweeps - 1; left > 0;) {
+        const int n = pairs && left % 2 == 0 ? 2 : 1;
+        left -= n;
+        if (left == 0 && n == 2)
+            launch_jor_pair(s, g, c, b, k.omega, x, k.b32, z, act);
+        else if (left == 0)
+            launch_jor_f32_to64(s, g, c, b, k.omega, x, k.b32, z, act, k.shape);
+        else if (n == 2)
+            launch_jor_pair(s, g, c, b, k.omega, x, k.b32, y, act);
+        else
+            launch_jor_f32(s, g, c, b, k.omega, x, k.b32, y, act, k.shape);
         std::swap(x, y);
     }
-    launch_jor_f32_to64(s, g, c, b, k.omega, x, k.b32, z, act, k.shape);
 }
 
 static void launch_s_update(hipStream_t s, const Geo &g, const Range3 &r, int64_t nb, const KrylovPtrs &k, bool first,

@@ -427,6 +427,10 @@ struct CycleBufs<float> {
     static const MgLevelDev<float> *dev(const MgDev &m) { return m.Ldev32; }
 };
 
+// launches of n sweeps of a level: two a launch where its range takes pairs
+inline bool level_pairs(const MgLevel &L, bool fp32) { return jor_pair_ok(L.g, L.c, L.pr, fp32); }
+inline int sweep_launches(int n, bool pairs) { return pairs ? (n + 1) / 2 : n; }
+
 inline void jor_any(hipStream_t s, const MgLevel &L, double omega, const double *x, const double *b, double *y,
                     const int *act, JorLaunch sh) {
     launch_jor(s, L.g, L.c, L.pr, omega, x, b, y, act, sh);
@@ -447,7 +451,9 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
     if (fp64) {
         // level 1 alternates between z and D over the cycle's sweeps; starting on
         // the buffer that makes the last sweep write z leaves the result in place
-        const int flips1 = G > 1 ? (m.n_down - 1) + m.n_up : (m.n_bottom - 1) + m.n_bottom;
+        const bool p1 = level_pairs(m.L[1], false);
+        const int flips1 = G > 1 ? sweep_launches(m.n_down - 1, p1) + sweep_launches(m.n_up, p1)
+                                 : sweep_launches(m.n_bottom - 1, p1) + sweep_launches(m.n_bottom, p1);
         b[1] = (T *)v;
         x[1] = (flips1 % 2 == 0) ? (T *)z : B_::D(m.L[1]);
         y[1] = (x[1] == (T *)z) ? B_::D(m.L[1]) : (T *)z;
@@ -479,9 +485,18 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
             }
             q = 2;
         }
-        for (; q <= n; ++q) {
-            if (launch) {
-                if (last_to_z && q == n)
+        const bool pairs = launch && level_pairs(L, !fp64);
+        while (q <= n) {
+            const int two = pairs && (n - q) % 2 == 1 ? 2 : 1;  // an odd count's single sweep comes first
+            q += two;
+            const bool to_z = last_to_z && q > n;
+            if (launch && two == 2) {
+                if (to_z)
+                    launch_jor_pair(s, L.g, L.c, L.pr, (float)omega, (const float *)x[g], (const float *)b[g], z, act);
+                else
+                    launch_jor_pair(s, L.g, L.c, L.pr, omega, (const T *)x[g], (const T *)b[g], y[g], act);
+            } else if (launch) {
+                if (to_z)
                     launch_jor_f32_to64(s, L.g, L.c, L.pr, (float)omega, (const float *)x[g], (const float *)b[g], z,
                                         act, B_::shape(L));
                 else

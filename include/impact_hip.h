@@ -476,7 +476,8 @@ int ih_kernel_timing_get(ih_case *c, const char *family, double *total_ms, int64
 /* `launches` launches of one kernel back to back between two events on the
  * case's stream: "jor" (an FP64 sweep over the pressure range), "jor_f32" (an
  * FP32 sweep of the mixed-precision preconditioner, on the case's float
- * fields), "apply" (the fused operator alone), the five kernels of a BiCGstab
+ * fields), "jor_pair" and "jor_pair_f32" (two such sweeps in one launch, where
+ * the case takes it), "apply" (the fused operator alone), the five kernels of a BiCGstab
  * iteration -- "p_update", "apply_w" (operator with <rh, Ap>), "s_update",
  * "apply_self" (operator with <r, Ar>, <Ar, Ar>), "x_update" -- on the case's
  * Krylov fields (their results are meaningless), and the substep stencils

@@ -96,6 +96,7 @@ struct ih_case {
     hipStream_t stream = nullptr;
     double *fields[IH_NFIELDS] = {};
     float *f32[3] = {};        // mixed precision: relaxed correction, right-hand side, ping-pong
+    double *stage = nullptr;   // dense rows on their way between a field and the host
     uint8_t *mask = nullptr;   // 3 * fe bytes
     int has_mask = 0;
     double *dcoef = nullptr;   // coefficient tables (SoA) + coordinates

@@ -387,18 +387,14 @@ int jacobi_pressure_bc(ih_case *c, double *rel, int substep, double dtime) {
 }
 
 void drop_mg(ih_case *c) {
-    if (!c->mg && !c->mgmem && !c->mgldev && !c->mgmem32 && !c->mgldev32) return;
+    if (!c->mg && !c->mgmem && !c->mgmem32) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     delete c->mg;
     c->mg = nullptr;
     if (c->mgmem) (void)hipFree(c->mgmem);
     c->mgmem = nullptr;
-    if (c->mgldev) (void)hipFree(c->mgldev);
-    c->mgldev = nullptr;
     if (c->mgmem32) (void)hipFree(c->mgmem32);
     c->mgmem32 = nullptr;
-    if (c->mgldev32) (void)hipFree(c->mgldev32);
-    c->mgldev32 = nullptr;
     c->mgh.clear();
     c->bytes -= c->mg_bytes;
     c->mg_bytes = 0;
@@ -529,9 +525,7 @@ void ih_case_destroy(ih_case *c) {
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     delete c->mg;
     if (c->mgmem) (void)hipFree(c->mgmem);
-    if (c->mgldev) (void)hipFree(c->mgldev);
     if (c->mgmem32) (void)hipFree(c->mgmem32);
-    if (c->mgldev32) (void)hipFree(c->mgldev32);
     resolve_timings(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1261,8 +1255,7 @@ static int64_t mg_alloc_bytes(const std::vector<HostMgLevel> &mgh) {
         arr32 += 4 * fe;
         for (int d = 0; d < 3; ++d) tab += 8 * (int64_t)(((N[d] + 1) + 7) / 8 * 8);
     }
-    return (int64_t)sizeof(double) * (arr + tab + 64) + (int64_t)sizeof(float) * (arr32 + tab) +
-           (int64_t)(G + 1) * (int64_t)(sizeof(MgLevelDev<float>) + sizeof(MgLevelDev<double>));
+    return (int64_t)sizeof(double) * (arr + tab + 64) + (int64_t)sizeof(float) * (arr32 + tab);
 }
 
 static int mg_setup(ih_case *c) {
@@ -1370,14 +1363,7 @@ static int mg_setup(ih_case *c) {
             L.cI[d] = tb + offI[g][d];
         }
     }
-    // levels from g0 on run inside one workgroup; their descriptors in device memory
-    for (int g = 2; g <= G; ++g) {
-        const Geo &q = m->L[g].g;
-        if ((int64_t)q.N[0] * q.N[1] * q.N[2] <= MG_FUSED_POINTS) {
-            m->g0 = g;
-            break;
-        }
-    }
+    m->g0 = mg_first_fused(*m);  // levels from g0 on run inside one workgroup
     // the FP32 cycle: float arrays (level 1 included: its Af is (float) of the
     // right-hand side) and the tables rounded once
     int64_t arr32 = 0;
@@ -1427,52 +1413,6 @@ static int mg_setup(ih_case *c) {
             }
         }
     }
-    std::vector<MgLevelDev<float>> ld32((size_t)G + 1);
-    for (int g = 1; g <= G; ++g) {
-        const MgLevel &L = m->L[g];
-        MgLevelDev<float> &d = ld32[g];
-        d.g = L.g;
-        for (int e = 0; e < 3; ++e) {
-            d.dg[e] = L.c.dgf[e];
-            d.cR[e] = L.cRf[e];
-            d.cI[e] = L.cIf[e];
-            d.dn[e] = L.dn[e];
-        }
-        d.A = L.Af;
-        d.B = L.Bf;
-        d.C = L.Cf;
-        d.D = L.Df;
-    }
-    if (hipMalloc(&c->mgldev32, sizeof(MgLevelDev<float>) * ld32.size()) != hipSuccess) {
-        delete m;
-        return fail(IH_ENOMEM, "out of device memory for the multigrid level descriptors");
-    }
-    HIPCHK(hipMemcpyAsync(c->mgldev32, ld32.data(), sizeof(MgLevelDev<float>) * ld32.size(), hipMemcpyHostToDevice,
-                          c->stream));
-    m->Ldev32 = (const MgLevelDev<float> *)c->mgldev32;
-    std::vector<MgLevelDev<double>> ld((size_t)G + 1);
-    for (int g = 1; g <= G; ++g) {
-        const MgLevel &L = m->L[g];
-        MgLevelDev<double> &d = ld[g];
-        d.g = L.g;
-        for (int e = 0; e < 3; ++e) {
-            d.dg[e] = L.c.dg[e];
-            d.cR[e] = L.cR[e];
-            d.cI[e] = L.cI[e];
-            d.dn[e] = L.dn[e];
-        }
-        d.A = L.A;
-        d.B = L.B;
-        d.C = L.C;
-        d.D = L.D;
-    }
-    if (hipMalloc(&c->mgldev, sizeof(MgLevelDev<double>) * ld.size()) != hipSuccess) {
-        delete m;
-        return fail(IH_ENOMEM, "out of device memory for the multigrid level descriptors");
-    }
-    HIPCHK(hipMemcpyAsync(c->mgldev, ld.data(), sizeof(MgLevelDev<double>) * ld.size(), hipMemcpyHostToDevice,
-                          c->stream));
-    m->Ldev = (const MgLevelDev<double> *)c->mgldev;
     c->mg_bytes = mg_alloc_bytes(c->mgh);
     c->bytes += c->mg_bytes;
     // launch shape of each level's sweep (a sweep is a pure function of its inputs)

@@ -30,33 +30,23 @@ struct MgLevel {
     JorLaunch shape32;
 };
 
-// A level as the fused coarse-level kernel reads it from device memory, for
-// the arithmetic type T of the cycle.
-template <typename T>
-struct MgLevelDev {
-    Geo g;
-    const T *dg[3];
-    const T *cR[3];
-    const T *cI[3];
-    int dn[3];
-    T *A, *B, *C, *D;
-};
-
 struct MgDev {
     int G = 0;
     int n_down = 4, n_up = 4, n_bottom = 4;
     double omega = 0.98;  // src/mod_laplace.f90:470
     MgLevel L[MG_LEVELS_MAX + 1];  // 1-based; level 1 uses the case's geometry and cdg
-    // levels g0..G run inside one single-workgroup launch (g0 > G: none);
-    // Ldev: device copy of levels 1..G (index 0 unused)
+    // levels g0..G run inside one single-workgroup launch (g0 > G: none)
     int g0 = MG_LEVELS_MAX + 1;
-    const MgLevelDev<double> *Ldev = nullptr;
-    const MgLevelDev<float> *Ldev32 = nullptr;
 };
-// points up to which a level runs inside the fused coarse-level launch
-// (one workgroup is latency-bound: a level of 2048 points takes two trips of
-// every step per thread, 9.5K points measured slower than its own launches)
-constexpr int64_t MG_FUSED_POINTS = 2048;
+// Levels that run inside the fused coarse-level launch: from the first with at most
+// MG_FUSED_POINTS points of its range (three a thread) whose arrays and tables, with
+// those of the coarser ones, fit MG_FUSED_LDS bytes of the workgroup's LDS.  A step
+// on a 97^3 grid with the limit at 2048, 3072 and 5120 points (13^3 = 2197 launched,
+// fused at three and at five points a thread): 54.7, 49.7, 50.1 ms; at 257x129x129
+// (17x9x9 in all three) 188.9, 189.2, 192.0.
+constexpr int64_t MG_FUSED_POINTS = 3072;
+constexpr int MG_FUSED_LDS = 128 * 1024;
+int mg_first_fused(const MgDev &m);  // that level; MG_LEVELS_MAX + 1: none
 
 // z = M v.  v's edges of wall pairs are averaged in place (restrict,
 // src/mod_solvers.f90:632-661), as the reference does to its pp and rr.

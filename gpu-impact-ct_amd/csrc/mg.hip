@@ -10,14 +10,15 @@
 // reference's operation order, so the cycle is bit-identical to the loop
 // restatement.
 //
-// Large levels run one launch per step (the JOR sweep of kernels.hip, and one
-// thread per output point for the rest).  A launch of a few-microsecond
-// kernel costs about as much as the work of a small level, so every level of
-// at most MG_FUSED_POINTS points runs inside one single-workgroup kernel that
-// walks the rest of the cycle with workgroup barriers between its steps.
+// Large levels run one launch per step (the JOR sweeps of kernels.hip, and one
+// thread per coarse point or cell for the transfers).  A launch of a few
+// microseconds costs about as much as the work of a small level, so the levels
+// from the first of at most MG_FUSED_POINTS points run inside one
+// single-workgroup kernel that walks the rest of the cycle in LDS.
 #include "ih_device.h"
 #include "ih_mg.h"
 
+#include <type_traits>
 #include <utility>
 
 namespace ih {
@@ -39,151 +40,82 @@ __device__ inline int64_t wix(const Geo &g, int i, int j, int k) {
     return gidx(g, wrapd(g, 0, i), wrapd(g, 1, j), wrapd(g, 2, k));
 }
 
-// ---- per-point steps (T: the arithmetic type of the cycle) -----------------
+// ---- per-point steps (T: the arithmetic type of the cycle)
 
 // first relaxation of a level (r == 1 with init_yes): rel = omega bb / diag
-// The per-point steps take their field pointers and coefficient tables as
-// template types: plain pointers from the launched kernels, global-qualified
-// ones from the fused kernel, which reads them from its level table (as plain
-// pointers the compiler could not tell they address global memory and would
-// emit flat accesses, which wait on both the vector-memory and LDS counters).
 template <typename T>
-using gptr = __attribute__((address_space(1))) T *;
-template <typename T>
-using gcptr = const __attribute__((address_space(1))) T *;
-
-template <typename T, typename TAB, typename PC, typename PM>
-__device__ inline void pt_init(const Geo &g, TAB dg, int i, int j, int k, T omega, PC bb, PM x) {
+__device__ inline void pt_init(const Geo &g, const T *const *dg, int i, int j, int k, T omega, const T *bb, T *x) {
     const int64_t p = gidx(g, i, j, k);
     const T d = (dg[0][g.cst[0] + i] + dg[1][g.cst[1] + j]) + dg[2][g.cst[2] + k];
     x[p] = omega * bb[p] / d;
 }
 
-// one Jacobi sweep point (src/mod_laplace.f90:514-518), out of place
-template <typename T, typename TAB, typename PC, typename PM>
-__device__ inline void pt_jor(const Geo &g, TAB dg, int i, int j, int k, T omega, PC x, PC bb, PM y) {
-    const int c0 = g.cst[0], c1 = g.cst[1], c2 = g.cst[2];
-    const int64_t p = gidx(g, i, j, k);
-    T t = bb[p];
-    t = t - dg[0][i] * x[wix(g, i - 1, j, k)];
-    t = t - dg[0][2 * c0 + i] * x[wix(g, i + 1, j, k)];
-    t = t - dg[1][j] * x[wix(g, i, j - 1, k)];
-    t = t - dg[1][2 * c1 + j] * x[wix(g, i, j + 1, k)];
-    t = t - dg[2][k] * x[wix(g, i, j, k - 1)];
-    t = t - dg[2][2 * c2 + k] * x[wix(g, i, j, k + 1)];
-    const T diag = (dg[0][c0 + i] + dg[1][c1 + j]) + dg[2][c2 + k];
-    y[p] = omega * t / diag + (T(1) - omega) * x[p];
-}
-
-// product_div_grad_relax (src/mod_laplace.f90:270-280)
-template <typename T, typename TAB, typename PC, typename PM>
-__device__ inline void pt_lap(const Geo &g, TAB dg, int i, int j, int k, PC x, PM lap) {
-    const int c0 = g.cst[0], c1 = g.cst[1], c2 = g.cst[2];
-    T t = dg[0][i] * x[wix(g, i - 1, j, k)];
-    t = t + dg[0][2 * c0 + i] * x[wix(g, i + 1, j, k)];
-    t = t + dg[1][j] * x[wix(g, i, j - 1, k)];
-    t = t + dg[1][2 * c1 + j] * x[wix(g, i, j + 1, k)];
-    t = t + dg[2][k] * x[wix(g, i, j, k - 1)];
-    t = t + dg[2][2 * c2 + k] * x[wix(g, i, j, k + 1)];
-    const int64_t p = gidx(g, i, j, k);
-    t = t + ((dg[0][c0 + i] + dg[1][c1 + j]) + dg[2][c2 + k]) * x[p];
-    lap[p] = t;
-}
-
-// restrict(.TRUE., g, coarse, bb, lap) at coarse point (ii, jj, kk)
-// (src/mod_solvers.f90:699-714); w: the coarse level's weights
-template <typename T, typename TAB, typename PC, typename PM>
-__device__ inline T pt_restrict(const Geo &gf, const Geo &gc, TAB w, const int *dd, int ii, int jj, int kk, PC bb,
-                                PC lap, PM out) {
-    const int i = dd[0] * (ii - 1) + 1, j = dd[1] * (jj - 1) + 1, k = dd[2] * (kk - 1) + 1;
-    auto df = [&](int a, int b, int c) {
-        const int64_t p = wix(gf, a, b, c);
-        return bb[p] - lap[p];
-    };
-    const int s1 = gc.cst[0], s2 = gc.cst[1], s3 = gc.cst[2];
-    T t = ((w[0][s1 + ii] + w[1][s2 + jj]) + w[2][s3 + kk]) * df(i, j, k);
-    t = t + w[0][ii] * df(i - 1, j, k);
-    t = t + w[0][2 * s1 + ii] * df(i + 1, j, k);
-    t = t + w[1][jj] * df(i, j - 1, k);
-    t = t + w[1][2 * s2 + jj] * df(i, j + 1, k);
-    t = t + w[2][kk] * df(i, j, k - 1);
-    t = t + w[2][2 * s3 + kk] * df(i, j, k + 1);
-    const T a = t / T(3);
-    out[gidx(gc, ii, jj, kk)] = a;
-    return a;
-}
-
-// interpolate(.TRUE., g, coarse, fine, work) at fine point (i, j, k)
-// (src/mod_solvers.f90:1046-1141): the injected coarse values, then the z, y
-// and x passes, evaluated with the operands each pass reads, added to fine;
-// w: the fine level's weights, dn: coarsening ratios
-template <typename T, typename TAB, typename PC, typename PM>
-__device__ inline void pt_interp(const Geo &gf, const Geo &gc, TAB w, const int *dn, int i, int j, int k, PC coarse,
-                                 PM x) {
-    auto lat = [&](int d, int t) { return dn[d] == 1 || ((t - 1) & 1) == 0; };
-    auto cix = [&](int d, int t) { return (t - 1) / dn[d] + 1; };
-    auto C = [&](int I, int J, int K) { return coarse[wix(gc, I, J, K)]; };
-    auto wz = [&](int a, int b, int c) {  // z pass (i, j on the coarse lattice)
-        const int I = cix(0, a), J = cix(1, b);
-        if (lat(2, c)) return C(I, J, cix(2, c));
-        const int K = c / 2;
-        return w[2][c] * C(I, J, K) + w[2][gf.cst[2] + c] * C(I, J, K + 1);
-    };
-    auto wy = [&](int a, int b, int c) {  // y pass (i on the lattice)
-        if (lat(1, b)) return wz(a, b, c);
-        return w[1][b] * wz(a, b - 1, c) + w[1][gf.cst[1] + b] * wz(a, b + 1, c);
-    };
-    T v;
-    if (lat(0, i))
-        v = wy(i, j, k);
-    else
-        v = w[0][i] * wy(i - 1, j, k) + w[0][gf.cst[0] + i] * wy(i + 1, j, k);
-    const int64_t p = gidx(gf, i, j, k);
-    x[p] = x[p] + v;
-}
-
 // Averaging on the edges of wall pairs, the reference's statements in order:
 // direction pairs (1,2), (1,3), (2,3), per pair the sides (L,L), (L,U), (U,L),
-// (U,U), each a line over 1..N of the third direction.  three = 0: two
-// neighbours / 2 (restrict, src/mod_solvers.f90:632-661); three = 1: three
-// neighbours / 3 (interpolate, :1028-1043).  Lines of one pair share no point
-// when every N >= 3, so a pair is one parallel step; pairs are ordered by
-// barriers (a later pair reads corners an earlier one wrote).  Runs on one
-// workgroup of nthr threads (tid); f2 may be null.
-template <typename T, typename PM = T *>
-__device__ inline void wg_edges(const Geo &g, PM f1, PM f2, int three, int tid, int nthr) {
-    const int pairs[3][3] = {{0, 1, 2}, {0, 2, 1}, {1, 2, 0}};
-    for (int pr = 0; pr < 3; ++pr) {
-        const int p = pairs[pr][0], q = pairs[pr][1], t = pairs[pr][2];
-        if (g.per[p] || g.per[q]) continue;
-        const int nt = g.N[t];
-        for (int u = tid; u < 4 * nt; u += nthr) {
-            const int side = u / nt, s = 1 + u - side * nt;
-            const int sp = side >> 1, sq = side & 1;
-            const int ep = sp ? g.N[p] : 1, ip = sp ? g.N[p] - 1 : 2;
-            const int eq = sq ? g.N[q] : 1, iq = sq ? g.N[q] - 1 : 2;
-            int e[3], a[3], b[3], cc[3];
-            e[p] = ep, e[q] = eq, e[t] = s;
-            a[p] = ip, a[q] = eq, a[t] = s;
-            b[p] = ep, b[q] = iq, b[t] = s;
-            cc[p] = ip, cc[q] = iq, cc[t] = s;
-            const int64_t pe = gidx(g, e[0], e[1], e[2]), pa = gidx(g, a[0], a[1], a[2]),
-                          pb = gidx(g, b[0], b[1], b[2]), pc = gidx(g, cc[0], cc[1], cc[2]);
-            // both fields' loads before either store: the loads of a pair never read a
-            // point that the pair writes, and f1 and f2 are different fields
-            T s1 = T(0), s2 = T(0);
-            if (three) {
-                if (f1) s1 = (f1[pa] + f1[pb] + f1[pc]) / T(3);
-                if (f2) s2 = (f2[pa] + f2[pb] + f2[pc]) / T(3);
-            } else {
-                if (f1) s1 = (f1[pa] + f1[pb]) / T(2);
-                if (f2) s2 = (f2[pa] + f2[pb]) / T(2);
-            }
-            if (f1) f1[pe] = s1;
-            if (f2) f2[pe] = s2;
-        }
-        __syncthreads();
+// (U,U), each a line over 1..N of the third direction.  THREE = false: two
+// neighbours / 2 (restrict, src/mod_solvers.f90:632-661); true: three neighbours
+// / 3 (interpolate, :1028-1043).
+// The pairs write only points with walls of two or more directions, and the last pair
+// to write a point reads points with fewer walls or ones that an earlier pair wrote
+// from such points, so the value after all three pairs is a function of the field
+// before them, of its points with at most one wall: a reader forms it where it needs
+// it, and it can be stored by one thread while others form theirs.  The corner's is
+// formed by the pair (2,3) from values that the pairs (1,3) and (1,2) left.
+template <typename T, bool THREE, typename F>
+__device__ inline T edge_value(const int *N, const bool *wall, int i, int j, int k, F f) {
+    const int ii = i == 1 ? 2 : N[0] - 1, jj = j == 1 ? 2 : N[1] - 1, kk = k == 1 ? 2 : N[2] - 1;
+    auto avg = [](T a, T b, T c) { return THREE ? (a + b + c) / T(3) : (a + b) / T(2); };
+    auto e01 = [&](int c) { return avg(f(ii, j, c), f(i, jj, c), THREE ? f(ii, jj, c) : T(0)); };
+    auto e02 = [&](int b) { return avg(f(ii, b, k), f(i, b, kk), THREE ? f(ii, b, kk) : T(0)); };
+    if (wall[1] && wall[2]) {
+        if (wall[0]) return avg(e02(jj), e01(kk), THREE ? f(i, jj, kk) : T(0));
+        return avg(f(i, jj, k), f(i, j, kk), THREE ? f(i, jj, kk) : T(0));
     }
+    return wall[2] ? e02(j) : e01(k);
+}
+
+// walls at (i, j, k), and whether they are two or more
+__device__ inline bool edge_point(const int *N, const int *per, int i, int j, int k, bool *wall) {
+    wall[0] = !per[0] && (i == 1 || i == N[0]);
+    wall[1] = !per[1] && (j == 1 || j == N[1]);
+    wall[2] = !per[2] && (k == 1 || k == N[2]);
+    return (int)wall[0] + (int)wall[1] + (int)wall[2] >= 2;
+}
+
+template <typename T, bool THREE>
+__device__ inline T edge_value(const Geo &g, int i, int j, int k, const T *f) {
+    bool w[3];
+    edge_point(g.N, g.per, i, j, k, w);
+    return edge_value<T, THREE>(g.N, w, i, j, k, [&](int a, int b, int c) { return f[gidx(g, a, b, c)]; });
+}
+
+// a point of a level's field as the averages need it: its walls, and the points that a
+// two-wall point is averaged from (inward along the one, the other and both walls'
+// directions; else the point itself), for loads without a branch
+struct EdgeAt {
+    int64_t p, a, b, c;
+    int walls;
+};
+__device__ inline EdgeAt edge_at(const Geo &g, int i, int j, int k) {
+    EdgeAt q;
+    bool w[3];
+    const bool in = i >= 1 && j >= 1 && k >= 1 && i <= g.N[0] && j <= g.N[1] && k <= g.N[2];
+    edge_point(g.N, g.per, i, j, k, w);
+    q.walls = in ? (int)w[0] + (int)w[1] + (int)w[2] : 0;
+    q.p = gidx(g, i, j, k);
+    const int64_t d0 = i == 1 ? 1 : -1, d1 = j == 1 ? g.px : -(int64_t)g.px, d2 = k == 1 ? g.pxy : -g.pxy;
+    const int64_t da = w[0] ? d0 : d1, db = w[2] ? d2 : d1;
+    q.a = q.walls == 2 ? q.p + da : q.p;
+    q.b = q.walls == 2 ? q.p + db : q.p;
+    q.c = q.walls == 2 ? q.p + da + db : q.p;
+    return q;
+}
+__device__ inline void point_of(const Geo &g, int64_t p, int &i, int &j, int &k) {
+    p -= g.lead;
+    k = (int)(p / g.pxy) - 3;
+    p -= (int64_t)(k + 3) * g.pxy;
+    j = (int)(p / g.px) - 3;
+    i = (int)(p - (int64_t)(j + 3) * g.px) - 3;
 }
 
 template <typename T>
@@ -219,34 +151,98 @@ __global__ void k_mg_init_f32_first(Geo g, Coef c, Range3 r, float omega, const 
 }
 
 
-// one workgroup of MG_EDGE_THREADS: the longest line set of the bench grid
-// (4 x 257 points) takes two passes
-constexpr int MG_EDGE_THREADS = 1024;
-
-template <typename T>
-__global__ __launch_bounds__(MG_EDGE_THREADS) void k_mg_edges(Geo g, T *f1, T *f2, int three, const int *active) {
-    if (active && !*active) return;
-    wg_edges<T>(g, f1, f2, three, (int)threadIdx.x, (int)blockDim.x);
-}
-
 template <typename T>
 struct LevelW {
     const T *w[3];
     int d[3];
 };
 
-// restriction; with xinit the coarse level's first relaxation as well
-// (omega A / diag at the same point, the value pt_init forms)
+// restrict(.TRUE., g, coarse, bb, lap) (src/mod_solvers.f90:632-714) by coarse points:
+// bb - lap on the seven fine points with both averaged on the edges; the averaged bb
+// (the later sweeps read it) is stored by the thread whose fine cell holds the point,
+// v's as well if given (the FP32 cycle's right-hand side is a copy of it).  With xinit
+// the coarse level's first relaxation too (omega A / diag at the same point, the value
+// pt_init forms).  Bound by latency but on level 1; with the averages in a launch of
+// their own, 7.8 + 5.7 microseconds over the levels of 257x129x129 (4.7 + 4.8 at 97^3),
+// here 11.7 (8.2).
 template <typename T>
-__global__ void k_mg_restrict(Geo gf, Geo gc, LevelW<T> R, Coef cc, Range3 r, const T *__restrict__ bb,
-                              const T *__restrict__ lap, T *__restrict__ out, T *__restrict__ xinit, T omega,
-                              const int *active) {
+__global__ __launch_bounds__(BX * BY) void k_mg_restrict(Geo gf, Geo gc, LevelW<T> R, Coef cc, Range3 r, T *bb, const T *__restrict__ lap,
+                              double *v, T *__restrict__ out, T *__restrict__ xinit, T omega, const int *active) {
     if (active && !*active) return;
     const int ii = r.lo0 + (int)(blockIdx.x * BX + threadIdx.x);
     const int jj = r.lo1 + (int)(blockIdx.y * BY + threadIdx.y);
     const int kk = r.lo2 + (int)blockIdx.z;
     if (ii >= r.lo0 + r.n0 || jj >= r.lo1 + r.n1) return;
-    const T a = pt_restrict<T>(gf, gc, R.w, R.d, ii, jj, kk, bb, lap, out);
+    const int i = R.d[0] * (ii - 1) + 1, j = R.d[1] * (jj - 1) + 1, k = R.d[2] * (kk - 1) + 1;
+    auto near_wall = [&](int d, int t) { return !gf.per[d] && (t <= 2 || t >= gf.N[d] - 1); };
+    T df[7];
+    auto raw = [&](int a, int b, int c) {
+        const int64_t p = wix(gf, a, b, c);
+        return bb[p] - lap[p];
+    };
+    if ((int)near_wall(0, i) + (int)near_wall(1, j) + (int)near_wall(2, k) < 2) {
+        df[0] = raw(i, j, k);
+        df[1] = raw(i - 1, j, k);
+        df[2] = raw(i + 1, j, k);
+        df[3] = raw(i, j - 1, k);
+        df[4] = raw(i, j + 1, k);
+        df[5] = raw(i, j, k - 1);
+        df[6] = raw(i, j, k + 1);
+    } else {
+        // all loads first: an edge point's two neighbours, else the point twice
+        EdgeAt q[7];
+        T fa[7], fb[7], la[7], lb[7];
+#pragma unroll
+        for (int e = 0; e < 7; ++e) {
+            q[e] = edge_at(gf, wrapd(gf, 0, i + (e == 2) - (e == 1)), wrapd(gf, 1, j + (e == 4) - (e == 3)),
+                           wrapd(gf, 2, k + (e == 6) - (e == 5)));
+            fa[e] = bb[q[e].a];
+            fb[e] = bb[q[e].b];
+            la[e] = lap[q[e].a];
+            lb[e] = lap[q[e].b];
+        }
+        auto store = [&](int64_t p, T value) {
+            bb[p] = value;
+            if (v) {
+                int a, b, c;
+                point_of(gf, p, a, b, c);
+                v[p] = edge_value<double, false>(gf, a, b, c, v);
+            }
+        };
+#pragma unroll
+        for (int e = 0; e < 7; ++e) {
+            T f = q[e].walls == 2 ? (fa[e] + fb[e]) / T(2) : fa[e], l = q[e].walls == 2 ? (la[e] + lb[e]) / T(2) : la[e];
+            if (q[e].walls == 3) {
+                int a, b, c;
+                point_of(gf, q[e].a, a, b, c);
+                f = edge_value<T, false>(gf, a, b, c, bb);
+                l = edge_value<T, false>(gf, a, b, c, lap);
+            }
+            df[e] = f - l;
+            // the thread's fine points: its own and, along a halved direction, the next
+            if (q[e].walls >= 2 && (e == 0 || (e % 2 == 0 && R.d[e / 2 - 1] == 2 && (e == 2 ? i : e == 4 ? j : k) < gf.N[e / 2 - 1])))
+                store(q[e].p, f);
+        }
+        // the last point along a periodic direction: no level reads it, its average is
+        // part of the field all the same
+        if (q[0].walls == 2) {
+            const bool last[3] = {ii == r.lo0 + r.n0 - 1, jj == r.lo1 + r.n1 - 1, kk == r.lo2 + r.n2 - 1};
+            for (int d = 0; d < 3; ++d) {
+                if (!gf.per[d] || !last[d]) continue;
+                const int a = d == 0 ? gf.N[0] : i, b = d == 1 ? gf.N[1] : j, c = d == 2 ? gf.N[2] : k;
+                store(gidx(gf, a, b, c), edge_value<T, false>(gf, a, b, c, bb));
+            }
+        }
+    }
+    const int s1 = gc.cst[0], s2 = gc.cst[1], s3 = gc.cst[2];
+    const T *const *w = R.w;
+    const T wc = (w[0][s1 + ii] + w[1][s2 + jj]) + w[2][s3 + kk];
+    const T wn[6] = {w[0][ii], w[0][2 * s1 + ii], w[1][jj], w[1][2 * s2 + jj], w[2][kk], w[2][2 * s3 + kk]};
+    T t = wc * df[0];
+#pragma unroll
+    for (int e = 0; e < 6; ++e) t = t + wn[e] * df[1 + e];
+    const T a = t / T(3);
+    out[gidx(gc, ii, jj, kk)] = a;
     if (xinit) {
         const T *const *dg = dg_of<T>(cc);
         const T d = (dg[0][gc.cst[0] + ii] + dg[1][gc.cst[1] + jj]) + dg[2][gc.cst[2] + kk];
@@ -254,12 +250,15 @@ __global__ void k_mg_restrict(Geo gf, Geo gc, LevelW<T> R, Coef cc, Range3 r, co
     }
 }
 
-// interpolate-and-add by coarse cells: the thread of cell (I, J, K) writes the
-// fine points dn*(T-1)+1+s, s < dn (s = 0 only at T = Nc), from the eight
-// coarse values around it; every fine value is formed with pt_interp's
-// operands and order
+// interpolate(.TRUE., g, coarse, fine, work) (src/mod_solvers.f90:1028-1141) added to
+// fine, by coarse cells: the thread of cell (I, J, K) writes the fine points
+// dn*(T-1)+1+s, s < dn (s = 0 only at T = Nc), from the eight coarse values around it
+// (averaged on the edges; nothing else reads those, so they are not stored): the
+// injected values, then the z, y and x passes with the operands each pass reads.
+// 8.9 + 5.7 microseconds over the levels of 257x129x129 with the averages in a launch
+// of their own, here 11.9 (97^3: 6.2 + 4.8, here 9.5)
 template <typename T>
-__global__ void k_mg_interp_cells(Geo gf, Geo gc, LevelW<T> W, const T *__restrict__ coarse, T *__restrict__ x,
+__global__ __launch_bounds__(BX * BY) void k_mg_interp_cells(Geo gf, Geo gc, LevelW<T> W, const T *__restrict__ coarse, T *__restrict__ fine,
                                   const int *active) {
     if (active && !*active) return;
     const int I = 1 + (int)(blockIdx.x * BX + threadIdx.x);
@@ -271,32 +270,72 @@ __global__ void k_mg_interp_cells(Geo gf, Geo gc, LevelW<T> W, const T *__restri
     for (int d = 0; d < 3; ++d) ns[d] = (W.d[d] == 2 && Tc[d] < gc.N[d]) ? 2 : 1;
     // coarse values at (I + a, J + b, K + e); a direction with one fine point
     // per cell reads index 0 only
-    T cv[2][2][2];
-    for (int e = 0; e < 2; ++e)
-        for (int b = 0; b < 2; ++b)
-            for (int a = 0; a < 2; ++a)
-                cv[a][b][e] = coarse[wix(gc, I + (a < ns[0] ? a : 0), J + (b < ns[1] ? b : 0), K + (e < ns[2] ? e : 0))];
     const int i0 = W.d[0] * (I - 1) + 1, j0 = W.d[1] * (J - 1) + 1, k0 = W.d[2] * (K - 1) + 1;
-    const T *w1 = W.w[0], *w2 = W.w[1], *w3 = W.w[2];
     const int s1 = gf.cst[0], s2 = gf.cst[1], s3 = gf.cst[2];
-    for (int se = 0; se < ns[2]; ++se) {
-        const int k = k0 + se;
+    // the weights of the points off the lattice and the fine values do not wait for the
+    // coarse ones
+    const int ix = i0 + ns[0] - 1, jx = j0 + ns[1] - 1, kx = k0 + ns[2] - 1;
+    const T w1a = W.w[0][ix], w1b = W.w[0][s1 + ix], w2a = W.w[1][jx], w2b = W.w[1][s2 + jx], w3a = W.w[2][kx],
+            w3b = W.w[2][s3 + kx];
+    typedef T T2 __attribute__((ext_vector_type(2)));
+    T2 fv[2][2];  // i0 is odd where a direction is halved: a pair of points is aligned
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const T *const f = fine + gidx(gf, i0, j0 + ((q & 1) < ns[1] ? q & 1 : 0), k0 + (q >> 1 < ns[2] ? q >> 1 : 0));
+        if (ns[0] == 2)
+            fv[q & 1][q >> 1] = *(const T2 *)f;
+        else
+            fv[q & 1][q >> 1] = T2{*f, T(0)};
+    }
+    T cv[2][2][2];
+    auto near_wall = [&](int d, int t) { return !gc.per[d] && (t == 1 || t >= gc.N[d] - 1); };
+    const bool edges = (int)near_wall(0, I) + (int)near_wall(1, J) + (int)near_wall(2, K) >= 2;
+    auto corner = [&](int q, int d) { return Tc[d] + ((q >> d & 1) < ns[d] ? q >> d & 1 : 0); };
+    if (!edges) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            cv[q & 1][q >> 1 & 1][q >> 2] = coarse[wix(gc, corner(q, 0), corner(q, 1), corner(q, 2))];
+    } else {
+        T f[8][3];
+        int walls[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const EdgeAt at =
+                edge_at(gc, wrapd(gc, 0, corner(q, 0)), wrapd(gc, 1, corner(q, 1)), wrapd(gc, 2, corner(q, 2)));
+            walls[q] = at.walls;
+            f[q][0] = coarse[at.a];
+            f[q][1] = coarse[at.b];
+            f[q][2] = coarse[at.c];
+        }
+        T three = T(0);  // a cell has one point on three walls at most
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) any = any || walls[q] == 3;
+        if (any)
+            three = edge_value<T, true>(gc, I == 1 ? 1 : gc.N[0], J == 1 ? 1 : gc.N[1], K == 1 ? 1 : gc.N[2], coarse);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            cv[q & 1][q >> 1 & 1][q >> 2] =
+                walls[q] == 3 ? three : (walls[q] == 2 ? (f[q][0] + f[q][1] + f[q][2]) / T(3) : f[q][0]);
+    }
+#pragma unroll
+    for (int se = 0; se < 2; ++se) {
         // z pass at the four lattice columns (a, b)
         T wz[2][2];
         for (int b = 0; b < 2; ++b)
-            for (int a = 0; a < 2; ++a)
-                wz[a][b] = se == 0 ? cv[a][b][0] : w3[k] * cv[a][b][0] + w3[s3 + k] * cv[a][b][1];
-        for (int sb = 0; sb < ns[1]; ++sb) {
-            const int j = j0 + sb;
+            for (int a = 0; a < 2; ++a) wz[a][b] = se == 0 ? cv[a][b][0] : w3a * cv[a][b][0] + w3b * cv[a][b][1];
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb) {
+            if (se >= ns[2] || sb >= ns[1]) continue;
             // y pass at the two lattice x positions
             T wy[2];
-            for (int a = 0; a < 2; ++a) wy[a] = sb == 0 ? wz[a][0] : w2[j] * wz[a][0] + w2[s2 + j] * wz[a][1];
-            for (int sa = 0; sa < ns[0]; ++sa) {
-                const int i = i0 + sa;
-                const T v = sa == 0 ? wy[0] : w1[i] * wy[0] + w1[s1 + i] * wy[1];
-                const int64_t p = gidx(gf, i, j, k);
-                x[p] = x[p] + v;
-            }
+            for (int a = 0; a < 2; ++a) wy[a] = sb == 0 ? wz[a][0] : w2a * wz[a][0] + w2b * wz[a][1];
+            T *const f = fine + gidx(gf, i0, j0 + sb, k0 + se);
+            const T2 v = {fv[sb][se][0] + wy[0], fv[sb][se][1] + (w1a * wy[0] + w1b * wy[1])};
+            if (ns[0] == 2)
+                *(T2 *)f = v;
+            else
+                *f = v[0];
         }
     }
 }
@@ -304,96 +343,299 @@ __global__ void k_mg_interp_cells(Geo gf, Geo gc, LevelW<T> W, const T *__restri
 // ---- levels g0..G in one workgroup ------------------------------------------
 
 constexpr int MG_FUSED_THREADS = 1024;
+constexpr int MG_FUSED_OWN = (int)(MG_FUSED_POINTS / MG_FUSED_THREADS);  // points of a level a thread owns
 
-// every point of [lo, lo + n) (three directions) once, over the workgroup
-template <typename F>
-__device__ inline void wg_points(const int *lo, const int *n, F f) {
-    const int tot = n[0] * n[1] * n[2];
-    for (int q = (int)threadIdx.x; q < tot; q += MG_FUSED_THREADS) {
-        const int a = q % n[0], r = q / n[0];
-        const int b = r % n[1], c = r / n[1];
-        f(lo[0] + a, lo[1] + b, lo[2] + c);
-    }
-    __syncthreads();
-}
+struct MgFusedLevel {
+    int P[3], N[3], dn[3], cst[3];  // points of the range, sizes, ratios to the next level, table strides
+    int tab;                        // its tables: per direction dg, cR (3 cst) and cI (2 cst)
+    int A, X;                       // right-hand side and iterate in the pool (X[0] is a zero, points from X[1])
+};
+struct MgFusedArgs {
+    MgFusedLevel L[MG_LEVELS_MAX + 1];
+    Geo g;  // of level g0
+    int g0, G, n_down, n_up, n_bottom;
+    int per[3];
+    int ntab, tmp;  // table elements (from 0 in the pool), the second iterate of any level (as X)
+};
 
-// the rest of the cycle from level g0: its right-hand side A is in place; the
-// iterate of g0 ends in B or D as the host's account of the same swaps says
+// The rest of the cycle from level g0: its right-hand side A is in place, its last
+// iterate goes to out.  Everything lives in LDS: the tables, and per level the points
+// of the pressure range without halos (a neighbour past a wall is the zero in front of
+// the iterate, one across a periodic pair the wrapped point).  A thread owns the same
+// points of a level through all its steps, with their coefficients, neighbours and
+// right-hand side in registers, so a sweep is seven LDS reads, the point's chain and a
+// barrier.  One workgroup's chain of about 40 steps a cycle: the latency of a step, and
+// the one compute unit's issue on its larger levels, bound it.  17x9x9 and coarser:
+// 111 -> 31 microseconds with the fields in LDS instead of the levels' arrays.
 template <typename T>
-__global__ __launch_bounds__(MG_FUSED_THREADS) void k_mg_fused(const MgLevelDev<T> *__restrict__ L, int g0, int G,
-                                                               int n_down, int n_up, int n_bottom, T omega,
+__global__ __launch_bounds__(MG_FUSED_THREADS) void k_mg_fused(MgFusedArgs args, const T *__restrict__ tables,
+                                                               const T *__restrict__ Ag, T *__restrict__ out, T omega,
                                                                const int *active) {
     if (active && !*active) return;
+    __shared__ T pool[MG_FUSED_LDS / sizeof(T)];
+    // the levels are indexed where they are passed (a reference to the parameter would
+    // be a copy of it in scratch memory)
+    (void)args;
+    const auto *const a =
+        (const __attribute__((address_space(4))) MgFusedArgs *)__builtin_amdgcn_kernarg_segment_ptr();
     const int tid = (int)threadIdx.x;
-    gptr<T> x[MG_LEVELS_MAX + 1], y[MG_LEVELS_MAX + 1];
-    for (int g = g0; g <= G; ++g) {
-        x[g] = (gptr<T>)L[g].B;
-        y[g] = (gptr<T>)L[g].D;
-    }
-    // a level's coefficient tables as global pointers
-    struct Tab {
-        gcptr<T> t[3];
+    const int g0 = a->g0, G = a->G, n_down = a->n_down, n_up = a->n_up, n_bottom = a->n_bottom, tmp = a->tmp;
+    const int per[3] = {a->per[0], a->per[1], a->per[2]};
+    constexpr int OWN = MG_FUSED_OWN;
+    // an owned point: its neighbours (a direction's two, 16 bits each, from the iterate's
+    // zero), coefficients, diagonal and right-hand side
+    struct Own {
+        unsigned nb[3];
+        T c[6], d, A;
     };
-    auto tab = [](const T *const *w) {
-        Tab r;
-        for (int d = 0; d < 3; ++d) r.t[d] = (gcptr<T>)w[d];
-        return r;
+    Own o[OWN];
+    struct Level {
+        int P[3], N[3], dn[3], cst[3], tab, A, X, n;
     };
-    auto range = [&](int g, int *lo, int *n) {
+    auto level = [&](int g) {
+        const auto &q = a->L[g];
+        Level l;
         for (int d = 0; d < 3; ++d) {
-            lo[d] = L[g].g.Sp[d];
-            n[d] = L[g].g.Np[d] - L[g].g.Sp[d] + 1;
+            l.P[d] = q.P[d];
+            l.N[d] = q.N[d];
+            l.dn[d] = q.dn[d];
+            l.cst[d] = q.cst[d];
         }
+        l.tab = q.tab;
+        l.A = q.A;
+        l.X = q.X;
+        l.n = l.P[0] * l.P[1] * l.P[2];
+        return l;
     };
-    auto relax = [&](int g, bool init, int nr) {
-        const MgLevelDev<T> &l = L[g];
-        int lo[3], n[3];
-        range(g, lo, n);
-        const Tab dg = tab(l.dg);
-        const gcptr<T> A = (gcptr<T>)l.A;
-        int q = 1;
-        if (init && nr >= 1) {
-            gptr<T> xx = x[g];
-            wg_points(lo, n, [&](int i, int j, int k) { pt_init<T>(l.g, dg.t, i, j, k, omega, A, xx); });
-            q = 2;
-        }
-        for (; q <= nr; ++q) {
-            const gcptr<T> xx = x[g];
-            gptr<T> yy = y[g];
-            wg_points(lo, n, [&](int i, int j, int k) { pt_jor<T>(l.g, dg.t, i, j, k, omega, xx, A, yy); });
-            gptr<T> tmp = x[g];
-            x[g] = y[g];
-            y[g] = tmp;
-        }
+    auto split = [](const Level &l, int q, int &i, int &j, int &k) {
+        const int r = q / l.P[0];
+        i = 1 + q - r * l.P[0];
+        k = 1 + r / l.P[1];
+        j = 1 + r - (k - 1) * l.P[1];
     };
-    for (int g = g0; g <= G - 1; ++g) {
-        const MgLevelDev<T> &l = L[g], &lc = L[g + 1];
-        relax(g, true, n_down);
-        int lo[3], n[3];
-        range(g, lo, n);
-        const gcptr<T> xx = x[g];
-        const Tab dg = tab(l.dg), cR = tab(lc.cR);
-        const gptr<T> A = (gptr<T>)l.A, Cl = (gptr<T>)l.C, Ac = (gptr<T>)lc.A;
-        wg_points(lo, n, [&](int i, int j, int k) { pt_lap<T>(l.g, dg.t, i, j, k, xx, Cl); });
-        wg_edges<T, gptr<T>>(l.g, A, Cl, 0, tid, MG_FUSED_THREADS);
-        int clo[3] = {1, 1, 1}, cn[3];
-        for (int d = 0; d < 3; ++d) cn[d] = lc.g.N[d] - (l.g.per[d] ? 1 : 0);
-        wg_points(clo, cn, [&](int ii, int jj, int kk) {
-            pt_restrict<T>(l.g, lc.g, cR.t, l.dn, ii, jj, kk, (gcptr<T>)A, (gcptr<T>)Cl, Ac);
-        });
+    const int lead = a->g.lead, px = a->g.px;
+    const int64_t pxy = a->g.pxy;
+    auto at = [&](int i, int j, int k) {  // gidx
+        return lead + (i + 3) + (int64_t)px * (j + 3) + pxy * (k + 3);
+    };
+    for (int t = tid; t < a->ntab; t += MG_FUSED_THREADS) pool[t] = tables[t];
+    if (tid == 0) {
+        for (int g = g0; g <= G; ++g) pool[a->L[g].X] = T(0);
+        pool[tmp] = T(0);
     }
-    relax(G, true, n_bottom);
-    relax(G, false, n_bottom);
+    {
+        const Level l = level(g0);
+        for (int q = tid; q < l.n; q += MG_FUSED_THREADS) {
+            int i, j, k;
+            split(l, q, i, j, k);
+            pool[l.A + q] = Ag[at(i, j, k)];
+        }
+    }
+    __syncthreads();
+    auto enter = [&](const Level &l) {
+        const T *const t0 = pool + l.tab, *const t1 = t0 + 8 * l.cst[0], *const t2 = t1 + 8 * l.cst[1];
+#pragma unroll
+        for (int m = 0; m < OWN; ++m) {
+            const int q = tid + m * MG_FUSED_THREADS;
+            if (q >= l.n) continue;
+            Own &p = o[m];
+            int i, j, k;
+            split(l, q, i, j, k);
+            auto nb = [&](int x, int P, int pr, int stride) {
+                const int lo = x > 1 ? q + 1 - stride : (pr ? q + 1 + (P - 1) * stride : 0);
+                const int hi = x < P ? q + 1 + stride : (pr ? q + 1 - (P - 1) * stride : 0);
+                return (unsigned)(lo | hi << 16);
+            };
+            p.nb[0] = nb(i, l.P[0], per[0], 1);
+            p.nb[1] = nb(j, l.P[1], per[1], l.P[0]);
+            p.nb[2] = nb(k, l.P[2], per[2], l.P[0] * l.P[1]);
+            p.c[0] = t0[i];
+            p.c[1] = t0[2 * l.cst[0] + i];
+            p.c[2] = t1[j];
+            p.c[3] = t1[2 * l.cst[1] + j];
+            p.c[4] = t2[k];
+            p.c[5] = t2[2 * l.cst[2] + k];
+            p.d = (t0[l.cst[0] + i] + t1[l.cst[1] + j]) + t2[l.cst[2] + k];
+            p.A = pool[l.A + q];
+        }
+    };
+    auto nbr = [](const Own &p, int e) { return (int)(e & 1 ? p.nb[e >> 1] >> 16 : p.nb[e >> 1] & 0xffffu); };
+    int x = 0, y = 0;  // the level's iterate and the other buffer
+    auto sweeps = [&](const Level &l, int n) {
+        for (; n > 0; --n) {
+#pragma unroll
+            for (int m = 0; m < OWN; ++m) {
+                const int q = tid + m * MG_FUSED_THREADS;
+                if (q >= l.n) continue;
+                const Own &p = o[m];
+                T v[6];
+#pragma unroll
+                for (int e = 0; e < 6; ++e) v[e] = pool[x + nbr(p, e)];
+                const T own = pool[x + q + 1];
+                T t = p.A;
+#pragma unroll
+                for (int e = 0; e < 6; ++e) t = t - p.c[e] * v[e];
+                pool[y + q + 1] = omega * t / p.d + (T(1) - omega) * own;
+            }
+            __syncthreads();
+            const int z = x;
+            x = y;
+            y = z;
+        }
+    };
+    // the first relaxation, from zero; flips: the sweeps that follow before the iterate
+    // has to be in X
+    auto first = [&](const Level &l, int flips) {
+        x = flips & 1 ? tmp : l.X;
+        y = flips & 1 ? l.X : tmp;
+#pragma unroll
+        for (int m = 0; m < OWN; ++m) {
+            const int q = tid + m * MG_FUSED_THREADS;
+            if (q < l.n) pool[x + q + 1] = omega * o[m].A / o[m].d;
+        }
+        __syncthreads();
+    };
+    // the averages on the edges of the arrays at f1 and (if >= 0) f2
+    auto edges = [&](const Level &l, auto three, int f1, int f2) {
+        for (int q = tid; q < l.n; q += MG_FUSED_THREADS) {
+            int i, j, k;
+            split(l, q, i, j, k);
+            bool w[3];
+            if (!edge_point(l.N, per, i, j, k, w)) continue;
+            for (int f = f1; f >= 0; f = f == f1 ? f2 : -1)
+                pool[f + q] = edge_value<T, decltype(three)::value>(l.N, w, i, j, k, [&](int u, int v, int t) {
+                    return pool[f + (u - 1) + l.P[0] * ((v - 1) + l.P[1] * (t - 1))];
+                });
+        }
+        __syncthreads();
+    };
+    Level l = level(g0);
+    for (int g = g0; g < G; ++g) {
+        const Level lc = level(g + 1);
+        enter(l);
+        first(l, n_down - 1);
+        sweeps(l, n_down - 1);
+        // the residual product, then the averages on the edges of it and of A
+        const int A = l.A, C = tmp + 1;
+#pragma unroll
+        for (int m = 0; m < OWN; ++m) {
+            const int q = tid + m * MG_FUSED_THREADS;
+            if (q >= l.n) continue;
+            const Own &p = o[m];
+            T t = p.c[0] * pool[l.X + nbr(p, 0)];
+#pragma unroll
+            for (int e = 1; e < 6; ++e) t = t + p.c[e] * pool[l.X + nbr(p, e)];
+            pool[C + q] = t + p.d * pool[l.X + q + 1];
+        }
+        __syncthreads();
+        edges(l, std::false_type{}, A, C);
+        // A - C on the points of the coarse level
+        const T *const w0 = pool + lc.tab + 3 * lc.cst[0], *const w1 = w0 + 5 * lc.cst[0] + 3 * lc.cst[1],
+                       *const w2 = w1 + 5 * lc.cst[1] + 3 * lc.cst[2];
+        for (int q = tid; q < lc.n; q += MG_FUSED_THREADS) {
+            int ii, jj, kk;
+            split(lc, q, ii, jj, kk);
+            const int st1 = l.P[0], st2 = l.P[0] * l.P[1];
+            const int c0 = l.dn[0] * (ii - 1), c1 = l.dn[1] * (jj - 1), c2 = l.dn[2] * (kk - 1);  // from 0
+            const int p = c0 + st1 * c1 + st2 * c2;
+            auto lo = [&](int c, int P, int pr, int st) { return c > 0 ? p - st : (pr ? p + (P - 1) * st : -1); };
+            auto hi = [&](int c, int P, int pr, int st) { return c < P - 1 ? p + st : (pr ? p - (P - 1) * st : -1); };
+            auto df = [&](int u) { return u < 0 ? T(0) : pool[A + u] - pool[C + u]; };
+            T t = ((w0[lc.cst[0] + ii] + w1[lc.cst[1] + jj]) + w2[lc.cst[2] + kk]) * df(p);
+            t = t + w0[ii] * df(lo(c0, l.P[0], per[0], 1));
+            t = t + w0[2 * lc.cst[0] + ii] * df(hi(c0, l.P[0], per[0], 1));
+            t = t + w1[jj] * df(lo(c1, l.P[1], per[1], st1));
+            t = t + w1[2 * lc.cst[1] + jj] * df(hi(c1, l.P[1], per[1], st1));
+            t = t + w2[kk] * df(lo(c2, l.P[2], per[2], st2));
+            t = t + w2[2 * lc.cst[2] + kk] * df(hi(c2, l.P[2], per[2], st2));
+            pool[lc.A + q] = t / T(3);
+        }
+        __syncthreads();
+        l = lc;
+    }
+    enter(l);
+    first(l, 0);
+    sweeps(l, 2 * n_bottom - 1);
     for (int g = G - 1; g >= g0; --g) {
-        const MgLevelDev<T> &l = L[g], &lc = L[g + 1];
-        wg_edges<T, gptr<T>>(lc.g, x[g + 1], (gptr<T>)nullptr, 1, tid, MG_FUSED_THREADS);
-        int flo[3] = {1, 1, 1}, fn[3] = {l.g.N[0], l.g.N[1], l.g.N[2]};
-        const gcptr<T> co = x[g + 1];
-        gptr<T> xx = x[g];
-        const Tab cI = tab(l.cI);
-        wg_points(flo, fn, [&](int i, int j, int k) { pt_interp<T>(l.g, lc.g, cI.t, l.dn, i, j, k, co, xx); });
-        relax(g, false, n_up);
+        const Level lc = l;
+        l = level(g);
+        const int xc = x + 1;
+        edges(lc, std::true_type{}, xc, -1);
+        enter(l);
+        const T *const i0 = pool + l.tab + 6 * l.cst[0], *const i1 = i0 + 2 * l.cst[0] + 6 * l.cst[1],
+                       *const i2 = i1 + 2 * l.cst[1] + 6 * l.cst[2];
+        for (int q = tid; q < l.n; q += MG_FUSED_THREADS) {
+            int i, j, k;
+            split(l, q, i, j, k);
+            // a direction's coarse neighbours below and above; the same one on the lattice
+            auto below = [](int t, int dn) { return (t - 1) >> (dn - 1); };  // from 0
+            auto above = [](int b, bool on, int P) { return on ? b : (b + 1 < P ? b + 1 : 0); };
+            const bool li = l.dn[0] == 1 || (i & 1), lj = l.dn[1] == 1 || (j & 1), lk = l.dn[2] == 1 || (k & 1);
+            const int I0 = below(i, l.dn[0]), J0 = below(j, l.dn[1]), K0 = below(k, l.dn[2]);
+            const int I1 = above(I0, li, lc.P[0]), J1 = above(J0, lj, lc.P[1]), K1 = above(K0, lk, lc.P[2]);
+            const T k0 = i2[k], k1 = i2[l.cst[2] + k], j0 = i1[j], j1 = i1[l.cst[1] + j], x0 = i0[i],
+                    x1 = i0[l.cst[0] + i];
+            auto wz = [&](int I, int J) {
+                const int r = xc + I + lc.P[0] * J, s2 = lc.P[0] * lc.P[1];
+                const T lo = pool[r + s2 * K0], hi = pool[r + s2 * K1];
+                return lk ? lo : k0 * lo + k1 * hi;
+            };
+            auto wy = [&](int I) {
+                const T lo = wz(I, J0), hi = wz(I, J1);
+                return lj ? lo : j0 * lo + j1 * hi;
+            };
+            const T lo = wy(I0), hi = wy(I1);
+            pool[l.X + q + 1] = pool[l.X + q + 1] + (li ? lo : x0 * lo + x1 * hi);
+        }
+        __syncthreads();
+        x = l.X;
+        y = tmp;
+        sweeps(l, n_up);
     }
+    for (int q = tid; q < l.n; q += MG_FUSED_THREADS) {
+        int i, j, k;
+        split(l, q, i, j, k);
+        out[at(i, j, k)] = pool[x + q + 1];
+    }
+}
+
+// the layout of levels g0..G in the pool; false if it does not fit
+bool fused_layout(const MgDev &m, int g0, MgFusedArgs &a) {
+    a = MgFusedArgs{};
+    a.g0 = g0;
+    a.G = m.G;
+    a.n_down = m.n_down;
+    a.n_up = m.n_up;
+    a.n_bottom = m.n_bottom;
+    a.g = m.L[g0].g;
+    int64_t at = 0, most = 0;
+    for (int g = g0; g <= m.G; ++g) {
+        MgFusedLevel &l = a.L[g];
+        l.tab = (int)at;
+        for (int d = 0; d < 3; ++d) {
+            const Geo &q = m.L[g].g;
+            l.P[d] = q.Np[d] - q.Sp[d] + 1;
+            l.N[d] = q.N[d];
+            l.dn[d] = m.L[g].dn[d];
+            l.cst[d] = q.cst[d];
+            a.per[d] = q.per[d];
+            at += 8 * l.cst[d];
+        }
+    }
+    a.ntab = (int)at;
+    for (int g = g0; g <= m.G; ++g) {
+        MgFusedLevel &l = a.L[g];
+        const int64_t n = (int64_t)l.P[0] * l.P[1] * l.P[2];
+        if (n > MG_FUSED_POINTS || l.P[0] > 1023 || l.P[1] > 1023 || l.P[2] > 1023) return false;
+        most = std::max(most, n);
+        l.A = (int)at;
+        at += n;
+        l.X = (int)at;
+        at += n + 1;
+    }
+    a.tmp = (int)at;
+    at += most + 1;
+    return at * (int64_t)sizeof(double) <= MG_FUSED_LDS;
 }
 
 inline Range3 full_range(const Geo &g) { return Range3{1, 1, 1, g.N[0], g.N[1], g.N[2]}; }
@@ -413,7 +655,7 @@ struct CycleBufs<double> {
     static const double *const *cR(const MgLevel &L) { return L.cR; }
     static const double *const *cI(const MgLevel &L) { return L.cI; }
     static JorLaunch shape(const MgLevel &L) { return L.shape; }
-    static const MgLevelDev<double> *dev(const MgDev &m) { return m.Ldev; }
+    static const double *tables(const MgLevel &L) { return L.c.dg[0]; }
 };
 template <>
 struct CycleBufs<float> {
@@ -424,7 +666,7 @@ struct CycleBufs<float> {
     static const float *const *cR(const MgLevel &L) { return L.cRf; }
     static const float *const *cI(const MgLevel &L) { return L.cIf; }
     static JorLaunch shape(const MgLevel &L) { return L.shape32; }
-    static const MgLevelDev<float> *dev(const MgDev &m) { return m.Ldev32; }
+    static const float *tables(const MgLevel &L) { return L.c.dgf[0]; }
 };
 
 // launches of n sweeps of a level: two a launch where its range takes pairs
@@ -467,15 +709,14 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
         x[g] = B_::B(m.L[g]);
         y[g] = B_::D(m.L[g]);
     }
-    // relaxation of level g; launch = false only follows the swaps (the fused kernel
-    // runs them); init_done: the restriction into g already wrote the first
+    // relaxation of level g; init_done: the restriction into g already wrote the first
     // relaxation; last_to_z: the FP32 cycle's final sweep, written to z as double
-    auto relax = [&](int g, bool init, int n, bool launch, bool init_done = false, bool last_to_z = false) {
+    auto relax = [&](int g, bool init, int n, bool init_done = false, bool last_to_z = false) {
         const MgLevel &L = m.L[g];
         const Range3 r = make_range(L.pr);
         int q = 1;
         if (init && n >= 1) {
-            if (launch && !init_done) {
+            if (!init_done) {
                 if (!fp64 && g == 1)
                     hipLaunchKernelGGL(k_mg_init_f32_first, grid_for(r), dim3(BX, BY, 1), 0, s, L.g, L.c, r,
                                        (float)omega, (const double *)v, (float *)b[1], (float *)x[1], act);
@@ -485,17 +726,17 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
             }
             q = 2;
         }
-        const bool pairs = launch && level_pairs(L, !fp64);
+        const bool pairs = level_pairs(L, !fp64);
         while (q <= n) {
             const int two = pairs && (n - q) % 2 == 1 ? 2 : 1;  // an odd count's single sweep comes first
             q += two;
             const bool to_z = last_to_z && q > n;
-            if (launch && two == 2) {
+            if (two == 2) {
                 if (to_z)
                     launch_jor_pair(s, L.g, L.c, L.pr, (float)omega, (const float *)x[g], (const float *)b[g], z, act);
                 else
                     launch_jor_pair(s, L.g, L.c, L.pr, omega, (const T *)x[g], (const T *)b[g], y[g], act);
-            } else if (launch) {
+            } else {
                 if (to_z)
                     launch_jor_f32_to64(s, L.g, L.c, L.pr, (float)omega, (const float *)x[g], (const float *)b[g], z,
                                         act, B_::shape(L));
@@ -506,25 +747,17 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
         }
     };
     if (G == 1) {
-        relax(1, true, m.n_bottom, true);
-        relax(1, false, m.n_bottom, true, false, !fp64);
+        relax(1, true, m.n_bottom);
+        relax(1, false, m.n_bottom, false, !fp64);
         return;
     }
     const int gl = std::min(g0, G) - 1;  // last level with launches of its own on the way down
     for (int g = 1; g <= gl; ++g) {
         const MgLevel &L = m.L[g], &Lc = m.L[g + 1];
-        relax(g, true, m.n_down, true, g >= 2);
+        relax(g, true, m.n_down, g >= 2);
         // the residual product with the JOR sweep's 16-byte lanes and launch shape
         // (one point a lane with seven 8-byte loads is bound by address issue)
         launch_lap(s, L.g, L.c, L.pr, (const T *)x[g], B_::C(L), act, B_::shape(L));
-        const bool walls = !(L.g.per[0] && L.g.per[1] && L.g.per[2]);
-        if (walls) {
-            hipLaunchKernelGGL(k_mg_edges<T>, dim3(1), dim3(MG_EDGE_THREADS), 0, s, L.g, b[g], B_::C(L), 0, act);
-            // the FP32 cycle works on a copy of v; v's edges change as the reference's do
-            if (!fp64 && g == 1)
-                hipLaunchKernelGGL(k_mg_edges<double>, dim3(1), dim3(MG_EDGE_THREADS), 0, s, L.g, v, (double *)nullptr,
-                                   0, act);
-        }
         LevelW<T> R;
         int nmax[3];
         for (int d = 0; d < 3; ++d) {
@@ -537,24 +770,19 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
         // levels run their own); nmax spans that level's pressure range
         const bool coarse_launched = g + 1 < g0;
         hipLaunchKernelGGL(k_mg_restrict<T>, grid_for(cr), dim3(BX, BY, 1), 0, s, L.g, Lc.g, R, Lc.c, cr, b[g],
-                           B_::C(L), B_::A(Lc), coarse_launched ? x[g + 1] : (T *)nullptr, omega, act);
+                           B_::C(L), !fp64 && g == 1 ? v : (double *)nullptr, B_::A(Lc), coarse_launched ? x[g + 1] : (T *)nullptr, omega, act);
     }
     if (g0 <= G) {
-        hipLaunchKernelGGL(k_mg_fused<T>, dim3(1), dim3(MG_FUSED_THREADS), 0, s, B_::dev(m), g0, G, m.n_down, m.n_up,
-                           m.n_bottom, omega, act);
-        // the fused levels' swaps, for the buffer that holds level g0's iterate
-        for (int g = g0; g <= G - 1; ++g) relax(g, true, m.n_down, false);
-        relax(G, true, m.n_bottom, false);
-        relax(G, false, m.n_bottom, false);
-        for (int g = G - 1; g >= g0; --g) relax(g, false, m.n_up, false);
+        MgFusedArgs a;
+        fused_layout(m, g0, a);
+        hipLaunchKernelGGL(k_mg_fused<T>, dim3(1), dim3(MG_FUSED_THREADS), 0, s, a, B_::tables(m.L[g0]), b[g0], x[g0],
+                           omega, act);
     } else {
-        relax(G, true, m.n_bottom, true, true);
-        relax(G, false, m.n_bottom, true);
+        relax(G, true, m.n_bottom, true);
+        relax(G, false, m.n_bottom);
     }
     for (int g = gl; g >= 1; --g) {
         const MgLevel &L = m.L[g], &Lc = m.L[g + 1];
-        if (!(Lc.g.per[0] && Lc.g.per[1] && Lc.g.per[2]))
-            hipLaunchKernelGGL(k_mg_edges<T>, dim3(1), dim3(MG_EDGE_THREADS), 0, s, Lc.g, x[g + 1], (T *)nullptr, 1, act);
         LevelW<T> W;
         for (int d = 0; d < 3; ++d) {
             W.w[d] = B_::cI(L)[d];
@@ -563,11 +791,18 @@ void mg_cycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *ac
         const Range3 cr = full_range(Lc.g);
         hipLaunchKernelGGL(k_mg_interp_cells<T>, grid_for(cr), dim3(BX, BY, 1), 0, s, L.g, Lc.g, W, x[g + 1], x[g],
                            act);
-        relax(g, false, m.n_up, true, false, !fp64 && g == 1);
+        relax(g, false, m.n_up, false, !fp64 && g == 1);
     }
 }
 
 }  // namespace
+
+int mg_first_fused(const MgDev &m) {
+    MgFusedArgs a;
+    for (int g = 2; g <= m.G; ++g)
+        if (fused_layout(m, g, a)) return g;
+    return MG_LEVELS_MAX + 1;
+}
 
 void launch_mg_vcycle(hipStream_t s, const MgDev &m, double *v, double *z, const int *act) {
     mg_cycle<double>(s, m, v, z, act);

@@ -2448,6 +2448,10 @@ struct ih_batch {
     int *pfirst_tile = nullptr, pfirst_ntiles = 0;
     ih::JorBatchItem *pmid[2] = {}, *plast[2] = {};
     int *pjor_tile = nullptr, pjor_ntiles = 0;
+    // the sweep pairs, where every case takes them (threads 0: single sweeps): pairs
+    // between the buffers by parity, and the last one, which writes Z1 or Z2
+    ih::JorBatchItem *ppair[2] = {}, *ppair_last[2] = {};
+    int *ppair_tile = nullptr, ppair_ntiles = 0, ppair_tpb = 0;
     int k_sweeps = -1;
     std::vector<const void *> k_sig;  // the pointers the tables were built from
     int *dflags = nullptr, *hflags = nullptr;
@@ -2468,7 +2472,9 @@ void batch_drop_step(ih_batch *b) {
     b->kg_iters = -1;
     for (void *q : {(void *)b->kcases, (void *)b->ktile, (void *)b->pfirst[0], (void *)b->pfirst[1],
                     (void *)b->pfirst_tile, (void *)b->pmid[0], (void *)b->pmid[1], (void *)b->plast[0],
-                    (void *)b->plast[1], (void *)b->pjor_tile, (void *)b->dflags, (void *)b->dscal})
+                    (void *)b->plast[1], (void *)b->pjor_tile, (void *)b->ppair[0], (void *)b->ppair[1],
+                    (void *)b->ppair_last[0], (void *)b->ppair_last[1], (void *)b->ppair_tile, (void *)b->dflags,
+                    (void *)b->dscal})
         if (q) (void)hipFree(q);
     if (b->hflags) (void)hipHostFree(b->hflags);
     if (b->hscal) (void)hipHostFree(b->hscal);
@@ -2476,6 +2482,9 @@ void batch_drop_step(ih_batch *b) {
     b->ktile = b->pfirst_tile = b->pjor_tile = nullptr;
     b->pfirst[0] = b->pfirst[1] = nullptr;
     b->pmid[0] = b->pmid[1] = b->plast[0] = b->plast[1] = nullptr;
+    b->ppair[0] = b->ppair[1] = b->ppair_last[0] = b->ppair_last[1] = nullptr;
+    b->ppair_tile = nullptr;
+    b->ppair_tpb = 0;
     b->dflags = b->hflags = nullptr;
     b->dscal = b->hscal = nullptr;
     b->k_sig.clear();
@@ -2813,7 +2822,8 @@ std::vector<const void *> step_signature(const ih_batch *b, int sweeps) {
         for (const void *q : {(const void *)c->part, (const void *)c->part2, (const void *)c->part3,
                               (const void *)c->part4, (const void *)c->ksc, (const void *)c->kfl,
                               (const void *)c->f32[0], (const void *)c->f32[1], (const void *)c->f32[2],
-                              (const void *)c->dcoef, (const void *)c->dcoef32})
+                              (const void *)c->dcoef, (const void *)c->dcoef32,
+                              (const void *)(intptr_t)c->c.dg_walls0})
             sig.push_back(q);
     }
     return sig;
@@ -2843,8 +2853,9 @@ int batch_step_tables(ih_batch *b, int sweeps) {
     std::vector<int> ktile;
     std::vector<JorFirstItem> first[2];
     std::vector<int> ftile;
-    std::vector<JorBatchItem> mid[2], last[2];
-    std::vector<int> jtile;
+    std::vector<JorBatchItem> mid[2], last[2], pair, pair_mid[2], pair_last[2];
+    std::vector<int> jtile, ptile;
+    bool pairs = sweeps > 2;  // two sweeps or more after the first
     b->k_pz = b->k_nonpz = b->k_px = false;
     for (int q = 0; q < n; ++q) {
         ih_case *c = b->cases[(size_t)q];
@@ -2916,6 +2927,9 @@ int batch_step_tables(ih_batch *b, int sweeps) {
                 m.bb = c->f32[1];
                 mid[par].push_back(m);
             }
+            it.zero = c->c.zero;
+            pairs = pairs && jor_pair_ok(g, c->c, pb, true);
+            pair.push_back(it);
             // the last sweep reads e0 after an even number of middle sweeps
             float *xl = ((sweeps - 2) % 2 == 0) ? e0 : e1;
             for (int w = 0; w < 2; ++w) {
@@ -2924,6 +2938,30 @@ int batch_step_tables(ih_batch *b, int sweeps) {
                 m.out = w ? (void *)F(c, IH_Z2) : (void *)F(c, IH_Z1);
                 m.bb = c->f32[1];
                 last[w].push_back(m);
+            }
+        }
+    }
+    if (pairs) {
+        const PairShape shape = jor_pair_batch_shape(pair);
+        b->ppair_tpb = shape.tpb;
+        // launches before the last pair: the single sweep of an odd count and the other pairs
+        const int before = (sweeps - 1) % 2 + (sweeps - 1) / 2 - 1;
+        for (int q = 0; q < n; ++q) {
+            ih_case *c = b->cases[(size_t)q];
+            JorBatchItem it = pair[(size_t)q];
+            const int nt = jor_pair_batch_tiles(shape, it);
+            it.tile0 = (int)ptile.size();
+            it.bb = c->f32[1];
+            for (int t = 0; t < nt; ++t) ptile.push_back(q);
+            float *e0 = c->f32[0], *e1 = c->f32[2];
+            for (int w = 0; w < 2; ++w) {
+                JorBatchItem m = it;
+                m.rel = w ? e1 : e0;
+                m.out = w ? e0 : e1;
+                pair_mid[w].push_back(m);
+                m.rel = before % 2 ? e1 : e0;
+                m.out = w ? (void *)F(c, IH_Z2) : (void *)F(c, IH_Z1);
+                pair_last[w].push_back(m);
             }
         }
     }
@@ -2945,6 +2983,10 @@ int batch_step_tables(ih_batch *b, int sweeps) {
                 ok = ok && owns(ftile, q, f.tile0, (int64_t)f.ntile * f.nbz) &&
                      owns(jtile, q, m.tile0, (int64_t)m.ntxy * m.nbz) && owns(jtile, q, l.tile0, (int64_t)l.ntxy * l.nbz);
             }
+        if (pairs) {
+            const JorBatchItem &m = pair_mid[0][(size_t)q];
+            ok = ok && owns(ptile, q, m.tile0, (int64_t)m.ntxy * m.nbz);
+        }
         if (!ok) return fail(IH_EINVAL, "batched step: tile table of case %d is inconsistent", q);
     }
     b->kntiles = (int)ktile.size();
@@ -2958,6 +3000,11 @@ int batch_step_tables(ih_batch *b, int sweeps) {
                 return rc;
         }
         if ((rc = upload_table(&b->pfirst_tile, ftile)) || (rc = upload_table(&b->pjor_tile, jtile))) return rc;
+        b->ppair_ntiles = (int)ptile.size();
+        for (int w = 0; pairs && w < 2; ++w)
+            if ((rc = upload_table(&b->ppair[w], pair_mid[w])) || (rc = upload_table(&b->ppair_last[w], pair_last[w])))
+                return rc;
+        if (pairs && (rc = upload_table(&b->ppair_tile, ptile))) return rc;
     }
     HIPCHK(hipMalloc(&b->dflags, sizeof(int) * KF_NSLOTS * (size_t)n));
     HIPCHK(hipMalloc(&b->dscal, sizeof(double) * KS_NSLOTS * (size_t)n));
@@ -2976,6 +3023,17 @@ void batch_precond(ih_batch *b, int w, int sweeps, float omega, bool first_done)
     if (!first_done)
         launch_jor_f32_first_batch(s, b->pfirst[w], b->pfirst_tile, b->pfirst_ntiles, omega, sweeps == 1);
     if (sweeps < 2) return;
+    if (b->ppair_tpb) {
+        int par = 0;  // the iterate is in e0, or in e1
+        if ((sweeps - 1) % 2) {  // an odd count's single sweep comes first
+            launch_jor_batch_f32(s, b->pmid[0], b->pjor_tile, b->pjor_ntiles, omega, false, b->k_px);
+            par = 1;
+        }
+        for (int left = (sweeps - 1) / 2; left > 1; --left, par ^= 1)
+            launch_jor_pair_batch(s, b->ppair[par], b->ppair_tile, b->ppair_ntiles, b->ppair_tpb, omega, false, b->k_px);
+        launch_jor_pair_batch(s, b->ppair_last[w], b->ppair_tile, b->ppair_ntiles, b->ppair_tpb, omega, true, b->k_px);
+        return;
+    }
     for (int q = 1; q < sweeps - 1; ++q)
         launch_jor_batch_f32(s, b->pmid[(q - 1) & 1], b->pjor_tile, b->pjor_ntiles, omega, false, b->k_px);
     launch_jor_batch_f32(s, b->plast[w], b->pjor_tile, b->pjor_ntiles, omega, true, b->k_px);

@@ -112,8 +112,8 @@ void launch_jor(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double
 void launch_jor_f32(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
                     const float *bb, float *out, const int *active = nullptr, JorLaunch shape = JorLaunch());
 // Two JOR sweeps in one launch, out = sweep(sweep(rel)), the bits of two single
-// ones.  jor_pair_ok: whether box b takes it (the whole pressure range, x not
-// periodic, no coupling past a wall, rows short enough for a block).
+// ones.  jor_pair_ok: whether box b takes it (the whole pressure range, no coupling
+// past a wall, rows short enough for a block).
 bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32);
 void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double omega, const double *rel,
                      const double *bb, double *out, const int *active);
@@ -169,6 +169,16 @@ struct JorBatchItem {
     void *out;
     int ntxy, nbz, tile0, pad;
     const int *active;  // the case's BiCGstab active flag (nullptr: always sweep)
+    const void *zero;   // zeros that the sweep pairs read for dead entries
+};
+// A box as the sweep pairs cut it: its vectors, its planes, stretches a plane.
+struct PairBox {
+    JorVecShape sh;
+    int planes;
+    int tiles(int tpb) const {
+        const int span = tpb - 2 * (sh.nent + 1);
+        return (sh.nent_all + span - 1) / span;
+    }
 };
 // One case of the batched first FP32 preconditioner sweep (k_jor_f32_first):
 // 4-point vectors from i0, nv a row, ntile tiles a chunk, nbz chunks.
@@ -204,6 +214,15 @@ void launch_jor_f32_first(hipStream_t s, const Geo &g, const Coef &c, const Box 
 // batched FP32 preconditioner sweeps (flat tile -> item table over ntiles tiles)
 void launch_jor_batch_f32(hipStream_t s, const JorBatchItem *items, const int *tile_item, int ntiles, float omega,
                           bool to64, bool any_periodic_x);
+// batched FP32 sweep pairs, each case's box taken by jor_pair_ok: the launch shape of a
+// batch, a case's tiles in it (sets sh, ntxy, nbz), the launch
+struct PairShape {
+    int tpb = 0, kc = 0;  // threads a block, planes a z chunk
+};
+PairShape jor_pair_batch_shape(const std::vector<JorBatchItem> &items);
+int jor_pair_batch_tiles(PairShape shape, JorBatchItem &it);
+void launch_jor_pair_batch(hipStream_t s, const JorBatchItem *items, const int *tile_item, int ntiles, int tpb,
+                           float omega, bool to64, bool any_periodic_x);
 int jor_first_tiles(const Box &b, const Geo &g, JorFirstItem &it);  // sets r, i0, nv, ntile, nbz; returns tiles
 void launch_jor_f32_first_batch(hipStream_t s, const JorFirstItem *items, const int *tile_item, int ntiles,
                                 float omega, bool to64);

@@ -936,7 +936,9 @@ __global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, Coef c, Range3 r, JorVec
 //     within a row of the stretch's ends load their outer y neighbour instead;
 //   - the first iterate of plane k goes through LDS the same way, a plane later, for
 //     the second sweep of plane k-1 (one barrier a plane, both double buffered);
-//   - z neighbours of both sweeps are register queues.
+//   - z neighbours of both sweeps are register queues;
+//   - across a periodic x the first sweep's neighbour is a load (the other end of the
+//     row may be in the next stretch), the second's is in LDS (a stored row is whole).
 // The first iterate is right on all TPB entries, the second on those a row and an
 // entry or more from the ends, so consecutive stretches overlap by 2 (nent + 1)
 // entries, and z chunks by one plane at either end.
@@ -951,23 +953,20 @@ __global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, Coef c, Range3 r, JorVec
 //   FP32        7.8 ->  5.4 8.4 -> 6.5 12.6 -> 10.7 14.4 -> 13.9 24.0 -> 22.4 55.2 -> 51.2
 // A reciprocal shared by the two sweeps with the quotient corrected to the IEEE
 // one costs, with the range checks, as many instructions as it saves.
-template <typename T, typename TO, int TPB, bool PZ>
-__global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVecShape sh, int nt, int nbz, T omega,
-                                                  const T *__restrict__ rel, const T *__restrict__ bb,
-                                                  TO *__restrict__ out, const int *active) {
-    if (active && !*active) return;
-    int tw, dummy, bz;
-    if (!xcd_tile(nt, 1, nbz, tw, dummy, bz)) return;
+// Block function of stretch tw, z chunk bz (the single-case and the batched kernel;
+// PX: x may be periodic; PZM: 0 z is not periodic, 1 it is, 2 decided at run time).
+template <typename T, typename TO, int TPB, bool PX, int PZM, typename PC, typename PO>
+__device__ inline void jor_pair_block(const Geo g, const Range3 r, const JorVecShape sh, int tw, int bz, int nbz,
+                                      T omega, PC rel, PC bb, PO out, PC g1, PC g2, const T *g3c, PC zeros) {
     constexpr int V = 16 / sizeof(T);
     typedef typename VecOf<T>::type VT;
     typedef TO VO __attribute__((ext_vector_type(V)));
     __shared__ VT s0[2][TPB], s1[2][TPB];
-    const T *const g1 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[0] : (const void *)c.dgf[0]);
-    const T *const g2 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[1] : (const void *)c.dgf[1]);
+    const bool PZ = PZM == 2 ? g.per[2] != 0 : PZM == 1;
     // scalar loads: a vector load of a uniform value would be waited for together with
     // the plane's prefetches
     typedef const __attribute__((address_space(4))) T *CP;
-    const CP g3 = (CP)(sizeof(T) == 8 ? (const void *)c.dg[2] : (const void *)c.dgf[2]);
+    const CP g3 = (CP)g3c;
     const int tid = threadIdx.x, lane = tid & 63;
     const int nent = sh.nent, H = nent + 1;
     const int q = tw * (TPB - 2 * H) - H + tid;
@@ -1001,14 +1000,14 @@ __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVe
     const int lo2 = r.lo2, hi2 = r.lo2 + r.n2 - 1;
     // plane index in memory: wrapped, or held to the range and m ghost planes
     auto plane = [&](int k, int m) {
-        if constexpr (PZ) return k < lo2 ? k + r.n2 : (k > hi2 ? k - r.n2 : k);
+        if (PZ) return k < lo2 ? k + r.n2 : (k > hi2 ? k - r.n2 : k);
         k = k < lo2 - m ? lo2 - m : k;
         return k > hi2 + m ? hi2 + m : k;
     };
     const int64_t xy = gidx(g, is, j, 0) - 3 * g.pxy;
     // dead entries read zeros, whatever the plane
-    const T *const xp = live ? rel + xy + 3 * g.pxy : (const T *)c.zero;
-    const T *const bp = live ? bb + xy + 3 * g.pxy : (const T *)c.zero;
+    const PC xp = live ? rel + xy + 3 * g.pxy : zeros;
+    const PC bp = live ? bb + xy + 3 * g.pxy : zeros;
     // outer y neighbour of the stretch's first and last row
     const bool lowe = tid < nent, highe = tid >= TPB - nent;
     int64_t dye = lowe ? -(int64_t)g.px : (int64_t)g.px;
@@ -1016,10 +1015,18 @@ __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVe
         if (lowe && j == g.Sp[1]) dye = (int64_t)(g.Np[1] - g.Sp[1]) * g.px;
         if (highe && j == g.Np[1]) dye = -(int64_t)(g.Np[1] - g.Sp[1]) * g.px;
     }
-    const T *const ep = live ? xp + dye : xp;
+    const PC ep = live ? xp + dye : xp;
+    // periodic x: the vectors with the row's first and last point, whose outer neighbour
+    // is the last and the first point (component wt of the vector wdist entries away)
+    const int is1 = sh.i0 + V * (sh.nv - 1);
+    const bool px = PX && g.per[0];
+    const bool wlow = px && e == 1, whigh = px && e == sh.nv;
+    const int tlo = r.lo0 - sh.i0, thi = hi0 - is1;  // of the first point, of the last
+    const int wofs = wlow ? V * (sh.nv - 1) + thi : tlo - V * (sh.nv - 1);  // values, from the vector's first
+    const PC wp = live && (wlow || whigh) ? xp + wofs : xp;
     const bool edge_wave = __builtin_amdgcn_readfirstlane(tid & ~63) < nent ||
                            __builtin_amdgcn_readfirstlane(tid | 63) >= TPB - nent;
-    auto ld = [&](const T *p, int k, int m) {
+    auto ld = [&](PC p, int k, int m) {
         const int64_t o = (int64_t)plane(k, m) * g.pxy;
         return vload<VT>(p + (live ? o : 0));
     };
@@ -1033,12 +1040,17 @@ __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVe
     };
     // one sweep of this thread's vector x on the right-hand side b
     auto relax = [&](const VT &b, const VT &x, const VT &ym, const VT &yp, const VT &zlo, const VT &zhi, T xl, T xr,
-                     const Zc &z, VT &res) {
+                     T xw, const Zc &z, VT &res) {
 #pragma unroll
         for (int t = 0; t < V; ++t) {
             T s = b[t];
-            s = s - a1m[t] * (t == 0 ? xl : x[t > 0 ? t - 1 : 0]);
-            s = s - a1p[t] * (t == V - 1 ? xr : x[t < V - 1 ? t + 1 : V - 1]);
+            T l = t == 0 ? xl : x[t > 0 ? t - 1 : 0], h = t == V - 1 ? xr : x[t < V - 1 ? t + 1 : V - 1];
+            if (PX) {
+                l = wlow && t == tlo ? xw : l;
+                h = whigh && t == thi ? xw : h;
+            }
+            s = s - a1m[t] * l;
+            s = s - a1p[t] * h;
             s = s - a2m * ym[t];
             s = s - a2p * yp[t];
             s = s - z.m * zlo[t];
@@ -1074,14 +1086,17 @@ __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVe
     // plane ahead, into two sets by turns
     struct Plane {
         VT zp, b, ye;
+        T xw;
     };
     auto fetch = [&](int k, Plane &P) {
         P.zp = ld(xp, k + 1, 1);
         P.b = ld(bp, k, 0);
         if (edge_wave) P.ye = ld(ep, k, 1);
+        if (PX) P.xw = wp[live ? (int64_t)plane(k, 1) * g.pxy : 0];
     };
     Plane A, B;
     A.ye = B.ye = zero;
+    A.xw = B.xw = T(0);
     fetch(kc0 - 1, A);
     s0[0][tid] = zc;
     auto step = [&](int k, int buf, Plane &P, Plane &next) {
@@ -1093,19 +1108,21 @@ __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVe
         T xl, xr, vl, vr;
         x_neighbours(s0[buf], zc, xl, xr);
         x_neighbours(s1[buf ^ 1], uc, vl, vr);
+        T vw = T(0);
+        if (PX && (wlow || whigh) && store) vw = ((const T *)s1[buf ^ 1])[V * tid + wofs];
         if (lowe) ym = P.ye;
         if (highe) yp = P.ye;
         VT u;
-        relax(P.b, zc, ym, yp, zm, P.zp, xl, xr, gc, u);
+        relax(P.b, zc, ym, yp, zm, P.zp, xl, xr, P.xw, gc, u);
         const bool in_z = PZ || (k >= lo2 && k <= hi2);
 #pragma unroll
         for (int t = 0; t < V; ++t) u[t] = real[t] && in_z ? u[t] : T(0);
         s1[buf][tid] = u;
         s0[buf ^ 1][tid] = P.zp;
         VT w;  // the second sweep of plane k-1 (from k = kc0 + 1 on)
-        relax(bm, uc, vm, vp, um, u, vl, vr, gm, w);
+        relax(bm, uc, vm, vp, um, u, vl, vr, vw, gm, w);
         if (store && k > kc0) {
-            TO *const o = out + xy + (int64_t)(k - 1 + 3) * g.pxy;
+            const PO o = out + xy + (int64_t)(k - 1 + 3) * g.pxy;
             if (full) {
                 VO v;
 #pragma unroll
@@ -1133,6 +1150,35 @@ __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVe
         step(k, 1, B, A);
         if (++k > kc1 + 1) break;
     }
+}
+
+template <typename T, typename TO, int TPB, bool PX, bool PZ>
+__global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVecShape sh, int nt, int nbz, T omega,
+                                                  const T *__restrict__ rel, const T *__restrict__ bb,
+                                                  TO *__restrict__ out, const int *active) {
+    if (active && !*active) return;
+    int tw, dummy, bz;
+    if (!xcd_tile(nt, 1, nbz, tw, dummy, bz)) return;
+    const T *const g1 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[0] : (const void *)c.dgf[0]);
+    const T *const g2 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[1] : (const void *)c.dgf[1]);
+    const T *const g3 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[2] : (const void *)c.dgf[2]);
+    jor_pair_block<T, TO, TPB, PX, PZ ? 1 : 0, const T *, TO *>(g, r, sh, tw, bz, nbz, omega, rel, bb, out, g1, g2, g3,
+                                                               (const T *)c.zero);
+}
+
+// the FP32 sweep pairs of many cases in one launch (tile -> item table)
+template <typename TO, int TPB, bool PX>
+__global__ __launch_bounds__(TPB) void k_jor_pair_batch(const JorBatchItem *__restrict__ items,
+                                                        const int *__restrict__ tile_item, int ntiles, float omega) {
+    int t, dummy, dummy2;
+    if (!xcd_tile(ntiles, 1, 1, t, dummy, dummy2)) return;
+    const JorBatchItem &it = items[tile_item[t]];
+    if (it.active && !*it.active) return;
+    const int local = t - it.tile0;
+    const int tw = local % it.ntxy, bz = local / it.ntxy;
+    jor_pair_block<float, TO, TPB, PX, 2, gconst<float>, gmut<TO>>(
+        it.g, it.r, it.sh, tw, bz, it.nbz, omega, (gconst<float>)it.rel, (gconst<float>)it.bb, (gmut<TO>)it.out,
+        (gconst<float>)it.dgf[0], (gconst<float>)it.dgf[1], it.dgf[2], (gconst<float>)it.zero);
 }
 
 // First FP32 sweep from e = 0 on A e = (float)v: b32 = (float)v is stored for
@@ -1785,48 +1831,65 @@ void launch_jor_f32_to64(hipStream_t s, const Geo &g, const Coef &c, const Box &
     launch_jor_vec<float, double>(s, g, c, b, omega, rel, bb, out, active, shape);
 }
 
-// Launch of a sweep pair: threads a block and z chunk by the estimated time of the
-// most loaded compute unit.  A block's plane costs its two sweeps' instructions
-// (about 1000 clocks a wavefront of 4 FP32 points or 2 FP64 ones, shared by the
-// wavefronts of a SIMD) or, where few wavefronts are resident, the latency of the
-// chain barrier to barrier; starting a block costs about five planes of latency.
-template <typename T, typename TO>
-static bool launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, T omega, const T *rel, const T *bb,
-                        TO *out, const int *active) {
-    const Range3 r = R(b);
-    int best_t = 0, best_nbz = 0, best_nt = 0;
-    double best = 0.0;
-    JorVecShape sh;
+// Shape of a launch of sweep pairs over n boxes: threads a block and planes a z chunk
+// by the estimated time of the most loaded compute unit.  A block's plane costs its
+// two sweeps' instructions (about 1000 clocks a wavefront of 4 FP32 points or 2 FP64
+// ones, shared by the wavefronts of a SIMD) or, where few wavefronts are resident,
+// the latency of the chain barrier to barrier; starting a block costs about five
+// planes of latency.  Within 6 % of the best of all shapes on 33x17x17 to
+// 385x193x193 (10 % of FP32 at 97^3).
+template <typename F>
+static PairShape pair_shape(int n, int max_planes, F box) {
+    PairShape best;
+    double best_time = 0.0;
     for (int tpb : {256, 512, 1024}) {
-        int nbw, nbz0;
-        sh = jor_vec_shape(g, r, 16 / (int)sizeof(T), 256, 0, nbw, nbz0);
-        const int span = tpb - 2 * (sh.nent + 1);
-        if (4 * (sh.nent + 1) > tpb) continue;
-        const int nt = (sh.nent_all + span - 1) / span;
-        for (int nbz = 1, kc; nbz <= r.n2; nbz = kc > 1 ? (r.n2 + kc - 2) / (kc - 1) : r.n2 + 1) {
-            kc = (r.n2 + nbz - 1) / nbz;  // the fewest chunks of each length
-            const double blocks = std::ceil((double)nt * nbz / 256.0);  // on the most loaded compute unit
-            const double resident = std::min(blocks, 1024.0 / tpb);
+        bool fits = true;
+        for (int q = 0; q < n; ++q) fits = fits && 4 * (box(q).sh.nent + 1) <= tpb;
+        if (!fits) continue;
+        for (int nbz = 1, kc; nbz <= max_planes; nbz = kc > 1 ? (max_planes + kc - 2) / (kc - 1) : max_planes + 1) {
+            kc = (max_planes + nbz - 1) / nbz;  // the fewest chunks of each length
+            int64_t blocks = 0;
+            for (int q = 0; q < n; ++q) blocks += (int64_t)box(q).tiles(tpb) * ((box(q).planes + kc - 1) / kc);
+            const double load = std::ceil((double)blocks / 256.0);  // on the most loaded compute unit
+            const double resident = std::min(load, 1024.0 / tpb);
             const double plane = std::max(1200.0, resident * tpb / 256.0 * 1000.0);
-            const double t = blocks / resident * (6000.0 + (kc + 2) * plane);
-            if (!best_t || t < best) {
-                best = t;
-                best_t = tpb;
-                best_nbz = nbz;
-                best_nt = nt;
+            const double t = load / resident * (6000.0 + (kc + 2) * plane);
+            if (best.tpb == 0 || t < best_time) {
+                best_time = t;
+                best = PairShape{tpb, kc};
             }
         }
     }
-    if (!best_t) return false;
+    return best;
+}
+
+static PairBox pair_box(const Geo &g, const Range3 &r, int V) {
+    int nbw, nbz;
+    return PairBox{jor_vec_shape(g, r, V, 256, 0, nbw, nbz), r.n2};
+}
+
+template <typename T, typename TO>
+static void launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, T omega, const T *rel, const T *bb,
+                        TO *out, const int *active) {
+    const Range3 r = R(b);
+    const PairBox pb = pair_box(g, r, 16 / (int)sizeof(T));
+    const PairShape shape = pair_shape(1, r.n2, [&](int) { return pb; });
+    const JorVecShape &sh = pb.sh;
+    const int best_t = shape.tpb, best_nt = pb.tiles(best_t), best_nbz = (r.n2 + shape.kc - 1) / shape.kc;
     const dim3 grid(xcd_grid((int64_t)best_nt * best_nbz));
+#define IH_JPL(TPBV, PX, PZ)                                                                                      \
+    hipLaunchKernelGGL((k_jor_pair<T, TO, TPBV, PX, PZ>), grid, dim3(TPBV), 0, s, g, c, r, sh, best_nt, best_nbz, \
+                       omega, rel, bb, out, active)
 #define IH_JP(TPBV)                                                                                               \
     do {                                                                                                          \
-        if (g.per[2])                                                                                             \
-            hipLaunchKernelGGL((k_jor_pair<T, TO, TPBV, true>), grid, dim3(TPBV), 0, s, g, c, r, sh, best_nt,        \
-                               best_nbz, omega, rel, bb, out, active);                                            \
+        if (g.per[0] && g.per[2])                                                                                 \
+            IH_JPL(TPBV, true, true);                                                                             \
+        else if (g.per[0])                                                                                        \
+            IH_JPL(TPBV, true, false);                                                                            \
+        else if (g.per[2])                                                                                        \
+            IH_JPL(TPBV, false, true);                                                                            \
         else                                                                                                      \
-            hipLaunchKernelGGL((k_jor_pair<T, TO, TPBV, false>), grid, dim3(TPBV), 0, s, g, c, r, sh, best_nt,       \
-                               best_nbz, omega, rel, bb, out, active);                                            \
+            IH_JPL(TPBV, false, false);                                                                           \
     } while (0)
     if (best_t == 256)
         IH_JP(256);
@@ -1835,7 +1898,7 @@ static bool launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b
     else
         IH_JP(1024);
 #undef IH_JP
-    return true;
+#undef IH_JPL
 }
 
 // The pair is the faster form at every size it fits (figures above k_jor_pair), so
@@ -1844,7 +1907,7 @@ static bool launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b
 // of entries to wrap a periodic y by, nothing that the second sweep would read
 // from a ghost point that is not there.
 bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32) {
-    if (!c.dg_walls0 || g.per[0]) return false;
+    if (!c.dg_walls0) return false;
     for (int d = 0; d < 3; ++d)
         if (b.lo[d] != g.Sp[d] || b.hi[d] != g.Np[d]) return false;
     int nbw, nbz;
@@ -1977,6 +2040,43 @@ void launch_jor_batch_f32(hipStream_t s, const JorBatchItem *items, const int *t
             hipLaunchKernelGGL((k_jor_batch<float, TPB, 0>), flat, dim3(TPB), 0, s, items, tile_item, 0, ntiles,
                                omega);
     }
+}
+
+PairShape jor_pair_batch_shape(const std::vector<JorBatchItem> &items) {
+    int planes = 0;
+    for (const JorBatchItem &it : items) planes = std::max(planes, it.r.n2);
+    std::vector<PairBox> boxes;
+    for (const JorBatchItem &it : items) boxes.push_back(pair_box(it.g, it.r, 4));
+    return pair_shape((int)items.size(), planes, [&](int q) -> const PairBox & { return boxes[(size_t)q]; });
+}
+
+int jor_pair_batch_tiles(PairShape shape, JorBatchItem &it) {
+    const PairBox pb = pair_box(it.g, it.r, 4);
+    it.sh = pb.sh;
+    it.ntxy = pb.tiles(shape.tpb);
+    it.nbz = (it.r.n2 + shape.kc - 1) / shape.kc;
+    return it.ntxy * it.nbz;
+}
+
+void launch_jor_pair_batch(hipStream_t s, const JorBatchItem *items, const int *tile_item, int ntiles, int tpb,
+                           float omega, bool to64, bool any_periodic_x) {
+    if (ntiles <= 0) return;
+    const dim3 grid(xcd_grid(ntiles));
+#define IH_JPB(TO, TPBV)                                                                                          \
+    do {                                                                                                          \
+        if (any_periodic_x)                                                                                       \
+            hipLaunchKernelGGL((k_jor_pair_batch<TO, TPBV, true>), grid, dim3(TPBV), 0, s, items, tile_item, ntiles, \
+                               omega);                                                                            \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_jor_pair_batch<TO, TPBV, false>), grid, dim3(TPBV), 0, s, items, tile_item, ntiles, \
+                               omega);                                                                            \
+    } while (0)
+    if (to64) {
+        if (tpb == 256) IH_JPB(double, 256); else if (tpb == 512) IH_JPB(double, 512); else IH_JPB(double, 1024);
+    } else {
+        if (tpb == 256) IH_JPB(float, 256); else if (tpb == 512) IH_JPB(float, 512); else IH_JPB(float, 1024);
+    }
+#undef IH_JPB
 }
 
 int jor_first_tiles(const Box &b, const Geo &g, JorFirstItem &it) {

@@ -1,7 +1,7 @@
 """Two JOR sweeps in one launch: rows whose vector count is at the limits of a
 block (64, 128 and 256 entries a row with the halo, in FP64 at 122, 250 and 506
 points, in FP32 at 244, 500 and 1012), stretches of a plane that end inside a
-row, periodic y and z down to the fewest points, and the ranges that keep the
+row, periodic directions down to the fewest points, and the ranges that keep the
 single sweeps.  Tolerance: none, the pair forms each value with the operands and
 in the order of two single sweeps, which are the oracle's (bit for bit)."""
 import ctypes
@@ -17,12 +17,16 @@ pytestmark = pytest.mark.gpu
 
 W6 = (1, 1, 1, 1, 1, 1)
 PY, PZ, PYZ, PX = (1, 1, -1, -1, 1, 1), (1, 1, 1, 1, -1, -1), (1, 1, -1, -1, -1, -1), (-1, -1, 1, 1, -1, -1)
+PXY, PXYZ = (-1, -1, -1, -1, 1, 1), (-1,) * 6
 # (sizes, boundaries): x lengths on both sides of each limit
 PAIRS = [((nx, 9 + nx % 4, 10), bc) for nx, bc in
          [(8, W6), (9, PYZ), (10, PY), (121, W6), (122, PY), (123, PZ), (124, W6), (243, PY), (244, W6), (245, PYZ),
           (249, W6), (250, PYZ), (251, W6), (499, W6), (501, PY), (505, W6), (507, PYZ), (509, W6), (1011, PY),
           (1013, W6), (1018, W6)]]
 PAIRS += [((33, 8, 8), PYZ), ((41, 70, 9), PY), ((65, 33, 67), W6), ((34, 37, 131), PZ), ((66, 30, 20), PX)]
+PAIRS += [((nx, 9 + nx % 3, 11), bc) for nx, bc in
+          [(8, PX), (9, PXYZ), (10, PXY), (11, PX), (65, PXYZ), (122, PXY), (123, PX), (246, PX), (247, PXYZ), (502, PX),
+           (506, PX), (507, PXY), (1014, PX), (1020, PX)]]
 
 
 def same(a, b, what):
@@ -83,3 +87,30 @@ def test_coupling_past_a_wall_keeps_single_sweeps():
         out.append(gc.download(ih.PRE))
     same(out[0], out[1], "coupled walls")
     gc.close()
+
+
+@pytest.mark.parametrize("sweeps", [3, 4, 7])
+@pytest.mark.parametrize("bcs", [(W6, PZ, W6, PY), (PX, W6, PXY, PZ), (W6, PX, W6)],
+                         ids=["walls-and-yz", "periodic-x", "a-row-too-long"])
+def test_pairs_in_a_batch(sweeps, bcs):
+    """M's FP32 sweeps of several cases in shared launches: each case as alone.  A
+    batch with a row past the limit (1100 points) keeps the single sweeps."""
+    sizes = [(41, 17, 33), (130, 19, 18), (246, 9, 15), (17, 33, 9)] if len(bcs) == 4 else [(33, 9, 17), (20, 11, 9), (1100, 8, 9)]
+    p = ih.StepParams(Re=100.0, dtime=1e-4, jor_sweeps=4, jor_omega=0.8, bicg_rel_tol=1e-12, bicg_max_it=3,
+                      level_pressure=1, jor_fp32=1, precond_sweeps=sweeps)
+    cases = [[ih.Case(N, bc, (2.0, 1.0, 1.0)) for N, bc in zip(sizes, bcs)] for _ in range(2)]
+    for cs in cases:
+        rng = np.random.default_rng(10)
+        for c in cs:
+            for f in (ih.VEL1, ih.VEL2, ih.VEL3):
+                c.upload(f, 0.01 * rng.standard_normal(c.shape))
+    bt = ih.Batch(cases[0])
+    sb = bt.timestep(p, 0.0)
+    for q, (a, c) in enumerate(zip(*cases)):
+        ss = c.timestep(p, 0.0)
+        assert list(sb[q].bicg_final) == list(ss.bicg_final) and np.all(np.isfinite(list(ss.bicg_final))), q
+        for f in (ih.PRE, ih.VEL1, ih.VEL2, ih.VEL3):
+            same(a.download(f), c.download(f), f"case {q}, field {f}")
+    bt.close()
+    for c in cases[0] + cases[1]:
+        c.close()

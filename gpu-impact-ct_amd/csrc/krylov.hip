@@ -1207,6 +1207,75 @@ __device__ inline void x_update_split_block(const Geo &g, const Range3 &r, int b
     }
 }
 
+// The operator's dot products from memory, for an operator launched in shorter z chunks
+// than the reduction's: <o, Ap>, and <Ap, Ap> with TWO, the planes of a reduction chunk
+// on UPD_ZG groups that take turns in plane order, so the partials are the fused ones'
+// bits.
+template <bool TWO>
+__global__ __launch_bounds__(UPD_ZG * RED_THREADS) void k_dots(Geo g, Range3 r, int nbx, int nby, int nbz,
+                                                               const double *__restrict__ Ap,
+                                                               const double *__restrict__ o, double *part1,
+                                                               double *part2, const int *active) {
+    if (active && !*active) return;
+    int bx, by, bz;
+    if (!xcd_tile(nbx, nby, nbz, bx, by, bz)) return;
+    const int64_t pi = (int64_t)bx + (int64_t)nbx * ((int64_t)by + (int64_t)nby * bz);
+    __shared__ double sm[8], carry[TWO ? 2 : 1][RED_THREADS];
+    const int tid = (int)(threadIdx.x + RED_TX * threadIdx.y);
+    const int zg = __builtin_amdgcn_readfirstlane((int)threadIdx.z);
+    const int i = r.lo0 + bx * RED_TX + (int)threadIdx.x;
+    const int j = r.lo1 + by * RED_TY + (int)threadIdx.y;
+    const bool own = i < r.lo0 + r.n0 && j < r.lo1 + r.n1;
+    int kc0, kc1;
+    red_chunk(r, bz, nbz, kc0, kc1);
+    int k0, cnt;
+    split_planes(zg, kc0, kc1, k0, cnt);
+    const int64_t x0 = gidx(g, own ? i : r.lo0, own ? j : r.lo1, 0);
+    double a[UPD_KP], b[UPD_KP];
+#pragma unroll
+    for (int u = 0; u < UPD_KP; ++u) {
+        a[u] = b[u] = 0.0;
+        if (u < cnt) {
+            const int64_t x = x0 + (int64_t)(k0 + u) * g.pxy;
+            a[u] = Ap[x];
+            b[u] = o[x];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < UPD_KP; ++u) {
+        b[u] = b[u] * a[u];
+        a[u] = a[u] * a[u];
+    }
+#pragma unroll
+    for (int z = 0; z < UPD_ZG; ++z) {
+        if (z > 0) __syncthreads();
+        if (zg == z) {
+            double s1 = z == 0 ? 0.0 : carry[0][tid], s2 = z == 0 || !TWO ? 0.0 : carry[TWO ? 1 : 0][tid];
+#pragma unroll
+            for (int u = 0; u < UPD_KP; ++u) {
+                s1 = own && u < cnt ? s1 + b[u] : s1;
+                if (TWO) s2 = own && u < cnt ? s2 + a[u] : s2;
+            }
+            if (z < UPD_ZG - 1) {
+                carry[0][tid] = s1;
+                if (TWO) carry[1][tid] = s2;
+            } else {
+                s1 = wave_sum(s1);
+                if (TWO) s2 = wave_sum(s2);
+                if ((tid & 63) == 0) {
+                    sm[tid >> 6] = s1;
+                    sm[4 + (tid >> 6)] = s2;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0 && zg == 0) {
+        part1[pi] = (sm[0] + sm[1]) + (sm[2] + sm[3]);
+        if (TWO) part2[pi] = (sm[4] + sm[5]) + (sm[6] + sm[7]);
+    }
+}
+
 // One block of it fills a compute unit (1024 threads of 104 or 120 VGPRs), so it is
 // taken where its blocks fill their rounds over the device: up to one round, or with
 // the last round at most an eighth of all empty.  A BiCGstab iteration with it and
@@ -1452,6 +1521,20 @@ __global__ void k_gather_batch(const KBatchCase *__restrict__ cases, int ncases,
 // ===========================================================================
 static inline Range3 Rk(const Box &b) { return make_range(b); }
 
+// z chunks of an operator that leaves its dot products to k_dots: as many as fill the
+// device with two blocks of teams a compute unit, of three planes or more.  A block
+// marches its chunk and six planes more at 0.6 us a plane, so a grid of few columns is
+// bound by the 32 planes of the reduction's chunk; k_dots costs 3.5 to 5 us.  Operator
+// fused / split without k_dots, a BiCGstab iteration fused / split, microseconds:
+//   33x17x17     14.1 /  6.5   48.1 / 45.0     118x71x91   22.5 / 12.9   83.1 / 70.9
+//   65^3         17.3 /  9.2   61.1 / 54.8     97^3        20.0 / 15.9   (not taken)
+//   129x65x65    17.6 / 11.4   65.5 / 61.2     193x97x97   28.9 / 27.1   (not taken)
+// hence at least APPLY_SPLIT times the reduction's chunks (97^3 has 10 for 4).
+static int apply_split(int columns, int planes) {
+    return (int)std::min<int64_t>((planes + 2) / 3, APPLY_TEAM_TILES / columns);
+}
+constexpr int APPLY_SPLIT = 3;
+
 void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, const double *src, double *dst,
                     const double *w, int dot_mode, double *part1, double *part2, const int *active) {
     Range3 r = Rk(pb);
@@ -1459,6 +1542,23 @@ void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, c
     // the operator tile is the reduction tile, so the fused dot partials follow the fixed tree
     const int nbx = (r.n0 + RED_TX - 1) / RED_TX, nby = (r.n1 + RED_TY - 1) / RED_TY, nbz = (r.n2 + RED_KC - 1) / RED_KC;
     const int64_t tiles = (int64_t)nbx * nby * nbz;
+    const int nsplit = apply_split(nbx * nby, r.n2);
+    if (nsplit >= APPLY_SPLIT * nbz) {
+        const dim3 grid(xcd_grid((int64_t)nbx * nby * nsplit)), block(RED_TX, RED_TY, 2);
+        if (g.per[2])
+            hipLaunchKernelGGL((k_apply<true, DOT_NONE, true>), grid, block, 0, s, g, c, r, nbx, nby, nsplit, src, dst,
+                               nullptr, nullptr, nullptr, active);
+        else
+            hipLaunchKernelGGL((k_apply<true, DOT_NONE, false>), grid, block, 0, s, g, c, r, nbx, nby, nsplit, src, dst,
+                               nullptr, nullptr, nullptr, active);
+        const dim3 dgrid(xcd_grid(tiles)), dblock(RED_TX, RED_TY, UPD_ZG);
+        if (dot_mode == DOT_W)
+            hipLaunchKernelGGL(k_dots<false>, dgrid, dblock, 0, s, g, r, nbx, nby, nbz, dst, w, part1, part2, active);
+        else if (dot_mode != DOT_NONE)
+            hipLaunchKernelGGL(k_dots<true>, dgrid, dblock, 0, s, g, r, nbx, nby, nbz, dst,
+                               dot_mode == DOT_SELF ? src : w, part1, part2, active);
+        return;
+    }
     const bool teams = tiles <= APPLY_TEAM_TILES;
     const dim3 grid(xcd_grid(tiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
 #define IH_APPLY_AS(T, DMV, PZV)                                                                               \

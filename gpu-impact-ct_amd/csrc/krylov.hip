@@ -1250,7 +1250,7 @@ __global__ __launch_bounds__(UPD_ZG * RED_THREADS) void k_dots(Geo g, Range3 r, 
     for (int z = 0; z < UPD_ZG; ++z) {
         if (z > 0) __syncthreads();
         if (zg == z) {
-            double s1 = z == 0 ? 0.0 : carry[0][tid], s2 = z == 0 || !TWO ? 0.0 : carry[TWO ? 1 : 0][tid];
+            double s1 = z == 0 ? 0.0 : carry[0][tid], s2 = z == 0 || !TWO ? 0.0 : carry[TWO][tid];
 #pragma unroll
             for (int u = 0; u < UPD_KP; ++u) {
                 s1 = own && u < cnt ? s1 + b[u] : s1;
@@ -1258,7 +1258,7 @@ __global__ __launch_bounds__(UPD_ZG * RED_THREADS) void k_dots(Geo g, Range3 r, 
             }
             if (z < UPD_ZG - 1) {
                 carry[0][tid] = s1;
-                if (TWO) carry[1][tid] = s2;
+                if (TWO) carry[TWO][tid] = s2;
             } else {
                 s1 = wave_sum(s1);
                 if (TWO) s2 = wave_sum(s2);
@@ -1294,20 +1294,45 @@ __global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_x_update_split(
                               phi, rr, ra, pa, Ar, rh, p1, p2, nb, sc, fl, pmax, pdot);
 }
 
-__global__ __launch_bounds__(256) void k_ctl_end(const double *pmax, const double *pdot, int64_t nb, double *sc,
-                                                 int *fl) {
-    if (!fl[KF_ACTIVE]) return;
+// The end of an iteration by one workgroup: the norm and <rr, rh> from the partials,
+// then the head of the next iteration, on copies of the scalars and flags that are
+// loaded with the partials (each read behind a store would be a trip to the cache of
+// its own, a dozen one after the other).
+__device__ inline void ctl_end_block(const double *pmax, const double *pdot, int64_t nb, double *sc, int *fl) {
     __shared__ double sm[8];
+    double s[KS_NSLOTS];
+    int f[KF_NSLOTS];
+#pragma unroll
+    for (int q = 0; q < KS_NSLOTS; ++q) s[q] = sc[q];
+#pragma unroll
+    for (int q = 0; q < KF_NSLOTS; ++q) f[q] = fl[q];
+    if (!f[KF_ACTIVE]) return;
     double tm, ts;
     thread_max_sum_parts(pmax, pdot, nb, (int)(threadIdx.x + threadIdx.y * blockDim.x), tm, ts);
-    const double nm = block_max(tm, sm);
-    __syncthreads();
-    const double dt = block_sum(ts, sm + 4);
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        sc[KS_NORM] = nm;
-        sc[KS_RHR_NEXT] = dt;
-        ctl_begin(sc, fl);  // the head of the next iteration
+    tm = wave_max(tm);
+    ts = wave_sum(ts);
+    const int tid = (int)(threadIdx.x + threadIdx.y * blockDim.x);
+    if ((tid & 63) == 0) {
+        sm[tid >> 6] = tm;
+        sm[4 + (tid >> 6)] = ts;
     }
+    __syncthreads();
+    if (tid == 0) {
+        double nm = sm[0];
+        for (int q = 1; q < 4; ++q) nm = max_nan(sm[q], nm);
+        s[KS_NORM] = nm;
+        s[KS_RHR_NEXT] = (sm[4] + sm[5]) + (sm[6] + sm[7]);
+        ctl_begin(s, f);
+#pragma unroll
+        for (int q = 0; q < KS_NSLOTS; ++q) sc[q] = s[q];
+#pragma unroll
+        for (int q = 0; q < KF_NSLOTS; ++q) fl[q] = f[q];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_ctl_end(const double *pmax, const double *pdot, int64_t nb, double *sc,
+                                                 int *fl) {
+    ctl_end_block(pmax, pdot, nb, sc, fl);
 }
 
 __global__ __launch_bounds__(256) void k_set_rhr(const double *part, int64_t nb, double *sc) {
@@ -1435,18 +1460,7 @@ __global__ __launch_bounds__(SPLIT ? RED_THREADS * UPD_ZG : RED_THREADS) void k_
 // one workgroup per case
 __global__ __launch_bounds__(256) void k_ctl_end_batch(const KBatchCase *__restrict__ cases) {
     const KBatchCase &K = cases[blockIdx.x];
-    if (!K.fl[KF_ACTIVE]) return;
-    __shared__ double sm[8];
-    double tm, ts;
-    thread_max_sum_parts(K.part3, K.part4, K.nb, (int)(threadIdx.x + threadIdx.y * blockDim.x), tm, ts);
-    const double nm = block_max(tm, sm);
-    __syncthreads();
-    const double dt = block_sum(ts, sm + 4);
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        K.sc[KS_NORM] = nm;
-        K.sc[KS_RHR_NEXT] = dt;
-        ctl_begin(K.sc, K.fl);
-    }
+    ctl_end_block(K.part3, K.part4, K.nb, K.sc, K.fl);
 }
 
 // rr = bb - rr, rh = rr with their partials, and max|bb| partials (part3)

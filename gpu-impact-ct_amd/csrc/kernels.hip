@@ -995,6 +995,7 @@ template <typename T, typename TO, int TPB, int PXM>
 __global__ __launch_bounds__(TPB) void k_jor_vec(Geo g, Coef c, Range3 r, JorVecShape sh, int nbw, int nbz,
                                                          T omega, const T *__restrict__ rel, const T *__restrict__ bb,
                                                          TO *__restrict__ out, const int *active) {
+    warm_args<Geo, Coef, Range3, JorVecShape, int, int, T, const T *, const T *, TO *, const int *>();
     if (active && !*active) return;
     int tw, dummy, bz;
     if (!xcd_tile(nbw, 1, nbz, tw, dummy, bz)) return;
@@ -1007,6 +1008,7 @@ __global__ __launch_bounds__(TPB) void k_jor_vec(Geo g, Coef c, Range3 r, JorVec
 template <typename T, int TPB, int PXM>
 __global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, Coef c, Range3 r, JorVecShape sh, int nbw, int nbz,
                                                  const T *__restrict__ x, T *__restrict__ lap, const int *active) {
+    warm_args<Geo, Coef, Range3, JorVecShape, int, int, const T *, T *, const int *>();
     if (active && !*active) return;
     int tw, dummy, bz;
     if (!xcd_tile(nbw, 1, nbz, tw, dummy, bz)) return;
@@ -1246,6 +1248,7 @@ template <typename T, typename TO, int TPB, bool PX, bool PZ>
 __global__ __launch_bounds__(TPB) void k_jor_pair(Geo g, Coef c, Range3 r, JorVecShape sh, int nt, int nbz, T omega,
                                                   const T *__restrict__ rel, const T *__restrict__ bb,
                                                   TO *__restrict__ out, const int *active) {
+    warm_args<Geo, Coef, Range3, JorVecShape, int, int, T, const T *, const T *, TO *, const int *>();
     if (active && !*active) return;
     int tw, dummy, bz;
     if (!xcd_tile(nt, 1, nbz, tw, dummy, bz)) return;

@@ -1933,6 +1933,10 @@ void launch_jor_f32_to64(hipStream_t s, const Geo &g, const Coef &c, const Box &
 // the latency of the chain barrier to barrier; starting a block costs about five
 // planes of latency.  Within 6 % of the best of all shapes on 33x17x17 to
 // 385x193x193 (10 % of FP32 at 97^3).
+// The cases of a batch stop at iterations of their own, so its shape has to serve the
+// last ones too: by the time with all of them running, a step of 32 tubes took 1935 to
+// 2366 ms as the iterations spread (2084 to 2266 with single sweeps), by the weighted
+// times below 1771 to 1972; of six tubes 338 and 329.
 template <typename F>
 static PairShape pair_shape(int n, int max_planes, F box) {
     PairShape best;
@@ -1943,12 +1947,21 @@ static PairShape pair_shape(int n, int max_planes, F box) {
         if (!fits) continue;
         for (int nbz = 1, kc; nbz <= max_planes; nbz = kc > 1 ? (max_planes + kc - 2) / (kc - 1) : max_planes + 1) {
             kc = (max_planes + nbz - 1) / nbz;  // the fewest chunks of each length
-            int64_t blocks = 0;
-            for (int q = 0; q < n; ++q) blocks += (int64_t)box(q).tiles(tpb) * ((box(q).planes + kc - 1) / kc);
-            const double load = std::ceil((double)blocks / 256.0);  // on the most loaded compute unit
-            const double resident = std::min(load, 1024.0 / tpb);
-            const double plane = std::max(1200.0, resident * tpb / 256.0 * 1000.0);
-            const double t = load / resident * (6000.0 + (kc + 2) * plane);
+            int64_t blocks = 0, largest = 0;
+            for (int q = 0; q < n; ++q) {
+                const int64_t b = (int64_t)box(q).tiles(tpb) * ((box(q).planes + kc - 1) / kc);
+                blocks += b;
+                largest = std::max(largest, b);
+            }
+            auto time = [&](int64_t b) {
+                const double load = std::ceil((double)b / 256.0);  // on the most loaded compute unit
+                const double resident = std::min(load, 1024.0 / tpb);
+                const double plane = std::max(1200.0, resident * tpb / 256.0 * 1000.0);
+                return load / resident * (6000.0 + (kc + 2) * plane);
+            };
+            // of several boxes some stop early: all of them half of the time, then half, then
+            // the largest alone
+            const double t = n == 1 ? time(blocks) : 2.0 * time(blocks) + time((blocks + 1) / 2) + time(largest);
             if (best.tpb == 0 || t < best_time) {
                 best_time = t;
                 best = PairShape{tpb, kc};

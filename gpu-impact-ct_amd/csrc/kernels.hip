@@ -1041,8 +1041,8 @@ __global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, Coef c, Range3 r, JorVec
 // vector ALU bounds it (about 30 instructions a point and sweep, 13 of them the
 // IEEE division).  Measured, microseconds for two sweeps, two launches -> a pair:
 //               33x17x17    65^3       97^3       193x97x97  257x129x129 385x193x193
-//   FP64        7.0 ->  4.9 8.8 -> 7.8 12.6 -> 12.3 19.4 -> 16.5 38.4 -> 30.9 164 -> 93.5
-//   FP32        7.8 ->  5.4 8.4 -> 6.5 12.6 -> 10.7 14.4 -> 13.9 24.0 -> 22.4 55.2 -> 51.2
+//   FP64        7.0 ->  4.9 8.8 -> 7.7 12.6 -> 12.2 19.4 -> 16.5 38.4 -> 28.7 164 -> 93.5
+//   FP32        7.8 ->  5.2 8.4 -> 6.4 12.6 -> 10.6 14.4 -> 13.9 24.0 -> 22.4 55.2 -> 51.2
 // A reciprocal shared by the two sweeps with the quotient corrected to the IEEE
 // one costs, with the range checks, as many instructions as it saves.
 // Block function of stretch tw, z chunk bz (the single-case and the batched kernel;

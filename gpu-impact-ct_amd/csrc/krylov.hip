@@ -925,7 +925,7 @@ __global__ void k_ctl_resume(double *sc, int *fl) {
 // may clear it while later workgroups start, and either value they see leads
 // to the same decision.
 __device__ inline bool wg_active(const int *fl, int *s_go) {
-    if (threadIdx.x == 0 && threadIdx.y == 0) *s_go = fl[KF_ACTIVE];
+    if (threadIdx.x == 0 && threadIdx.y == 0 && threadIdx.z == 0) *s_go = fl[KF_ACTIVE];
     __syncthreads();
     return *s_go != 0;
 }
@@ -959,7 +959,8 @@ __device__ inline void split_sum_parts(const double *part, int64_t nb, int tid, 
 // a thread that walks its chunk's planes one by one waits once a plane.  Four groups
 // of planes against one: 5.4 -> 3.7 us at 33x17x17, 6.6 -> 4.4 at 65^3, 12.3 -> 8.1 at
 // 193x97x97, 18.9 -> 18.0 at 257x129x129 (5.7 TB/s), 58.2 -> 54.6 at 385x193x193.
-template <bool FIRST = false>
+// ASK: the flag is asked before anything is loaded (a batch's stopped cases load nothing).
+template <bool FIRST, bool ASK>
 __device__ inline void s_update_block(const Geo &g, const Range3 &r, int bx, int by, int bz, int nbz, int64_t pi,
                                       double *rr, const double *Ap, const double *part, int64_t nb, double *sc,
                                       int *fl, const FirstSweep &fs = FirstSweep{}) {
@@ -967,7 +968,8 @@ __device__ inline void s_update_block(const Geo &g, const Range3 &r, int bx, int
     __shared__ int s_go;
     const int tid = (int)(threadIdx.x + RED_TX * threadIdx.y);
     const int zg = __builtin_amdgcn_readfirstlane((int)threadIdx.z);
-    if (tid == 0 && zg == 0) s_go = fl[KF_ACTIVE];
+    if (ASK && !wg_active(fl, &s_go)) return;
+    if (!ASK && tid == 0 && zg == 0) s_go = fl[KF_ACTIVE];
     const int i = r.lo0 + bx * RED_TX + (int)threadIdx.x;
     const int j = r.lo1 + by * RED_TY + (int)threadIdx.y;
     const bool own = i < r.lo0 + r.n0 && j < r.lo1 + r.n1;
@@ -1014,7 +1016,7 @@ template <bool FIRST>
 __global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_s_update_alpha(Geo g, Range3 r, double *rr, const double *Ap,
                                                                         const double *part, int64_t nb, double *sc,
                                                                         int *fl, FirstSweep fs) {
-    s_update_block<FIRST>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(), rr,
+    s_update_block<FIRST, false>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(), rr,
                           Ap, part, nb, sc, fl, fs);
 }
 
@@ -1118,9 +1120,9 @@ __global__ __launch_bounds__(256) void k_x_update_omega(Geo g, Range3 r, double 
 // The same update with the chunk's planes on UPD_ZG groups.  The chunk's sum is still
 // formed in plane order: the groups take turns, each adding its products to what the
 // group below passes on, so the partials are the same bits.  PRE: ra is another
-// field than rr (the preconditioned direction).  8.3 -> 7.1 us at 33x17x17, 11.0 ->
-// 9.2 at 65^3, 16.9 -> 11.7 at 118x71x91, 17.0 -> 14.5 at 129x97x97.
-template <bool PRE>
+// field than rr (the preconditioned direction); ASK as in the s update.  8.3 -> 7.1 us
+// at 33x17x17, 11.0 -> 9.2 at 65^3, 16.9 -> 11.7 at 118x71x91, 17.0 -> 14.5 at 129x97x97.
+template <bool PRE, bool ASK>
 __device__ inline void x_update_split_block(const Geo &g, const Range3 &r, int bx, int by, int bz, int nbz, int64_t pi,
                                             double *phi, double *rr, const double *ra, const double *pa,
                                             const double *Ar, const double *rh, const double *p1, const double *p2,
@@ -1129,7 +1131,8 @@ __device__ inline void x_update_split_block(const Geo &g, const Range3 &r, int b
     __shared__ int s_go;
     const int tid = (int)(threadIdx.x + RED_TX * threadIdx.y);
     const int zg = __builtin_amdgcn_readfirstlane((int)threadIdx.z);
-    if (tid == 0 && zg == 0) s_go = fl[KF_ACTIVE];
+    if (ASK && !wg_active(fl, &s_go)) return;
+    if (!ASK && tid == 0 && zg == 0) s_go = fl[KF_ACTIVE];
     const int i = r.lo0 + bx * RED_TX + (int)threadIdx.x;
     const int j = r.lo1 + by * RED_TY + (int)threadIdx.y;
     const bool own = i < r.lo0 + r.n0 && j < r.lo1 + r.n1;
@@ -1290,7 +1293,7 @@ template <bool PRE>
 __global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_x_update_split(
     Geo g, Range3 r, double *phi, double *rr, const double *ra, const double *pa, const double *Ar, const double *rh,
     const double *p1, const double *p2, int64_t nb, double *sc, int *fl, double *pmax, double *pdot) {
-    x_update_split_block<PRE>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(),
+    x_update_split_block<PRE, false>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(),
                               phi, rr, ra, pa, Ar, rh, p1, p2, nb, sc, fl, pmax, pdot);
 }
 
@@ -1434,9 +1437,8 @@ __global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_s_update_batch(const KB
     const int q = batch_tile(cases, tile_case, ntiles, bx, by, bz, pi);
     if (q < 0) return;
     const KBatchCase &K = cases[q];
-    if (!K.fl[KF_ACTIVE]) return;  // a stopped case loads nothing
-    s_update_block<FIRST>(K.g, K.r, bx, by, bz, K.nbz, pi, K.rr, K.Ap, K.part1, K.nb, K.sc, K.fl,
-                          batch_first(K, omega));
+    s_update_block<FIRST, true>(K.g, K.r, bx, by, bz, K.nbz, pi, K.rr, K.Ap, K.part1, K.nb, K.sc, K.fl,
+                                batch_first(K, omega));
 }
 
 template <bool SPLIT>
@@ -1447,11 +1449,10 @@ __global__ __launch_bounds__(SPLIT ? RED_THREADS * UPD_ZG : RED_THREADS) void k_
     const int q = batch_tile(cases, tile_case, ntiles, bx, by, bz, pi);
     if (q < 0) return;
     const KBatchCase &K = cases[q];
-    if (!K.fl[KF_ACTIVE]) return;
     const double *ra = pre ? K.z2 : K.rr, *pa = pre ? K.z1 : K.pk;
     if constexpr (SPLIT)
-        x_update_split_block<true>(K.g, K.r, bx, by, bz, K.nbz, pi, K.phi, K.rr, ra, pa, K.Ar, K.rh, K.part1, K.part2,
-                                   K.nb, K.sc, K.fl, K.part3, K.part4);
+        x_update_split_block<true, true>(K.g, K.r, bx, by, bz, K.nbz, pi, K.phi, K.rr, ra, pa, K.Ar, K.rh, K.part1,
+                                         K.part2, K.nb, K.sc, K.fl, K.part3, K.part4);
     else
         x_update_block(K.g, K.r, bx, by, bz, K.nbz, pi, K.phi, K.rr, ra, pa, K.Ar, K.rh, K.part1, K.part2, K.nb, K.sc,
                        K.fl, K.part3, K.part4);

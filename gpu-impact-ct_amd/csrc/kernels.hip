@@ -2013,13 +2013,16 @@ static void launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b
 // the rule is what it can do: rows of which four fit a block (half of its entries
 // are then stored: FP64 rows to 506 points, FP32 to 1012), at least two rows' worth
 // of entries to wrap a periodic y by, nothing that the second sweep would read
-// from a ghost point that is not there.
+// from a ghost point that is not there, and, across a periodic x, rows of two vectors
+// or more (the pair carries one wrapped neighbour a vector; a level of a thin grid may
+// have both ends of its row in one).
 bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32) {
     if (!c.dg_walls0) return false;
     for (int d = 0; d < 3; ++d)
         if (b.lo[d] != g.Sp[d] || b.hi[d] != g.Np[d]) return false;
     int nbw, nbz;
     const JorVecShape sh = jor_vec_shape(g, R(b), fp32 ? 4 : 2, 256, 0, nbw, nbz);
+    if (g.per[0] && sh.nv < 2) return false;
     return 4 * (sh.nent + 1) <= 1024 && 2 * (sh.nent + 1) <= sh.nent_all && b.hi[2] > b.lo[2];
 }
 

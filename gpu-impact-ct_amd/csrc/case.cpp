@@ -1048,7 +1048,8 @@ static int jor_run(ih_case *c, int n_sweeps, double omega, const Box &b, ih_fiel
         HIPCHK(hipMemcpyAsync(y, x, sizeof(double) * (size_t)c->g.fe, hipMemcpyDeviceToDevice, c->stream));
     const bool with_bc = pbc_substep == 3 && c->ctlab;
     int rc;
-    const bool pairs = whole && !with_bc && jor_pair_ok(c->g, c->c, b, false);
+    // (a field relaxed on itself: a pair's blocks read bb beyond the points they write)
+    const bool pairs = whole && !with_bc && rel != bb && jor_pair_ok(c->g, c->c, b, false);
     const bool singles = n_sweeps > 0 && (!pairs || n_sweeps % 2);
     const JorLaunch sh = singles ? jor_shape(c, b, false, [&](JorLaunch l) {
         launch_jor(c->stream, c->g, c->c, b, omega, x, B, y, l);
@@ -2245,8 +2246,9 @@ int ih_device_jacobi_solver(ih_case *c, int grid_id, double omega, int SS1, int 
     bool stopped = false;
     // Between two tests nothing but the sweeps touches rel unless the pressure is
     // imposed: they are one call then, over the whole range with nothing coupled past
-    // a wall (sweeps over less, or reading ghost points, are a call each).
-    bool run = c->c.dg_walls0 && !(c->ctlab && substep == 3);
+    // a wall (sweeps over less, or reading ghost points, or on rel itself, whose result
+    // is the next one's right-hand side, are a call each).
+    bool run = c->c.dg_walls0 && !(c->ctlab && substep == 3) && ar.field != ab.field;
     const Box pb = pbox(c->g);
     for (int d = 0; d < 3; ++d) run = run && b.lo[d] == pb.lo[d] && b.hi[d] == pb.hi[d];
     const int trips = run ? mode_j : 1;

@@ -1062,18 +1062,21 @@ __device__ inline void jor_pair_block(const Geo g, const Range3 r, const JorVecS
     const int tid = threadIdx.x, lane = tid & 63;
     const int nent = sh.nent, H = nent + 1;
     const int q = tw * (TPB - 2 * H) - H + tid;
-    // past the first or the last row: the opposite row of a periodic y, else dead
+    // past the first or the last row: the opposite row of a periodic y, else the row of
+    // ghost points beyond the wall, whose coefficients are zero (loaded all the same: zero
+    // times a value that is not finite reaches the wall point); further out dead
     const bool inside = q >= 0 && q < sh.nent_all;
     // (from one row below, where the outer neighbours are loads, to two above: nothing
     // further out is used)
-    const bool live = inside || (g.per[1] && q < sh.nent_all + 2 * H);
-    int qm = q < 0 ? q + sh.nent_all : (q >= sh.nent_all ? q - sh.nent_all : q);
-    if (!live) qm = 0;
-    const int jj = qm / nent, e = qm - jj * nent;
+    const bool live = q >= -nent && q < sh.nent_all + (g.per[1] ? 2 * H : nent);
+    int qm = q + nent;
+    if (g.per[1]) qm += q < 0 ? sh.nent_all : (q >= sh.nent_all ? -sh.nent_all : 0);
+    if (!live) qm = nent;
+    const int jj = qm / nent - 1, e = qm - (jj + 1) * nent;
     const int j = r.lo1 + jj;
     const int is = sh.i0 + V * (e - 1);
     const int hi0 = r.lo0 + r.n0 - 1;
-    const bool row = live && e >= 1 && e <= sh.nv;  // a vector with points of the range
+    const bool row = live && (inside || g.per[1]) && e >= 1 && e <= sh.nv;  // a vector with points of the range
     const bool full = row && is >= r.lo0 && is + V - 1 <= hi0;
     const bool store = inside && row && tid >= H && tid < TPB - H;
     const int c0 = g.cst[0], c1 = g.cst[1], c2 = g.cst[2];
@@ -1086,7 +1089,8 @@ __device__ inline void jor_pair_block(const Geo g, const Range3 r, const JorVecS
         a1p[t] = g1[2 * c0 + ic];
         a1d[t] = g1[1 * c0 + ic];
     }
-    const T a2m = g2[0 * c1 + j], a2p = g2[2 * c1 + j], a2d = g2[1 * c1 + j];
+    const int jc = j < r.lo1 + r.n1 ? j : r.lo1;  // (the tables start at 0)
+    const T a2m = g2[0 * c1 + jc], a2p = g2[2 * c1 + jc], a2d = g2[1 * c1 + jc];
     int kc0, kc1;
     red_chunk(r, bz, nbz, kc0, kc1);
     const int lo2 = r.lo2, hi2 = r.lo2 + r.n2 - 1;
@@ -1099,7 +1103,7 @@ __device__ inline void jor_pair_block(const Geo g, const Range3 r, const JorVecS
     const int64_t xy = gidx(g, is, j, 0) - 3 * g.pxy;
     // dead entries read zeros, whatever the plane
     const PC xp = live ? rel + xy + 3 * g.pxy : zeros;
-    const PC bp = live ? bb + xy + 3 * g.pxy : zeros;
+    const PC bp = live ? bb + gidx(g, is, jc, 0) : zeros;
     // outer y neighbour of the stretch's first and last row
     const bool lowe = tid < nent, highe = tid >= TPB - nent;
     int64_t dye = lowe ? -(int64_t)g.px : (int64_t)g.px;

@@ -1183,7 +1183,8 @@ static int bicgstab_run(ih_case *c, double eps, int n_it_max, const int ss[3], c
     // iterations enqueued per convergence check: a preconditioned iteration is
     // many launches, and those enqueued past the stop run as no-ops
     const int batch = mg ? 2 : 8;
-    for (;;) {
+    for (int enqueued = 0;; enqueued += batch) {
+        k.ask = enqueued < KRYLOV_ASK;
         for (int q = 0; q < batch; ++q) launch_krylov_iteration(s, c->g, c->c, b, k);
         LAUNCHCHK();
         HIPCHK(hipMemcpyAsync(c->hkfl, c->kfl, sizeof(int) * KF_NSLOTS, hipMemcpyDeviceToHost, s));

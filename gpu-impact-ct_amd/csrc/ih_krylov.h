@@ -50,7 +50,16 @@ struct KrylovPtrs {
     // max-norm and <r, rh> partials of the solution update: their own buffers,
     // because that kernel reduces the operator's partials in part1/part2 itself
     double *part3 = nullptr, *part4 = nullptr;
+    // the s and x updates ask for the active flag before they load anything: for the
+    // first KRYLOV_ASK iterations of a solve
+    bool ask = false;
 };
+// Of the iterations enqueued together up to seven follow the stop.  One of them costs 7
+// (118x71x91) to 32 (257x129x129) and 135 us (385x193x193) more where its updates do not
+// ask, an iteration that runs 0.4 to 1.3 us more where they do: the costs are even at
+// 50 to 350 iterations a solve.  Solves of 1 iteration, not asking and asking:
+// 257x129x129 660 and 427 us, 385x193x193 2020 and 1095.
+constexpr int KRYLOV_ASK = 64;
 
 // dot modes of the operator kernel
 enum { KDOT_NONE = 0, KDOT_W = 1, KDOT_SELF = 2, KDOT_PAIR = 3 };

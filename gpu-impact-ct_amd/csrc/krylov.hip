@@ -959,11 +959,13 @@ __device__ inline void split_sum_parts(const double *part, int64_t nb, int tid, 
 // a thread that walks its chunk's planes one by one waits once a plane.  Four groups
 // of planes against one: 5.4 -> 3.7 us at 33x17x17, 6.6 -> 4.4 at 65^3, 12.3 -> 8.1 at
 // 193x97x97, 18.9 -> 18.0 at 257x129x129 (5.7 TB/s), 58.2 -> 54.6 at 385x193x193.
-// ASK: the flag is asked before anything is loaded (a batch's stopped cases load nothing).
+// ASK: the flag is asked before anything is loaded, so an iteration enqueued past the stop
+// (up to seven a solve, and a batch's stopped cases) moves nothing; else it is read with
+// the loads, which is the faster form of an iteration that runs (KrylovPtrs::ask).
 template <bool FIRST, bool ASK>
 __device__ inline void s_update_block(const Geo &g, const Range3 &r, int bx, int by, int bz, int nbz, int64_t pi,
                                       double *rr, const double *Ap, const double *part, int64_t nb, double *sc,
-                                      int *fl, const FirstSweep &fs = FirstSweep{}) {
+                                      int *fl, const FirstSweep &fs) {
     __shared__ double sm[4];
     __shared__ int s_go;
     const int tid = (int)(threadIdx.x + RED_TX * threadIdx.y);
@@ -1012,12 +1014,12 @@ __device__ inline void s_update_block(const Geo &g, const Range3 &r, int bx, int
     }
 }
 
-template <bool FIRST>
+template <bool FIRST, bool ASK>
 __global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_s_update_alpha(Geo g, Range3 r, double *rr, const double *Ap,
                                                                         const double *part, int64_t nb, double *sc,
                                                                         int *fl, FirstSweep fs) {
-    s_update_block<FIRST, false>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(), rr,
-                          Ap, part, nb, sc, fl, fs);
+    s_update_block<FIRST, ASK>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(),
+                               rr, Ap, part, nb, sc, fl, fs);
 }
 
 // omega = <r, Ar>/<Ar, Ar> (a vanishing <Ar, Ar> is a breakdown), then
@@ -1289,12 +1291,12 @@ static bool x_split(int64_t tiles) {
     return rounds <= 1 || 8 * tiles >= 7 * rounds * cus;
 }
 
-template <bool PRE>
+template <bool PRE, bool ASK>
 __global__ __launch_bounds__(RED_THREADS *UPD_ZG) void k_x_update_split(
     Geo g, Range3 r, double *phi, double *rr, const double *ra, const double *pa, const double *Ar, const double *rh,
     const double *p1, const double *p2, int64_t nb, double *sc, int *fl, double *pmax, double *pdot) {
-    x_update_split_block<PRE, false>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z, part_index(),
-                              phi, rr, ra, pa, Ar, rh, p1, p2, nb, sc, fl, pmax, pdot);
+    x_update_split_block<PRE, ASK>(g, r, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.z,
+                                   part_index(), phi, rr, ra, pa, Ar, rh, p1, p2, nb, sc, fl, pmax, pdot);
 }
 
 // The end of an iteration by one workgroup: the norm and <rr, rh> from the partials,
@@ -1668,25 +1670,23 @@ static void launch_precond(hipStream_t s, const Geo &g, const Coef &c, const Box
 
 static void launch_s_update(hipStream_t s, const Geo &g, const Range3 &r, int64_t nb, const KrylovPtrs &k, bool first,
                             const FirstSweep &fs) {
-    if (first)
-        hipLaunchKernelGGL(k_s_update_alpha<true>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.rr, k.Ap,
-                           k.part1, nb, k.sc, k.fl, fs);
-    else
-        hipLaunchKernelGGL(k_s_update_alpha<false>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.rr, k.Ap,
-                           k.part1, nb, k.sc, k.fl, fs);
+    auto *const kern = first ? (k.ask ? k_s_update_alpha<true, true> : k_s_update_alpha<true, false>)
+                             : (k.ask ? k_s_update_alpha<false, true> : k_s_update_alpha<false, false>);
+    hipLaunchKernelGGL(kern, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.rr, k.Ap, k.part1, nb, k.sc, k.fl,
+                       fs);
 }
 
 static void launch_x_update(hipStream_t s, const Geo &g, const Range3 &r, int64_t nb, const KrylovPtrs &k, bool pre) {
     const double *ra = pre ? k.z2 : k.rr, *pa = pre ? k.z1 : k.pk;
-    if (x_split(nb) && pre)
-        hipLaunchKernelGGL(k_x_update_split<true>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.phi, k.rr,
-                           ra, pa, k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
-    else if (x_split(nb))
-        hipLaunchKernelGGL(k_x_update_split<false>, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.phi, k.rr,
-                           ra, pa, k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
-    else
+    if (!x_split(nb)) {
         hipLaunchKernelGGL(k_x_update_omega, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.phi, k.rr, ra, pa,
                            k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
+        return;
+    }
+    auto *const kern = pre ? (k.ask ? k_x_update_split<true, true> : k_x_update_split<true, false>)
+                           : (k.ask ? k_x_update_split<false, true> : k_x_update_split<false, false>);
+    hipLaunchKernelGGL(kern, red_grid(r), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, g, r, k.phi, k.rr, ra, pa, k.Ar, k.rh,
+                       k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
 }
 
 void launch_krylov_iteration(hipStream_t s, const Geo &g, const Coef &c, const Box &b, const KrylovPtrs &k) {

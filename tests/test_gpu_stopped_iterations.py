@@ -1,0 +1,54 @@
+"""Iterations of BiCGstab that are enqueued past the stop: solves that end at every
+place of the eight enqueued together, before and after the updates change the way
+they learn of it (64 iterations), against the oracle bit for bit; and what a stopped
+iteration costs, against one that runs."""
+import time
+
+import numpy as np
+import pytest
+
+import impact_hip as ih
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+W6, PZ = (1,) * 6, (1, 1, 1, 1, -1, -1)
+
+
+@pytest.mark.parametrize("its", [1, 2, 7, 8, 9, 63, 64, 65, 71, 73])
+@pytest.mark.parametrize("sweeps", [0, 3])
+def test_solves_that_stop(its, sweeps):
+    N = (34, 19, 37)
+    oc, gc = O.OracleCase(N, PZ, (2.0, 1.0, 1.0), (0.0, 0.0, 0.0)), ih.Case(N, PZ, (2.0, 1.0, 1.0))
+    s = tuple(slice(oc.Sp[d] + 3, oc.Np[d] + 4) for d in (2, 1, 0))
+    rng = np.random.default_rng(16)
+    bb, phi = rng.standard_normal(oc.shape), rng.standard_normal(oc.shape)
+    gc.upload(ih.RES, bb)
+    gc.upload(ih.PRE, phi)
+    if sweeps:
+        so, sg = oc.bicgstab_mixed(0.0, its, oc.Sp, oc.Np, bb, phi, sweeps), gc.bicgstab_mixed(0.0, its, oc.Sp, oc.Np, sweeps)
+    else:
+        so, sg = oc.bicgstab(0.0, its, oc.Sp, oc.Np, bb, phi), gc.bicgstab(0.0, its, oc.Sp, oc.Np)
+    assert (so.iterations, so.exit_reason, so.norm_inf_final) == (sg.iterations, sg.exit_reason, sg.norm_inf_final)
+    got = gc.download(ih.PRE)[s]
+    assert np.array_equal(got, phi[s]), f"{int((got != phi[s]).sum())} values differ"
+    gc.close()
+
+
+def test_a_stopped_iteration_moves_nothing():
+    """A solve of one iteration enqueues eight.  The updates of one that runs are two
+    fifths of it; if the stopped ones moved as much, the solve of one would take over
+    two fifths of the solve of eight (0.42 measured so), and takes 0.23 if not."""
+    N = (385, 193, 193)
+    gc = ih.Case(N, W6, (2.0, 1.0, 1.0))
+    gc.upload(ih.RES, np.random.default_rng(17).standard_normal(gc.shape))
+    best = {1: np.inf, 8: np.inf}
+    for _ in range(10):
+        for its in best:
+            gc.fill(ih.PRE, 0.0)
+            gc.sync()
+            t = time.perf_counter()
+            gc.bicgstab(0.0, its, (1, 1, 1), N)
+            best[its] = min(best[its], time.perf_counter() - t)
+    assert best[1] < 0.33 * best[8], best
+    gc.close()

@@ -2931,7 +2931,7 @@ int batch_step_tables(ih_batch *b, int sweeps) {
                 mid[par].push_back(m);
             }
             it.zero = c->c.zero;
-            pairs = pairs && jor_pair_ok(g, c->c, pb, true);
+            pairs = pairs && jor_pair_fits(g, c->c, pb, true);
             pair.push_back(it);
             // the last sweep reads e0 after an even number of middle sweeps
             float *xl = ((sweeps - 2) % 2 == 0) ? e0 : e1;
@@ -2944,6 +2944,7 @@ int batch_step_tables(ih_batch *b, int sweeps) {
             }
         }
     }
+    pairs = pairs && jor_pair_batch_ok(pair);
     if (pairs) {
         const PairShape shape = jor_pair_batch_shape(pair);
         b->ppair_tpb = shape.tpb;

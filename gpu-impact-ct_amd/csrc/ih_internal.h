@@ -112,8 +112,9 @@ void launch_jor(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double
 void launch_jor_f32(hipStream_t s, const Geo &g, const Coef &c, const Box &b, float omega, const float *rel,
                     const float *bb, float *out, const int *active = nullptr, JorLaunch shape = JorLaunch());
 // Two JOR sweeps in one launch, out = sweep(sweep(rel)), the bits of two single
-// ones.  jor_pair_ok: whether box b takes it (the whole pressure range, no coupling
-// past a wall, rows short enough for a block).
+// ones.  jor_pair_fits: whether box b can take it (the whole pressure range, no coupling
+// past a wall, rows short enough for a block); jor_pair_ok: and whether it is the faster.
+bool jor_pair_fits(const Geo &g, const Coef &c, const Box &b, bool fp32);
 bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32);
 void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double omega, const double *rel,
                      const double *bb, double *out, const int *active);
@@ -214,11 +215,13 @@ void launch_jor_f32_first(hipStream_t s, const Geo &g, const Coef &c, const Box 
 // batched FP32 preconditioner sweeps (flat tile -> item table over ntiles tiles)
 void launch_jor_batch_f32(hipStream_t s, const JorBatchItem *items, const int *tile_item, int ntiles, float omega,
                           bool to64, bool any_periodic_x);
-// batched FP32 sweep pairs, each case's box taken by jor_pair_ok: the launch shape of a
-// batch, a case's tiles in it (sets sh, ntxy, nbz), the launch
+// batched FP32 sweep pairs, each case's box of jor_pair_fits: whether they are the faster
+// form (of the items g and r are read), the launch shape of a batch, a case's tiles in
+// it (sets sh, ntxy, nbz), the launch
 struct PairShape {
     int tpb = 0, kc = 0;  // threads a block, planes a z chunk
 };
+bool jor_pair_batch_ok(const std::vector<JorBatchItem> &items);
 PairShape jor_pair_batch_shape(const std::vector<JorBatchItem> &items);
 int jor_pair_batch_tiles(PairShape shape, JorBatchItem &it);
 void launch_jor_pair_batch(hipStream_t s, const JorBatchItem *items, const int *tile_item, int ntiles, int tpb,

@@ -2013,14 +2013,13 @@ static void launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b
 #undef IH_JPL
 }
 
-// The pair is the faster form at every size it fits (figures above k_jor_pair), so
-// the rule is what it can do: rows of which four fit a block (half of its entries
-// are then stored: FP64 rows to 506 points, FP32 to 1012), at least two rows' worth
-// of entries to wrap a periodic y by, nothing that the second sweep would read
-// from a ghost point that is not there, and, across a periodic x, rows of two vectors
-// or more (the pair carries one wrapped neighbour a vector; a level of a thin grid may
-// have both ends of its row in one).
-bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32) {
+// What the pair can do: rows of which four fit a block (half of its entries are then
+// stored: FP64 rows to 506 points, FP32 to 1012), at least two rows' worth of entries to
+// wrap a periodic y by, nothing that the second sweep would read from a ghost point that
+// is not there, and, across a periodic x, rows of two vectors or more (the pair carries
+// one wrapped neighbour a vector; a level of a thin grid may have both ends of its row
+// in one).
+bool jor_pair_fits(const Geo &g, const Coef &c, const Box &b, bool fp32) {
     if (!c.dg_walls0) return false;
     for (int d = 0; d < 3; ++d)
         if (b.lo[d] != g.Sp[d] || b.hi[d] != g.Np[d]) return false;
@@ -2028,6 +2027,43 @@ bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32) {
     const JorVecShape sh = jor_vec_shape(g, R(b), fp32 ? 4 : 2, 256, 0, nbw, nbz);
     if (g.per[0] && sh.nv < 2) return false;
     return 4 * (sh.nent + 1) <= 1024 && 2 * (sh.nent + 1) <= sh.nent_all && b.hi[2] > b.lo[2];
+}
+
+// Where it is the faster form.  Rows of which four fit 512 threads (FP64 to 250 points,
+// FP32 to 500): taken.  Longer rows leave blocks of 1024 threads, of which one fills a
+// compute unit with a barrier a plane, and of these a share of 1 - 2 (nent + 1)/1024
+// stores (0.74 to 0.50):
+//   - past the last-level cache (what a sweep moves, 24 or 12 bytes a point, over 240 MB)
+//     two sweeps of one pass are the faster at every share,
+//   - within it the instructions of the dead entries decide, FP32 the sooner (half of the
+//     bytes for the same instructions),
+//   - on small grids a launch is two sweeps' chain of one block, which is longer in a
+//     block of 1024 threads than in two launches of small ones.
+// Two single sweeps / a pair, microseconds:
+//   FP64 (share)         17x17       65x65       129x129     257x129
+//     270 points (.73)   6.4 / 7.9   13.9 / 12.9  35.0 / 27.2  65.7 / 46.6
+//     420        (.58)   6.7 / 7.9   18.0 / 17.8  51.8 / 46.3   162 / 97
+//     505        (.50)   6.8 / 7.8   20.7 / 20.9  61.1 / 63.2   198 / 101
+//   FP32
+//     505 points (.75)   7.1 / 9.8   14.8 / 14.6  35.2 / 32.3  63.6 / 59.5
+//     640        (.68)   6.9 / 9.8   17.6 / 18.4  41.7 / 41.4   112 / 74
+//     1000       (.50)   8.0 / 10.1  23.3 / 26.9  61.2 / 73.4   180 / 137
+// (33 x 33 rows lose at every long row, 33 x 129 ones, 24 MB and up, are even.)
+// A row of 480 points in FP32 takes 9.0 / 9.1, 14.4 / 14.9, 34.1 / 31.7 and 56.9 / 54.7,
+// at worst (33x129) 14.4 / 17.0.
+static bool pair_pays(bool wide, double bytes, double share, bool fp32) {
+    if (!wide || bytes >= 240e6) return true;
+    return bytes >= 24e6 && share >= (fp32 ? 0.70 : 0.58);
+}
+static bool pair_wide(const JorVecShape &sh) { return 4 * (sh.nent + 1) > 512; }
+static double pair_share(const JorVecShape &sh) { return 1.0 - 2.0 * (sh.nent + 1) / 1024.0; }
+
+bool jor_pair_ok(const Geo &g, const Coef &c, const Box &b, bool fp32) {
+    if (!jor_pair_fits(g, c, b, fp32)) return false;
+    const Range3 r = R(b);
+    int nbw, nbz;
+    const JorVecShape sh = jor_vec_shape(g, r, fp32 ? 4 : 2, 256, 0, nbw, nbz);
+    return pair_pays(pair_wide(sh), (fp32 ? 12.0 : 24.0) * r.n0 * r.n1 * r.n2, pair_share(sh), fp32);
 }
 
 void launch_jor_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double omega, const double *rel,
@@ -2155,6 +2191,21 @@ void launch_jor_batch_f32(hipStream_t s, const JorBatchItem *items, const int *t
             hipLaunchKernelGGL((k_jor_batch<float, TPB, 0>), flat, dim3(TPB), 0, s, items, tile_item, 0, ntiles,
                                omega);
     }
+}
+
+// The rule of one box on the batch's sums: its launches cover all cases, in blocks that
+// the longest row decides.
+bool jor_pair_batch_ok(const std::vector<JorBatchItem> &items) {
+    bool wide = false;
+    double points = 0.0, stored = 0.0;
+    for (const JorBatchItem &it : items) {
+        const JorVecShape sh = pair_box(it.g, it.r, 4).sh;
+        const double n = (double)it.r.n0 * it.r.n1 * it.r.n2;
+        wide = wide || pair_wide(sh);
+        points += n;
+        stored += n * pair_share(sh);
+    }
+    return pair_pays(wide, 12.0 * points, stored / points, true);
 }
 
 PairShape jor_pair_batch_shape(const std::vector<JorBatchItem> &items) {

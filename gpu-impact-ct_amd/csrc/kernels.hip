@@ -109,11 +109,20 @@ __global__ void k_interp_vel_pre(Geo g, Coef c, Range3 r, int q, const double *p
 // them (16 clocks a load and wavefront, of coefficients as of field values), so a
 // thread reads coefficients that its planes share once and overlapping taps along z
 // once, and coefficients along y and z, uniform in a wavefront, are scalar loads.
-// Microseconds at 129x65x65, one point a thread with vector loads -> here:
-//   interp_pre_vel 6.0 -> 4.5, nonlinear_one 7.4 -> 5.9 (7.7 along z: 56 scalar loads a
-// thread), helmholtz_one 11.1 -> 7.8
+// Several planes a thread pay where there are wavefronts left to fill the device; below
+// that a launch is the chain of one thread, which they lengthen (few_waves).
+// Microseconds, one point a thread with vector loads -> one plane here / several:
+//                            33^3 (992 waves)     65^3 (4032)          129x65x65 (8064)     257x129x129
+//   interp_pre_vel along x   3.0 -> 2.8 / 3.2 (4) 4.2 -> 4.0 / 3.6 (4) 5.9 -> 4.6 / 4.2 (4) 27 -> 23 / 15 (4)
+//                        y   3.0 -> 2.5 / 3.4 (4) 4.2 -> 3.5 / 3.6 (4) 5.9 -> 4.4 / 4.7 (4) 27 -> 19 / 19 (4)
+//                        z   3.0 -> 2.8 / 3.2 (4) 4.2 -> 3.6 / 3.4 (4) 5.9 -> 4.6 / 4.1 (4) 27 -> 19 / 13 (4)
+//   nonlinear_one along x    3.2 -> 3.2 / 3.9 (4) 5.0 -> 5.2 / 4.2 (4) 7.6 -> 7.7 / 5.5 (4) 39 -> 43 / 23 (4)
+//                       y    3.2 -> 3.3 / 3.2 (2) 5.0 -> 4.0 / 3.8 (2) 7.6 -> 5.5 / 5.3 (2) 39 -> 29 / 30 (2)
+//                       z    3.2 -> 3.4 / 3.8 (2) 5.0 -> 4.4 / 4.2 (2) 7.6 -> 6.3 / 5.7 (2) 39 -> 31 / 26 (2)
+//   helmholtz_one            3.5 -> 3.6 / 5.3 (4) 6.6 -> 5.9 / 5.5 (4) 10.9 -> 9.0 / 7.8 (4) 63 -> 53 / 35 (4)
+// (nonlinear_one along y at 9x129x129: 10.4 -> 7.4 / 11.3 with 2, 13.2 with 4: one plane
+// always; four planes along z read 56 scalar coefficients a thread, 5.0 at 33^3.)
 typedef const __attribute__((address_space(4))) double *Cs;
-constexpr int KZ = 4;
 
 #define IH_POINT_ROWS(r)                                                                                 \
     const int i = (r).lo0 + (int)(blockIdx.x * BX + threadIdx.x);                                        \
@@ -124,12 +133,12 @@ constexpr int KZ = 4;
     int kk[KZ]; /* planes past the range are formed on its last one and not stored */                    \
     _Pragma("unroll") for (int z = 0; z < KZ; ++z) kk[z] = k0 + z < hi2 ? k0 + z : hi2;
 
-inline dim3 grid_rows(const Range3 &r) {
+inline dim3 grid_rows(const Range3 &r, int KZ) {
     return dim3((unsigned)((r.n0 + BX - 1) / BX), (unsigned)((r.n1 + BY - 1) / BY), (unsigned)((r.n2 + KZ - 1) / KZ));
 }
 
 // values f[z][t] = phi at t + FROM along direction D from plane kk[z]
-template <int D, int N, int FROM>
+template <int D, int N, int FROM, int KZ>
 __device__ inline void load_taps(const Geo &g, const double *phi, int64_t x0, const int *kk, double (*f)[N]) {
     const int64_t s = sh(g, D);
     if constexpr (D < 2) {
@@ -160,12 +169,12 @@ __device__ inline double taps(PC c, int cst, const double *f) {
     return v;
 }
 
-template <int Q>
+template <int Q, int KZ>
 __global__ __launch_bounds__(BX * BY) void k_interp_pre_vel(Geo g, Coef c, Range3 r, const double *__restrict__ phi,
                                                             double *__restrict__ inter) {
     IH_POINT_ROWS(r);
     double f[KZ][6], cx[6];
-    load_taps<Q, 6, -2>(g, phi, x0, kk, f);
+    load_taps<Q, 6, -2, KZ>(g, phi, x0, kk, f);
 #pragma unroll
     for (int t = 0; t < 6; ++t) cx[t] = Q == 0 ? c.Ip[0][t * g.cst[0] + i] : (Q == 1 ? ((Cs)c.Ip[1])[t * g.cst[1] + j] : 0.0);
 #pragma unroll
@@ -545,7 +554,7 @@ __global__ __launch_bounds__(x6::NT) void k_xyz6_t(Geo g, Range3 r, int nbx, int
 }
 
 // one (component, direction) pass of nonlinear, for device_Nonlinear_upwind
-template <int D>
+template <int D, int KZ>
 __global__ __launch_bounds__(BX * BY) void k_nonlinear_one(Geo g, Coef c, Range3 r, int q,
                                                            const double *__restrict__ pp_f,
                                                            const double *__restrict__ vel, double *__restrict__ nl,
@@ -561,7 +570,7 @@ __global__ __launch_bounds__(BX * BY) void k_nonlinear_one(Geo g, Coef c, Range3
         pp[z] = pp_f[x];
         old[z] = assign ? 0.0 : nl[x];
     }
-    load_taps<D, 7, -3>(g, vel, x0, kk, f);
+    load_taps<D, 7, -3, KZ>(g, vel, x0, kk, f);
 #pragma unroll
     for (int t = 0; t < 7; ++t) {
         u[t] = D == 0 ? cU[t * cst + i] : (D == 1 ? ((Cs)cU)[t * cst + j] : 0.0);
@@ -584,6 +593,7 @@ __global__ __launch_bounds__(BX * BY) void k_nonlinear_one(Geo g, Coef c, Range3
     }
 }
 
+template <int KZ>
 __global__ __launch_bounds__(BX * BY) void k_helmholtz_one(Geo g, Coef c, Range3 r, int q, double multL,
                                                            const double *__restrict__ vel, double *__restrict__ nl) {
     IH_POINT_ROWS(r);
@@ -591,7 +601,7 @@ __global__ __launch_bounds__(BX * BY) void k_helmholtz_one(Geo g, Coef c, Range3
     const Cs c2 = (Cs)((q == 1) ? c.u2[1] : c.p2[1]) + j;
     const Cs c3 = (Cs)((q == 2) ? c.u2[2] : c.p2[2]);
     double f1[KZ][7], f2[KZ][7], f3[KZ][7], old[KZ], cx[7];
-    load_taps<2, 7, -3>(g, vel, x0, kk, f3);
+    load_taps<2, 7, -3, KZ>(g, vel, x0, kk, f3);
 #pragma unroll
     for (int z = 0; z < KZ; ++z) {
         const int64_t x = x0 + (int64_t)kk[z] * g.pxy;
@@ -1746,11 +1756,20 @@ void launch_interp_vel_pre(hipStream_t s, const Geo &g, const Coef &c, int q, co
     hipLaunchKernelGGL(k_interp_vel_pre, grid_for(r), dim3(BX, BY, 1), 0, s, g, c, r, q, phi, inter);
 }
 
+// At most eight wavefronts a compute unit at one plane each: measured at 1984 (129x33x33)
+// and 2256 (65x49x49), microseconds with one plane / several:
+//   interp_pre_vel along x 3.2 / 3.2 and 3.5 / 3.3, nonlinear_one along x 3.8 / 4.0 and
+// 4.5 / 4.0, along z 3.8 / 3.9 and 4.0 / 4.0, helmholtz_one 4.4 / 5.4 and 5.2 / 5.5
+// (3120 waves: 5.8 / 5.6).
+static bool few_waves(const Range3 &r) { return (int64_t)((r.n0 + BX - 1) / BX) * r.n1 * r.n2 <= 2048; }
+
 void launch_interp_pre_vel(hipStream_t s, const Geo &g, const Coef &c, int q, const double *phi, double *inter) {
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
-    auto *const k = q == 0 ? k_interp_pre_vel<0> : (q == 1 ? k_interp_pre_vel<1> : k_interp_pre_vel<2>);
-    hipLaunchKernelGGL(k, grid_rows(r), dim3(BX, BY, 1), 0, s, g, c, r, phi, inter);
+    const bool few = few_waves(r);
+    auto *const k = q == 0 ? (few ? k_interp_pre_vel<0, 1> : k_interp_pre_vel<0, 4>)
+                           : (q == 1 ? k_interp_pre_vel<1, 1> : (few ? k_interp_pre_vel<2, 1> : k_interp_pre_vel<2, 4>));
+    hipLaunchKernelGGL(k, grid_rows(r, few || q == 1 ? 1 : 4), dim3(BX, BY, 1), 0, s, g, c, r, phi, inter);
 }
 
 // z chunks of k_nl_helm_rhs_t: at most nlh::AZ planes each, and, where the tile
@@ -1802,15 +1821,20 @@ void launch_nonlinear_one(hipStream_t s, const Geo &g, const Coef &c, int q, int
                           const double *vel, double *nl, int assign) {
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
-    auto *const k = d == 0 ? k_nonlinear_one<0> : (d == 1 ? k_nonlinear_one<1> : k_nonlinear_one<2>);
-    hipLaunchKernelGGL(k, grid_rows(r), dim3(BX, BY, 1), 0, s, g, c, r, q, pp, vel, nl, assign);
+    const bool few = few_waves(r);
+    auto *const k = d == 0 ? (few ? k_nonlinear_one<0, 1> : k_nonlinear_one<0, 4>)
+                           : (d == 1 ? k_nonlinear_one<1, 1> : (few ? k_nonlinear_one<2, 1> : k_nonlinear_one<2, 2>));
+    hipLaunchKernelGGL(k, grid_rows(r, few || d == 1 ? 1 : (d == 0 ? 4 : 2)), dim3(BX, BY, 1), 0, s, g, c, r, q, pp,
+                       vel, nl, assign);
 }
 
 void launch_helmholtz_one(hipStream_t s, const Geo &g, const Coef &c, int q, double multL, const double *vel,
                           double *nl) {
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
-    hipLaunchKernelGGL(k_helmholtz_one, grid_rows(r), dim3(BX, BY, 1), 0, s, g, c, r, q, multL, vel, nl);
+    const bool few = few_waves(r);
+    hipLaunchKernelGGL(few ? k_helmholtz_one<1> : k_helmholtz_one<4>, grid_rows(r, few ? 1 : 4), dim3(BX, BY, 1), 0, s,
+                       g, c, r, q, multL, vel, nl);
 }
 
 void launch_bc_planes(hipStream_t s, const Geo &g, const Coef &c, double *rhs1, double *rhs2, double *rhs3,

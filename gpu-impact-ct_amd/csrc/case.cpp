@@ -1181,9 +1181,11 @@ static int bicgstab_run(ih_case *c, double eps, int n_it_max, const int ss[3], c
     launch_krylov_init(s, c->g, b, F(c, bbf), k.rr, k.rh, k.part1, k.part2, k.sc, k.fl, eps, n_it_max);
     LAUNCHCHK();
     // iterations enqueued per convergence check: a preconditioned iteration is
-    // many launches, and those enqueued past the stop run as no-ops
-    const int batch = mg ? 2 : 8;
-    for (int enqueued = 0;; enqueued += batch) {
+    // many launches, and those enqueued past the stop run as no-ops (on a small grid
+    // eight to ten launches of 3.3 us on the host each, so the first eight are checked
+    // in two parts: a solve of one iteration at 33x17x17 227 -> 169 us)
+    for (int enqueued = 0, batch = 0;; enqueued += batch) {
+        batch = mg ? 2 : (enqueued < 8 ? 4 : 8);
         k.ask = enqueued < KRYLOV_ASK;
         for (int q = 0; q < batch; ++q) launch_krylov_iteration(s, c->g, c->c, b, k);
         LAUNCHCHK();

@@ -57,8 +57,8 @@ struct KrylovPtrs {
 // Of the iterations enqueued together up to seven follow the stop.  One of them costs 7
 // (118x71x91) to 32 (257x129x129) and 135 us (385x193x193) more where its updates do not
 // ask, an iteration that runs 0.4 to 1.3 us more where they do: the costs are even at
-// 50 to 350 iterations a solve.  Solves of 1 iteration, not asking and asking:
-// 257x129x129 660 and 427 us, 385x193x193 2020 and 1095.
+// 50 to 350 iterations a solve.  A solve of 1 iteration at 385x193x193, not asking and
+// asking: 1337 and 910 us.
 constexpr int KRYLOV_ASK = 64;
 
 // dot modes of the operator kernel

@@ -1,5 +1,5 @@
 """Iterations of BiCGstab that are enqueued past the stop: solves that end at every
-place of the eight enqueued together, before and after the updates change the way
+place of the four or eight enqueued together, before and after the updates change the way
 they learn of it (64 iterations), against the oracle bit for bit; and what a stopped
 iteration costs, against one that runs."""
 import time
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 W6, PZ = (1,) * 6, (1, 1, 1, 1, -1, -1)
 
 
-@pytest.mark.parametrize("its", [1, 2, 7, 8, 9, 63, 64, 65, 71, 73])
+@pytest.mark.parametrize("its", [1, 2, 4, 5, 7, 8, 9, 63, 64, 65, 71, 73])
 @pytest.mark.parametrize("sweeps", [0, 3])
 def test_solves_that_stop(its, sweeps):
     N = (34, 19, 37)
@@ -36,9 +36,9 @@ def test_solves_that_stop(its, sweeps):
 
 
 def test_a_stopped_iteration_moves_nothing():
-    """A solve of one iteration enqueues eight.  The updates of one that runs are two
-    fifths of it; if the stopped ones moved as much, the solve of one would take over
-    two fifths of the solve of eight (0.42 measured so), and takes 0.23 if not."""
+    """A solve of one iteration enqueues four.  The updates are two fifths of one that
+    runs; if the stopped ones moved as much, the solve of one would take 0.28 of the
+    solve of eight, and takes 0.19 if not."""
     N = (385, 193, 193)
     gc = ih.Case(N, W6, (2.0, 1.0, 1.0))
     gc.upload(ih.RES, np.random.default_rng(17).standard_normal(gc.shape))
@@ -50,5 +50,5 @@ def test_a_stopped_iteration_moves_nothing():
             t = time.perf_counter()
             gc.bicgstab(0.0, its, (1, 1, 1), N)
             best[its] = min(best[its], time.perf_counter() - t)
-    assert best[1] < 0.33 * best[8], best
+    assert best[1] < 0.25 * best[8], best
     gc.close()

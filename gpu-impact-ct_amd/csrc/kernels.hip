@@ -1001,31 +1001,42 @@ __device__ inline void jor_vec_block(const Geo &g, const Range3 &r, const JorVec
     }
 }
 
-template <typename T, typename TO, int TPB, int PXM>
-__global__ __launch_bounds__(TPB) void k_jor_vec(Geo g, Coef c, Range3 r, JorVecShape sh, int nbw, int nbz,
+// The tables of a sweep, as the single sweeps take them (in the whole Coef their arguments
+// are five lines longer).
+template <typename T>
+struct SweepCoef {
+    const T *dg[3];
+};
+template <typename T>
+inline SweepCoef<T> sweep_coef(const Coef &c) {
+    if constexpr (sizeof(T) == 8)
+        return SweepCoef<T>{{c.dg[0], c.dg[1], c.dg[2]}};
+    else
+        return SweepCoef<T>{{c.dgf[0], c.dgf[1], c.dgf[2]}};
+}
+
+template <typename T, typename TO, int TPB, int PXM, bool WARM>
+__global__ __launch_bounds__(TPB) void k_jor_vec(Geo g, SweepCoef<T> c, Range3 r, JorVecShape sh, int nbw, int nbz,
                                                          T omega, const T *__restrict__ rel, const T *__restrict__ bb,
                                                          TO *__restrict__ out, const int *active) {
-    warm_args<Geo, Coef, Range3, JorVecShape, int, int, T, const T *, const T *, TO *, const int *>();
+    if constexpr (WARM)
+        warm_args<Geo, SweepCoef<T>, Range3, JorVecShape, int, int, T, const T *, const T *, TO *, const int *>();
     if (active && !*active) return;
     int tw, dummy, bz;
     if (!xcd_tile(nbw, 1, nbz, tw, dummy, bz)) return;
-    const T *g1 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[0] : (const void *)c.dgf[0]);
-    const T *g2 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[1] : (const void *)c.dgf[1]);
-    const T *g3 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[2] : (const void *)c.dgf[2]);
-    jor_vec_block<T, TO, TPB, PXM, const T *, TO *>(g, r, sh, tw, bz, nbz, omega, rel, bb, out, g1, g2, g3);
+    jor_vec_block<T, TO, TPB, PXM, const T *, TO *>(g, r, sh, tw, bz, nbz, omega, rel, bb, out, c.dg[0], c.dg[1],
+                                                   c.dg[2]);
 }
 
 template <typename T, int TPB, int PXM>
-__global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, Coef c, Range3 r, JorVecShape sh, int nbw, int nbz,
+__global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, SweepCoef<T> c, Range3 r, JorVecShape sh, int nbw, int nbz,
                                                  const T *__restrict__ x, T *__restrict__ lap, const int *active) {
-    warm_args<Geo, Coef, Range3, JorVecShape, int, int, const T *, T *, const int *>();
+    warm_args<Geo, SweepCoef<T>, Range3, JorVecShape, int, int, const T *, T *, const int *>();
     if (active && !*active) return;
     int tw, dummy, bz;
     if (!xcd_tile(nbw, 1, nbz, tw, dummy, bz)) return;
-    const T *g1 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[0] : (const void *)c.dgf[0]);
-    const T *g2 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[1] : (const void *)c.dgf[1]);
-    const T *g3 = (const T *)(sizeof(T) == 8 ? (const void *)c.dg[2] : (const void *)c.dgf[2]);
-    jor_vec_block<T, T, TPB, PXM, const T *, T *, true>(g, r, sh, tw, bz, nbz, T(0), x, x, lap, g1, g2, g3);
+    jor_vec_block<T, T, TPB, PXM, const T *, T *, true>(g, r, sh, tw, bz, nbz, T(0), x, x, lap, c.dg[0], c.dg[1],
+                                                       c.dg[2]);
 }
 
 // Two sweeps in one launch: out = sweep(sweep(rel)), each value formed with the
@@ -1920,9 +1931,19 @@ static void launch_jor_vec(hipStream_t s, const Geo &g, const Coef &c, const Box
     int nbw, nbz;
     const JorVecShape sh = jor_vec_shape(g, r, 16 / (int)sizeof(T), tpb, shape.kc, nbw, nbz);
     const dim3 grid(xcd_grid((int64_t)nbw * nbz));
-#define IH_JV(TPBV, PXV)                                                                                        \
-    hipLaunchKernelGGL((k_jor_vec<T, TO, TPBV, PXV>), grid, dim3(TPBV), 0, s, g, c, r, sh, nbw, nbz, omega, rel, bb, \
-                       out, active)
+    // warm arguments, without / with: FP64 65^3 4.3 / 3.8 us, 97^3 5.8 / 5.8, 129x129x65 6.7 / 6.9,
+    // 900x129x129 82 / 86; FP32 65^3 4.3 / 3.8, 97^3 5.9 / 5.6, 600x129x129 19.5 / 20.0, 900x129x129 27.6 / 26.9
+    const bool warm = sizeof(T) == 4 || (int64_t)r.n0 * r.n1 * r.n2 <= (1 << 19);
+#define IH_JVW(TPBV, PXV, WARM)                                                                                     \
+    hipLaunchKernelGGL((k_jor_vec<T, TO, TPBV, PXV, WARM>), grid, dim3(TPBV), 0, s, g, sweep_coef<T>(c), r, sh, nbw, \
+                       nbz, omega, rel, bb, out, active)
+#define IH_JV(TPBV, PXV)                                                                                            \
+    do {                                                                                                            \
+        if (warm)                                                                                                   \
+            IH_JVW(TPBV, PXV, true);                                                                                \
+        else if constexpr (sizeof(T) == 8)                                                                          \
+            IH_JVW(TPBV, PXV, false);                                                                               \
+    } while (0)
     const bool px = g.per[0] != 0;
     if (tpb == 128) {
         if (px) IH_JV(128, 1); else IH_JV(128, 0);
@@ -1932,6 +1953,7 @@ static void launch_jor_vec(hipStream_t s, const Geo &g, const Coef &c, const Box
         if (px) IH_JV(256, 1); else IH_JV(256, 0);
     }
 #undef IH_JV
+#undef IH_JVW
 }
 
 void launch_jor(hipStream_t s, const Geo &g, const Coef &c, const Box &b, double omega, const double *rel,
@@ -2114,7 +2136,8 @@ static void launch_lap_vec(hipStream_t s, const Geo &g, const Coef &c, const Box
     const JorVecShape sh = jor_vec_shape(g, r, 16 / (int)sizeof(T), tpb, shape.kc, nbw, nbz);
     const dim3 grid(xcd_grid((int64_t)nbw * nbz));
 #define IH_LV(TPBV, PXV)                                                                                        \
-    hipLaunchKernelGGL((k_lap_vec<T, TPBV, PXV>), grid, dim3(TPBV), 0, s, g, c, r, sh, nbw, nbz, x, lap, active)
+    hipLaunchKernelGGL((k_lap_vec<T, TPBV, PXV>), grid, dim3(TPBV), 0, s, g, sweep_coef<T>(c), r, sh, nbw, nbz, x, lap, \
+                       active)
     const bool px = g.per[0] != 0;
     if (tpb == 128) {
         if (px) IH_LV(128, 1); else IH_LV(128, 0);

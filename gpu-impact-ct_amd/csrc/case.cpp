@@ -702,6 +702,12 @@ int64_t ih_field_elems(const ih_case *c) {
 
 int64_t ih_case_bytes(const ih_case *c) { return c ? c->bytes : 0; }
 
+constexpr int64_t STAGE_BYTES = 4 << 20;  // a row is at most 64 KiB
+// rows of the case's transfer buffer (N: points of the grid)
+static int64_t stage_rows(const int *N) {
+    return std::min<int64_t>((int64_t)(N[1] + 7) * (N[2] + 7), STAGE_BYTES / (8 * (int64_t)(N[0] + 7)));
+}
+
 int64_t ih_grid_bytes(const ih_grid_desc *gd) {
     if (!gd) return 0;
     for (int d = 0; d < 3; ++d)
@@ -713,7 +719,8 @@ int64_t ih_grid_bytes(const ih_grid_desc *gd) {
     for (int d = 0; d < 3; ++d) tables += (int64_t)(((gd->N[d] + 1) + 7) / 8 * 8) * 80 * 12 + 2 * (gd->N[d] + 7) * 8;
     const int64_t parts = 2 * 8 * std::max<int64_t>(4096, ((gd->N[0] + 15) / 16) * ((gd->N[1] + 15) / 16) *
                                                              ((gd->N[2] + 31) / 32));
-    return IH_NFIELDS * 8 * fe + 3 * 4 * fe + 3 * fe + tables + parts + (1 << 20);
+    const int64_t stage = 8 * (int64_t)(gd->N[0] + 7) * stage_rows(gd->N);
+    return IH_NFIELDS * 8 * fe + 3 * 4 * fe + 3 * fe + tables + parts + stage + (1 << 20);
 }
 
 int64_t ih_grid_bytes_step(const ih_grid_desc *gd, const ih_step_params *p) {
@@ -726,8 +733,6 @@ int64_t ih_grid_bytes_step(const ih_grid_desc *gd, const ih_step_params *p) {
     host_mg_levels(hg, 15, mgh);
     return base + mg_alloc_bytes(mgh);
 }
-
-constexpr int64_t STAGE_BYTES = 4 << 20;  // a row is at most 64 KiB
 
 // A whole field between the device and a dense host array.  From and to memory that
 // the runtime does not know (not pinned) its copy goes row by row at 4 to 9
@@ -747,7 +752,7 @@ static int field_transfer(ih_case *c, ih_field f, double *host, bool to_device) 
     const int64_t rows = (int64_t)(g.N[1] + 7) * (g.N[2] + 7);
     const size_t w = sizeof(double) * (size_t)n, pitch = sizeof(double) * (size_t)g.px;
     double *const field = c->fields[f] + g.lead;
-    const int64_t step = std::min<int64_t>(rows, STAGE_BYTES / (int64_t)w);
+    const int64_t step = stage_rows(g.N);
     hipPointerAttribute_t at{};
     const bool known = hipPointerGetAttributes(&at, host) == hipSuccess && at.type != hipMemoryTypeUnregistered;
     (void)hipGetLastError();  // an unknown pointer may be reported as an error

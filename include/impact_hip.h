@@ -451,7 +451,8 @@ typedef struct {
     double admit_wait_mean_s;
 } ih_serve_summary;
 
-/* HBM a case of grid g holds (fields, FP32 buffers, mask, tables). */
+/* HBM a case of grid g holds (fields, FP32 buffers, mask, tables, and the buffer of at
+ * most 4 MiB that its first transfer of a host array that is not pinned allocates). */
 int64_t ih_grid_bytes(const ih_grid_desc *g);
 /* The same for a case that runs steps with p: the multigrid levels and their
  * FP32 copies are added when p selects preconditioner 1. */

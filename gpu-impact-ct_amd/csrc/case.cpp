@@ -754,8 +754,10 @@ static int field_transfer(ih_case *c, ih_field f, double *host, bool to_device) 
     double *const field = c->fields[f] + g.lead;
     const int64_t step = stage_rows(g.N);
     hipPointerAttribute_t at{};
-    const bool known = hipPointerGetAttributes(&at, host) == hipSuccess && at.type != hipMemoryTypeUnregistered;
-    (void)hipGetLastError();  // an unknown pointer may be reported as an error
+    // an error that the caller has yet to look at stays: one of this call's own is taken back
+    const hipError_t asked = hipPointerGetAttributes(&at, host);
+    if (asked != hipSuccess) (void)hipGetLastError();
+    const bool known = asked == hipSuccess && at.type != hipMemoryTypeUnregistered;
     if (!known && !c->stage) {
         if (hipMalloc(&c->stage, w * (size_t)step) == hipSuccess) {
             c->bytes += (int64_t)w * step;
@@ -775,12 +777,11 @@ static int field_transfer(ih_case *c, ih_field f, double *host, bool to_device) 
         const int64_t m = std::min(step, rows - r);
         if (to_device) {
             HIPCHK(hipMemcpyAsync(c->stage, host + r * n, w * (size_t)m, hipMemcpyHostToDevice, c->stream));
-            launch_rows_in(c->stream, c->stage, field + r * g.px, n, g.px, m);
+            HIPCHK(launch_rows_in(c->stream, c->stage, field + r * g.px, n, g.px, m));
         } else {
-            launch_rows_out(c->stream, field + r * g.px, c->stage, n, g.px, m);
+            HIPCHK(launch_rows_out(c->stream, field + r * g.px, c->stage, n, g.px, m));
             HIPCHK(hipMemcpyAsync(host + r * n, c->stage, w * (size_t)m, hipMemcpyDeviceToHost, c->stream));
         }
-        LAUNCHCHK();
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     (to_device ? c->n_up : c->n_down) += 1;

@@ -130,9 +130,10 @@ void launch_pack_box(hipStream_t s, const Geo &g, const int lo[3], const int n[3
                      const double *field, double *dense);
 void launch_unpack_box(hipStream_t s, const Geo &g, const int lo[3], const int n[3], const int st[3],
                        const double *dense, double *field);
-// nrows rows of n values, from and to a dense array
-void launch_rows_in(hipStream_t s, const double *dense, double *rows, int n, int px, int64_t nrows);
-void launch_rows_out(hipStream_t s, const double *rows, double *dense, int n, int px, int64_t nrows);
+// nrows rows of n values, from and to a dense array; returns the launch's own error (the
+// thread's last error may be another call's)
+hipError_t launch_rows_in(hipStream_t s, const double *dense, double *rows, int n, int px, int64_t nrows);
+hipError_t launch_rows_out(hipStream_t s, const double *rows, double *dense, int n, int px, int64_t nrows);
 void launch_axpby(hipStream_t s, const Geo &g, double a, double b, const double *x, const double *y, double *z,
                   int64_t n);
 void launch_fill(hipStream_t s, double *f, double v, int64_t n);

@@ -2411,14 +2411,19 @@ void launch_unpack_box(hipStream_t s, const Geo &g, const int lo[3], const int n
     hipLaunchKernelGGL(k_unpack_box, grid, dim3(BX, BY, 1), 0, s, g, pack_box(lo, n, st), dense, field);
 }
 
-void launch_rows_in(hipStream_t s, const double *dense, double *rows, int n, int px, int64_t nrows) {
-    const int64_t cnt = nrows * n;
-    hipLaunchKernelGGL(k_rows<true>, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, dense, rows, n, px, cnt);
+static hipError_t launch_rows(const void *kernel, hipStream_t s, const double *src, double *dst, int n, int px,
+                              int64_t nrows) {
+    int64_t cnt = nrows * n;
+    void *args[] = {&src, &dst, &n, &px, &cnt};
+    return hipLaunchKernel(kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), args, 0, s);
 }
 
-void launch_rows_out(hipStream_t s, const double *rows, double *dense, int n, int px, int64_t nrows) {
-    const int64_t cnt = nrows * n;
-    hipLaunchKernelGGL(k_rows<false>, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, rows, dense, n, px, cnt);
+hipError_t launch_rows_in(hipStream_t s, const double *dense, double *rows, int n, int px, int64_t nrows) {
+    return launch_rows((const void *)k_rows<true>, s, dense, rows, n, px, nrows);
+}
+
+hipError_t launch_rows_out(hipStream_t s, const double *rows, double *dense, int n, int px, int64_t nrows) {
+    return launch_rows((const void *)k_rows<false>, s, rows, dense, n, px, nrows);
 }
 
 void launch_fill_f32(hipStream_t s, float *f, float v, int64_t n, const int *active) {

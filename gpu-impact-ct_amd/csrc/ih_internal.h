@@ -56,6 +56,9 @@ struct Coef {
 
 constexpr int COEF6_LEAD = 8, COEF6_TAIL = 40;
 
+// compute units of the current device (256 on a whole MI355X, fewer on a partition)
+int compute_units();
+
 // Reduction tree constants, shared with the oracle's restatement: blocks of
 // RED_TX x RED_TY threads over (i, j); along k the range is cut into
 // ceil(n / RED_KC) chunks of balanced length (chunk b holds the planes

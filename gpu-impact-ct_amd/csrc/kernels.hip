@@ -1767,12 +1767,26 @@ void launch_interp_vel_pre(hipStream_t s, const Geo &g, const Coef &c, int q, co
     hipLaunchKernelGGL(k_interp_vel_pre, grid_for(r), dim3(BX, BY, 1), 0, s, g, c, r, q, phi, inter);
 }
 
+int compute_units() {
+    // looked up once per device; concurrent first calls store the same value
+    static std::atomic<int> cus[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+    if (!cus[dev].load()) {
+        int n = 0;
+        cus[dev].store(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256);
+    }
+    return cus[dev].load();
+}
+
 // At most eight wavefronts a compute unit at one plane each: measured at 1984 (129x33x33)
 // and 2256 (65x49x49), microseconds with one plane / several:
 //   interp_pre_vel along x 3.2 / 3.2 and 3.5 / 3.3, nonlinear_one along x 3.8 / 4.0 and
 // 4.5 / 4.0, along z 3.8 / 3.9 and 4.0 / 4.0, helmholtz_one 4.4 / 5.4 and 5.2 / 5.5
 // (3120 waves: 5.8 / 5.6).
-static bool few_waves(const Range3 &r) { return (int64_t)((r.n0 + BX - 1) / BX) * r.n1 * r.n2 <= 2048; }
+static bool few_waves(const Range3 &r) {
+    return (int64_t)((r.n0 + BX - 1) / BX) * r.n1 * r.n2 <= 8 * (int64_t)compute_units();
+}
 
 void launch_interp_pre_vel(hipStream_t s, const Geo &g, const Coef &c, int q, const double *phi, double *inter) {
     Range3 r = R(ibox(g, q));
@@ -1788,15 +1802,7 @@ void launch_interp_pre_vel(hipStream_t s, const Geo &g, const Coef &c, int q, co
 // (the kernel is latency-bound, and a second, partial round measured slowest),
 // down to chunks of 8 planes
 static int nlh_chunks(int q, int columns, int n2) {
-    // looked up once (per kernel, per device); concurrent first calls store the same value
-    static std::atomic<int> per_cu[3] = {};
-    static std::atomic<int> cus[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (!cus[dev].load()) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) cus[dev].store(n);
-    }
+    static std::atomic<int> per_cu[3] = {};  // looked up once
     if (!per_cu[q].load()) {
         const void *fn = q == 0 ? (const void *)k_nl_helm_rhs_t<0>
                                 : (q == 1 ? (const void *)k_nl_helm_rhs_t<1> : (const void *)k_nl_helm_rhs_t<2>);
@@ -1804,8 +1810,8 @@ static int nlh_chunks(int q, int columns, int n2) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, nlh::NT, 0) == hipSuccess) per_cu[q].store(n);
     }
     // chunks of at least 8 planes: shorter ones pay the 7-plane queue prologue on little work
-    const int least = (n2 + nlh::AZ - 1) / nlh::AZ, most = (n2 + 7) / 8, nc = cus[dev].load(), pc = per_cu[q].load();
-    if (columns <= 0 || nc <= 0 || pc <= 0) return least;
+    const int least = (n2 + nlh::AZ - 1) / nlh::AZ, most = (n2 + 7) / 8, nc = compute_units(), pc = per_cu[q].load();
+    if (columns <= 0 || pc <= 0) return least;
     return std::max(least, std::min(most, pc * nc / columns));
 }
 
@@ -1991,6 +1997,7 @@ template <typename F>
 static PairShape pair_shape(int n, int max_planes, F box) {
     PairShape best;
     double best_time = 0.0;
+    const double cus = compute_units();
     for (int tpb : {256, 512, 1024}) {
         bool fits = true;
         for (int q = 0; q < n; ++q) fits = fits && 4 * (box(q).sh.nent + 1) <= tpb;
@@ -2004,7 +2011,7 @@ static PairShape pair_shape(int n, int max_planes, F box) {
                 largest = std::max(largest, b);
             }
             auto time = [&](int64_t b) {
-                const double load = std::ceil((double)b / 256.0);  // on the most loaded compute unit
+                const double load = std::ceil((double)b / cus);  // on the most loaded compute unit
                 const double resident = std::min(load, 1024.0 / tpb);
                 const double plane = std::max(1200.0, resident * tpb / 256.0 * 1000.0);
                 return load / resident * (6000.0 + (kc + 2) * plane);

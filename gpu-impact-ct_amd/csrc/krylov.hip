@@ -115,7 +115,7 @@ enum { DOT_NONE = 0, DOT_W = 1, DOT_SELF = 2, DOT_PAIR = 3 };
 // Measured and not taken: segments of four points a thread in each direction in
 // turn with all coefficients scalar (9/4 gradients a point, bound by VALU: 48 us
 // at 257x129x129 against 45); the teams at 80 VGPRs for three blocks (spills).
-constexpr int64_t APPLY_TEAM_TILES = 512;
+static int64_t apply_team_tiles() { return 2 * (int64_t)compute_units(); }
 constexpr int APPLY_THREADS = 2 * RED_TX * RED_TY;
 
 // Keeps the compiler to the order written: nothing moves across.
@@ -1287,7 +1287,7 @@ __global__ __launch_bounds__(UPD_ZG * RED_THREADS) void k_dots(Geo g, Range3 r, 
 // without: 118x71x91 (120 tiles) 78.1 / 82 us, 193x97x97 (364, the second round 42 %
 // full) 105.3 / 104.7, 257x129x129 (765) 175.1 / 175.1, 385x193x193 (2275) 584 / 589.
 static bool x_split(int64_t tiles) {
-    const int64_t cus = 256, rounds = (tiles + cus - 1) / cus;
+    const int64_t cus = compute_units(), rounds = (tiles + cus - 1) / cus;
     return rounds <= 1 || 8 * tiles >= 7 * rounds * cus;
 }
 
@@ -1548,7 +1548,7 @@ static inline Range3 Rk(const Box &b) { return make_range(b); }
 //   129x65x65    17.6 / 11.4   65.5 / 61.2     193x97x97   28.9 / 27.1   (not taken)
 // hence at least APPLY_SPLIT times the reduction's chunks (97^3 has 10 for 4).
 static int apply_split(int columns, int planes) {
-    return (int)std::min<int64_t>((planes + 2) / 3, APPLY_TEAM_TILES / columns);
+    return (int)std::min<int64_t>((planes + 2) / 3, apply_team_tiles() / columns);
 }
 constexpr int APPLY_SPLIT = 3;
 
@@ -1576,7 +1576,7 @@ void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, c
                                dot_mode == DOT_SELF ? src : w, part1, part2, active);
         return;
     }
-    const bool teams = tiles <= APPLY_TEAM_TILES;
+    const bool teams = tiles <= apply_team_tiles();
     const dim3 grid(xcd_grid(tiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
 #define IH_APPLY_AS(T, DMV, PZV)                                                                               \
     hipLaunchKernelGGL((k_apply<T, DMV, PZV>), grid, block, 0, s, g, c, r, nbx, nby, nbz, src, dst, w, part1, part2, \
@@ -1743,7 +1743,7 @@ void launch_krylov_part(hipStream_t s, const Geo &g, const Coef &c, const Box &b
 void launch_apply_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, int form, bool pre,
                         bool any_pz, bool any_nonpz) {
     if (ntiles <= 0) return;
-    const bool teams = ntiles <= APPLY_TEAM_TILES;
+    const bool teams = ntiles <= apply_team_tiles();
     const dim3 grid(xcd_grid(ntiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
 #define IH_APB_AS(T, DMV, PZV)                                                                                    \
     hipLaunchKernelGGL((k_apply_batch<T, DMV, PZV>), grid, block, 0, s, cases, tile_case, ntiles, form, (int)pre)

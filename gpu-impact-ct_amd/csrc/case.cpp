@@ -1252,8 +1252,7 @@ static void mg_free(ih_case *c) { drop_mg(c); }
 
 // Device bytes mg_setup allocates for the levels of mgh: the FP64 level arrays
 // (2 fields on level 1, 4 below), the FP64 tables (cdg, cR: 3 taps, cI: 2 taps
-// per direction) and 64 zeros, the FP32 arrays (4 per level) and tables, and
-// the two descriptor arrays.
+// per direction) and 64 zeros, the FP32 arrays (4 per level) and tables.
 static int64_t mg_alloc_bytes(const std::vector<HostMgLevel> &mgh) {
     const int G = (int)mgh.size();
     int64_t arr = 0, tab = 0, arr32 = 0;

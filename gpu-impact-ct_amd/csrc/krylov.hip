@@ -62,7 +62,7 @@ __device__ inline bool g_src(const Geo &g, int d, int &idx) {
 
 __device__ inline bool wall_plane(const Geo &g, int e, int idx) { return !g.per[e] && (idx == 1 || idx == g.N[e]); }
 
-// p_src, g_src and wall_plane along z with the periodicity of z a compile-time
+// p_src and wall_plane along z with the periodicity of z a compile-time
 // constant: the plane loop of k_apply then has no branches on it (they cost
 // scalar instructions and branch joins every plane)
 template <bool PZ>
@@ -72,14 +72,6 @@ __device__ inline bool p_src_z(const Geo &g, int &idx) {
         return true;
     }
     return idx >= 1 && idx <= g.N[2];
-}
-template <bool PZ>
-__device__ inline bool g_src_z(const Geo &g, int &idx) {
-    if (PZ) {
-        idx = wrap_p(g, 2, idx);
-        return true;
-    }
-    return idx >= 1 && idx <= g.N[2] - 1;
 }
 template <bool PZ>
 __device__ inline bool wall_z(const Geo &g, int idx) {
@@ -1539,7 +1531,8 @@ __global__ void k_gather_batch(const KBatchCase *__restrict__ cases, int ncases,
 static inline Range3 Rk(const Box &b) { return make_range(b); }
 
 // z chunks of an operator that leaves its dot products to k_dots: as many as fill the
-// device with two blocks of teams a compute unit, of three planes or more.  A block
+// device with two blocks of teams a compute unit, of about three planes (balanced: where
+// the planes limit their number some have two).  A block
 // marches its chunk and six planes more at 0.6 us a plane, so a grid of few columns is
 // bound by the 32 planes of the reduction's chunk; k_dots costs 3.5 to 5 us.  Operator
 // fused / split without k_dots, a BiCGstab iteration fused / split, microseconds:

@@ -137,6 +137,16 @@ def stencil_table(ih, grid, launches=20):
     return out
 
 
+def sweeps_per_launch(ih, c, pair):
+    """2 where the case takes two JOR sweeps a launch (`pair` names that kernel's
+    benchmark entry, which the library refuses elsewhere), else 1."""
+    try:
+        c.bench_kernel(pair, 1)
+    except ih.IHError:
+        return 1
+    return 2
+
+
 def operator_roofline(table, grid, traffic=None):
     """roofline of the fused Poisson operator k_apply in the two forms a BiCGstab
     iteration launches (Ap with <rh, Ap>: 24 B/point; As with <s, As>, <As, As>:
@@ -650,9 +660,10 @@ def main():
     bi_ms, bi_n = fams["bicgstab"]
     P = N[0] * N[1] * N[2]
     jor_bytes = JOR_BYTES_PER_POINT * P
-    jor_avg_ms = 2 * jor_ms / max(jor_n, 1)  # a launch is two sweeps and moves what one would
+    per = sweeps_per_launch(ih, c, "jor_pair")
+    jor_avg_ms = per * jor_ms / max(jor_n, 1)  # two sweeps in a launch move what one would
     achieved = jor_bytes / (jor_avg_ms * 1e-3) / 1e9
-    traffic = read_traffic("jor_pair_257x129x129_counters.txt")
+    traffic = read_traffic("jor_pair_257x129x129_counters.txt" if per == 2 else "jor_sweep_256x128x128_counters.txt")
     log("kernel table ...")
     table = kernel_table(ih, N)
     log("stencil table ...")
@@ -681,7 +692,7 @@ def main():
         },
         "roofline": operator_roofline(table, N, read_traffic("poisson_operator_256x128x128_counters.txt")),
         "roofline_jor": {
-            "kernel": "k_jor_pair<double, double> (two sweeps a launch)",
+            "kernel": "k_jor_pair<double, double> (two sweeps a launch)" if per == 2 else "k_jor_vec<double, double>",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
@@ -718,6 +729,7 @@ def main():
         ms_m, fams_m, iters_m, _ = run_steps(ih, cm, pm, args.steps, args.warmup, "mixed")
         err = rel_errors(ih, cm, c)  # both cases advanced warmup + steps + 1 steps from the same state
         f32_ms, f32_n = fams_m["jor_f32"]
+        f32_launch_ms = sweeps_per_launch(ih, cm, "jor_pair_f32") * f32_ms / max(f32_n, 1)
         result["mixed_precision"] = {
             "form": (f"{JOR_SWEEPS} FP32 JOR sweeps as defect correction, then BiCGstab right-preconditioned by "
                      f"{args.precond_sweeps} FP32 JOR sweeps; residuals, inner products and updates FP64"),
@@ -725,8 +737,8 @@ def main():
             "ms_per_step": ms_m,
             "speedup_vs_fp64": ms_per_step / ms_m,
             "bicgstab_iterations_per_step": iters_m,
-            "jor_f32_avg_launch_ms": 2 * f32_ms / max(f32_n, 1),  # two sweeps a launch
-            "jor_f32_achieved_GBs": JOR32_BYTES_PER_POINT * P / (2 * f32_ms / max(f32_n, 1) * 1e-3) / 1e9,
+            "jor_f32_avg_launch_ms": f32_launch_ms,
+            "jor_f32_achieved_GBs": JOR32_BYTES_PER_POINT * P / (f32_launch_ms * 1e-3) / 1e9,
             "steps_compared": args.warmup + args.steps + 1,
             **{f"{k}_vs_fp64": v for k, v in err.items()},
         }

@@ -2095,18 +2095,20 @@ bool jor_pair_fits(const Geo &g, const Coef &c, const Box &b, bool fp32) {
 // Two single sweeps / a pair, microseconds:
 //   FP64 (share)         17x17       65x65       129x129     257x129
 //     270 points (.73)   6.4 / 7.9   13.9 / 12.9  35.0 / 27.2  65.7 / 46.6
-//     420        (.58)   6.7 / 7.9   18.0 / 17.8  51.8 / 46.3   162 / 97
+//     420        (.58)   6.7 / 7.9   18.0 / 17.8  51.8 / 46.3   162 / 97     (a V cycle of eight sweeps at
+//                        426x199x53, share .577: 355 with single sweeps, 333 with pairs)
 //     505        (.50)   6.8 / 7.8   20.7 / 20.9  61.1 / 63.2   198 / 101
 //   FP32
 //     505 points (.75)   7.1 / 9.8   14.8 / 14.6  35.2 / 32.3  63.6 / 59.5
 //     640        (.68)   6.9 / 9.8   17.6 / 18.4  41.7 / 41.4   112 / 74
 //     1000       (.50)   8.0 / 10.1  23.3 / 26.9  61.2 / 73.4   180 / 137
-// (33 x 33 rows lose at every long row, 33 x 129 ones, 24 MB and up, are even.)
+// Between them a long row breaks even at about 24 MB: a ratio of 0.75 to 0.95 up to 11 MB
+// (33x33), of 0.87 to 1.08 to 24 MB, of 0.95 to 1.16 beyond.
 // A row of 480 points in FP32 takes 9.0 / 9.1, 14.4 / 14.9, 34.1 / 31.7 and 56.9 / 54.7,
 // at worst (33x129) 14.4 / 17.0.
 static bool pair_pays(bool wide, double bytes, double share, bool fp32) {
     if (!wide || bytes >= 240e6) return true;
-    return bytes >= 24e6 && share >= (fp32 ? 0.70 : 0.58);
+    return bytes >= 24e6 && share >= (fp32 ? 0.70 : 0.57);
 }
 static bool pair_wide(const JorVecShape &sh) { return 4 * (sh.nent + 1) > 512; }
 static double pair_share(const JorVecShape &sh) { return 1.0 - 2.0 * (sh.nent + 1) / 1024.0; }

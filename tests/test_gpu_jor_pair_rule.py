@@ -24,7 +24,7 @@ def takes(c, name):
 @pytest.mark.parametrize("N,fp64,fp32", [
     ((249, 9, 9), True, True), ((251, 9, 9), False, True), ((499, 9, 9), False, True), ((501, 9, 9), False, False),
     ((270, 60, 61), False, True), ((270, 62, 61), True, True),          # 24 MB in FP64
-    ((424, 65, 65), True, True), ((425, 65, 65), False, True),          # the share in FP64
+    ((434, 65, 65), True, True), ((435, 65, 65), False, True),          # the share in FP64
     ((450, 149, 149), False, True), ((450, 150, 149), True, True),      # 240 MB in FP64
     ((505, 62, 62), False, False), ((505, 65, 62), False, True),        # 24 MB in FP32
     ((600, 65, 65), False, True), ((601, 65, 65), False, False),        # the share in FP32
@@ -37,7 +37,7 @@ def test_route(N, fp64, fp32):
     c.close()
 
 
-@pytest.mark.parametrize("N,bc", [((270, 62, 61), PY), ((424, 65, 65), W6), ((422, 70, 67), PX), ((505, 201, 101), PY),
+@pytest.mark.parametrize("N,bc", [((270, 62, 61), PY), ((434, 65, 65), W6), ((432, 70, 67), PX), ((505, 201, 101), PY),
                                   ((506, 150, 133), W6), ((505, 150, 135), PX)], ids=lambda v: "x".join(map(str, v)))
 def test_long_rows_fp64(N, bc):
     c = ih.Case(N, bc, (2.0, 1.0, 1.0))

@@ -443,6 +443,8 @@ int ih_case_create(const ih_grid_desc *gd, int device, ih_case **out) {
     Geo &g = c->g;
     for (int d = 0; d < 3; ++d) g.N[d] = gd->N[d];
     init_limits(g, gd->bc);
+    if (hipDeviceGetAttribute(&g.cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || g.cus <= 0)
+        g.cus = 256;
     g.lead = 12;  // puts i = 1 of every row on a 128-byte boundary
     g.px = ((g.N[0] + 7) + 15) / 16 * 16;
     g.pxy = (int64_t)g.px * (g.N[1] + 7);
@@ -1299,6 +1301,7 @@ static int mg_setup(ih_case *c) {
             for (int d = 0; d < 3; ++d) q.N[d] = c->mgh[g - 1].N[d];
             init_limits(q, bc6);
             q.lead = 12;
+            q.cus = c->g.cus;
             q.px = ((q.N[0] + 7) + 15) / 16 * 16;
             q.pxy = (int64_t)q.px * (q.N[1] + 7);
             q.fe = ((q.lead + q.pxy * (q.N[2] + 7)) + 63) / 64 * 64;
@@ -3056,17 +3059,18 @@ void batch_iteration(ih_batch *b, int sweeps, float omega) {
     const bool pre = sweeps > 0;
     // two or more sweeps: the p and s updates also form M's first sweep
     const bool fuse = sweeps >= 2;
+    const int cus = b->cases[0]->g.cus;
     launch_p_update_batch(s, b->kcases, b->ktile, b->kntiles, fuse, omega);
     if (pre) batch_precond(b, 0, sweeps, omega, fuse);
-    launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_W, pre, b->k_pz, b->k_nonpz);
+    launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_W, pre, b->k_pz, b->k_nonpz, cus);
     launch_s_update_batch(s, b->kcases, b->ktile, b->kntiles, fuse, omega);
     if (pre) {
         batch_precond(b, 1, sweeps, omega, fuse);
-        launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_PAIR, pre, b->k_pz, b->k_nonpz);
+        launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_PAIR, pre, b->k_pz, b->k_nonpz, cus);
     } else {
-        launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_SELF, pre, b->k_pz, b->k_nonpz);
+        launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_SELF, pre, b->k_pz, b->k_nonpz, cus);
     }
-    launch_x_update_batch(s, b->kcases, b->ktile, b->kntiles, pre);
+    launch_x_update_batch(s, b->kcases, b->ktile, b->kntiles, pre, cus);
     launch_ctl_end_batch(s, b->kcases, (int)b->cases.size());
 }
 
@@ -3089,7 +3093,8 @@ int batch_bicgstab(ih_batch *b, const ih_step_params *p, int sweeps, std::vector
             if ((rc = exch(c, m, 0, F(c, IH_PRE)))) return rc;
     }
     // rr = A phi, then rr = bb - rr, rh = rr, eps = tol * max|bb| and the first head
-    launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_PHI, false, b->k_pz, b->k_nonpz);
+    launch_apply_batch(s, b->kcases, b->ktile, b->kntiles, KB_APPLY_PHI, false, b->k_pz, b->k_nonpz,
+                       b->cases[0]->g.cus);
     launch_krylov_init_batch(s, b->kcases, n, b->ktile, b->kntiles, p->bicg_rel_tol, p->bicg_max_it);
     LAUNCHCHK();
     // iterations enqueued per convergence check, replayed from a captured graph

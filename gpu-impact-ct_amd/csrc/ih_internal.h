@@ -17,6 +17,7 @@ struct Geo {
     int px;
     int64_t pxy;
     int lead;
+    int cus;             // compute units of the case's device (256 on a whole MI355X, fewer on a partition)
     int64_t fe;          // elements allocated per field (padded)
     int per[3];          // 1 if the direction is periodic
     int Sp[3], Np[3];    // pressure range
@@ -55,9 +56,6 @@ struct Coef {
 };
 
 constexpr int COEF6_LEAD = 8, COEF6_TAIL = 40;
-
-// compute units of the current device (256 on a whole MI355X, fewer on a partition)
-int compute_units();
 
 // Reduction tree constants, shared with the oracle's restatement: blocks of
 // RED_TX x RED_TY threads over (i, j); along k the range is cut into

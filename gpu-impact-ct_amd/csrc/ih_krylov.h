@@ -85,7 +85,7 @@ struct KBatchCase {
 // with <Ap, rh>, A rr -> Ar with <rr, Ar>, <Ar, Ar>, A z2 -> Ar with <rr, Ar>, <Ar, Ar>
 enum { KB_APPLY_PHI = 0, KB_APPLY_W = 1, KB_APPLY_SELF = 2, KB_APPLY_PAIR = 3 };
 void launch_apply_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, int form, bool pre,
-                        bool any_pz, bool any_nonpz);
+                        bool any_pz, bool any_nonpz, int cus);
 // rr = bb - rr (rr holding A phi), rh = rr, the max-norm/<rr, rh> partials, and
 // max|bb| partials in part3; then per case eps = tol * max|bb| and the iteration
 // head (k_ctl_setup's work)
@@ -99,7 +99,8 @@ void launch_p_update_batch(hipStream_t s, const KBatchCase *cases, const int *ti
                            float omega);
 void launch_s_update_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, bool first,
                            float omega);
-void launch_x_update_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, bool pre);
+void launch_x_update_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, bool pre,
+                           int cus);
 void launch_ctl_end_batch(hipStream_t s, const KBatchCase *cases, int ncases);
 // fl_out[q*KF_NSLOTS + s] = case q's flag s, sc_out[q*KS_NSLOTS + s] its scalar s
 void launch_gather_batch(hipStream_t s, const KBatchCase *cases, int ncases, int *fl_out, double *sc_out);

@@ -1767,31 +1767,19 @@ void launch_interp_vel_pre(hipStream_t s, const Geo &g, const Coef &c, int q, co
     hipLaunchKernelGGL(k_interp_vel_pre, grid_for(r), dim3(BX, BY, 1), 0, s, g, c, r, q, phi, inter);
 }
 
-int compute_units() {
-    // looked up once per device; concurrent first calls store the same value
-    static std::atomic<int> cus[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (!cus[dev].load()) {
-        int n = 0;
-        cus[dev].store(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256);
-    }
-    return cus[dev].load();
-}
-
 // At most eight wavefronts a compute unit at one plane each: measured at 1984 (129x33x33)
 // and 2256 (65x49x49), microseconds with one plane / several:
 //   interp_pre_vel along x 3.2 / 3.2 and 3.5 / 3.3, nonlinear_one along x 3.8 / 4.0 and
 // 4.5 / 4.0, along z 3.8 / 3.9 and 4.0 / 4.0, helmholtz_one 4.4 / 5.4 and 5.2 / 5.5
 // (3120 waves: 5.8 / 5.6).
-static bool few_waves(const Range3 &r) {
-    return (int64_t)((r.n0 + BX - 1) / BX) * r.n1 * r.n2 <= 8 * (int64_t)compute_units();
+static bool few_waves(const Geo &g, const Range3 &r) {
+    return (int64_t)((r.n0 + BX - 1) / BX) * r.n1 * r.n2 <= 8 * (int64_t)g.cus;
 }
 
 void launch_interp_pre_vel(hipStream_t s, const Geo &g, const Coef &c, int q, const double *phi, double *inter) {
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
-    const bool few = few_waves(r);
+    const bool few = few_waves(g, r);
     auto *const k = q == 0 ? (few ? k_interp_pre_vel<0, 1> : k_interp_pre_vel<0, 4>)
                            : (q == 1 ? k_interp_pre_vel<1, 1> : (few ? k_interp_pre_vel<2, 1> : k_interp_pre_vel<2, 4>));
     hipLaunchKernelGGL(k, grid_rows(r, few || q == 1 ? 1 : 4), dim3(BX, BY, 1), 0, s, g, c, r, phi, inter);
@@ -1801,7 +1789,7 @@ void launch_interp_pre_vel(hipStream_t s, const Geo &g, const Coef &c, int q, co
 // columns leave room, as many as fill exactly one round of resident blocks
 // (the kernel is latency-bound, and a second, partial round measured slowest),
 // down to chunks of 8 planes
-static int nlh_chunks(int q, int columns, int n2) {
+static int nlh_chunks(int q, int columns, int n2, int nc) {
     static std::atomic<int> per_cu[3] = {};  // looked up once
     if (!per_cu[q].load()) {
         const void *fn = q == 0 ? (const void *)k_nl_helm_rhs_t<0>
@@ -1810,7 +1798,7 @@ static int nlh_chunks(int q, int columns, int n2) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, nlh::NT, 0) == hipSuccess) per_cu[q].store(n);
     }
     // chunks of at least 8 planes: shorter ones pay the 7-plane queue prologue on little work
-    const int least = (n2 + nlh::AZ - 1) / nlh::AZ, most = (n2 + 7) / 8, nc = compute_units(), pc = per_cu[q].load();
+    const int least = (n2 + nlh::AZ - 1) / nlh::AZ, most = (n2 + 7) / 8, pc = per_cu[q].load();
     if (columns <= 0 || pc <= 0) return least;
     return std::max(least, std::min(most, pc * nc / columns));
 }
@@ -1821,7 +1809,7 @@ void launch_nl_helm_rhs(hipStream_t s, const Geo &g, const Coef &c, int q, const
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
     const int nbx = (r.n0 + nlh::TX - 1) / nlh::TX, nby = (r.n1 + nlh::TY - 1) / nlh::TY;
-    const int nbz = nlh_chunks(q, nbx * nby, r.n2);
+    const int nbz = nlh_chunks(q, nbx * nby, r.n2, g.cus);
     const dim3 grid(xcd_grid((int64_t)nbx * nby * nbz)), block(nlh::TX, nlh::TY, 1);
     if (q == 0)
         hipLaunchKernelGGL(k_nl_helm_rhs_t<0>, grid, block, 0, s, g, c, r, nbx, nby, nbz, w1, w2, w3, vel, nl, rhs,
@@ -1838,7 +1826,7 @@ void launch_nonlinear_one(hipStream_t s, const Geo &g, const Coef &c, int q, int
                           const double *vel, double *nl, int assign) {
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
-    const bool few = few_waves(r);
+    const bool few = few_waves(g, r);
     auto *const k = d == 0 ? (few ? k_nonlinear_one<0, 1> : k_nonlinear_one<0, 4>)
                            : (d == 1 ? k_nonlinear_one<1, 1> : (few ? k_nonlinear_one<2, 1> : k_nonlinear_one<2, 2>));
     hipLaunchKernelGGL(k, grid_rows(r, few || d == 1 ? 1 : (d == 0 ? 4 : 2)), dim3(BX, BY, 1), 0, s, g, c, r, q, pp,
@@ -1849,7 +1837,7 @@ void launch_helmholtz_one(hipStream_t s, const Geo &g, const Coef &c, int q, dou
                           double *nl) {
     Range3 r = R(ibox(g, q));
     if (empty(r)) return;
-    const bool few = few_waves(r);
+    const bool few = few_waves(g, r);
     hipLaunchKernelGGL(few ? k_helmholtz_one<1> : k_helmholtz_one<4>, grid_rows(r, few ? 1 : 4), dim3(BX, BY, 1), 0, s,
                        g, c, r, q, multL, vel, nl);
 }
@@ -1994,10 +1982,9 @@ void launch_jor_f32_to64(hipStream_t s, const Geo &g, const Coef &c, const Box &
 // 2366 ms as the iterations spread (2084 to 2266 with single sweeps), by the weighted
 // times below 1771 to 1972; of six tubes 338 and 329.
 template <typename F>
-static PairShape pair_shape(int n, int max_planes, F box) {
+static PairShape pair_shape(int n, int max_planes, double cus, F box) {
     PairShape best;
     double best_time = 0.0;
-    const double cus = compute_units();
     for (int tpb : {256, 512, 1024}) {
         bool fits = true;
         for (int q = 0; q < n; ++q) fits = fits && 4 * (box(q).sh.nent + 1) <= tpb;
@@ -2038,7 +2025,7 @@ static void launch_pair(hipStream_t s, const Geo &g, const Coef &c, const Box &b
                         TO *out, const int *active) {
     const Range3 r = R(b);
     const PairBox pb = pair_box(g, r, 16 / (int)sizeof(T));
-    const PairShape shape = pair_shape(1, r.n2, [&](int) { return pb; });
+    const PairShape shape = pair_shape(1, r.n2, g.cus, [&](int) { return pb; });
     const JorVecShape &sh = pb.sh;
     const int best_t = shape.tpb, best_nt = pb.tiles(best_t), best_nbz = (r.n2 + shape.kc - 1) / shape.kc;
     const dim3 grid(xcd_grid((int64_t)best_nt * best_nbz));
@@ -2269,7 +2256,7 @@ PairShape jor_pair_batch_shape(const std::vector<JorBatchItem> &items) {
     for (const JorBatchItem &it : items) planes = std::max(planes, it.r.n2);
     std::vector<PairBox> boxes;
     for (const JorBatchItem &it : items) boxes.push_back(pair_box(it.g, it.r, 4));
-    return pair_shape((int)items.size(), planes, [&](int q) -> const PairBox & { return boxes[(size_t)q]; });
+    return pair_shape((int)items.size(), planes, items[0].g.cus, [&](int q) -> const PairBox & { return boxes[(size_t)q]; });
 }
 
 int jor_pair_batch_tiles(PairShape shape, JorBatchItem &it) {

@@ -107,7 +107,7 @@ enum { DOT_NONE = 0, DOT_W = 1, DOT_SELF = 2, DOT_PAIR = 3 };
 // Measured and not taken: segments of four points a thread in each direction in
 // turn with all coefficients scalar (9/4 gradients a point, bound by VALU: 48 us
 // at 257x129x129 against 45); the teams at 80 VGPRs for three blocks (spills).
-static int64_t apply_team_tiles() { return 2 * (int64_t)compute_units(); }
+static int64_t apply_team_tiles(int cus) { return 2 * (int64_t)cus; }
 constexpr int APPLY_THREADS = 2 * RED_TX * RED_TY;
 
 // Keeps the compiler to the order written: nothing moves across.
@@ -1278,8 +1278,8 @@ __global__ __launch_bounds__(UPD_ZG * RED_THREADS) void k_dots(Geo g, Range3 r, 
 // the last round at most an eighth of all empty.  A BiCGstab iteration with it and
 // without: 118x71x91 (120 tiles) 78.1 / 82 us, 193x97x97 (364, the second round 42 %
 // full) 105.3 / 104.7, 257x129x129 (765) 175.1 / 175.1, 385x193x193 (2275) 584 / 589.
-static bool x_split(int64_t tiles) {
-    const int64_t cus = compute_units(), rounds = (tiles + cus - 1) / cus;
+static bool x_split(int64_t tiles, int64_t cus) {
+    const int64_t rounds = (tiles + cus - 1) / cus;
     return rounds <= 1 || 8 * tiles >= 7 * rounds * cus;
 }
 
@@ -1540,8 +1540,8 @@ static inline Range3 Rk(const Box &b) { return make_range(b); }
 //   65^3         17.3 /  9.2   61.1 / 54.8     97^3        20.0 / 15.9   (not taken)
 //   129x65x65    17.6 / 11.4   65.5 / 61.2     193x97x97   28.9 / 27.1   (not taken)
 // hence at least APPLY_SPLIT times the reduction's chunks (97^3 has 10 for 4).
-static int apply_split(int columns, int planes) {
-    return (int)std::min<int64_t>((planes + 2) / 3, apply_team_tiles() / columns);
+static int apply_split(int columns, int planes, int cus) {
+    return (int)std::min<int64_t>((planes + 2) / 3, apply_team_tiles(cus) / columns);
 }
 constexpr int APPLY_SPLIT = 3;
 
@@ -1552,7 +1552,7 @@ void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, c
     // the operator tile is the reduction tile, so the fused dot partials follow the fixed tree
     const int nbx = (r.n0 + RED_TX - 1) / RED_TX, nby = (r.n1 + RED_TY - 1) / RED_TY, nbz = (r.n2 + RED_KC - 1) / RED_KC;
     const int64_t tiles = (int64_t)nbx * nby * nbz;
-    const int nsplit = apply_split(nbx * nby, r.n2);
+    const int nsplit = apply_split(nbx * nby, r.n2, g.cus);
     if (nsplit >= APPLY_SPLIT * nbz) {
         const dim3 grid(xcd_grid((int64_t)nbx * nby * nsplit)), block(RED_TX, RED_TY, 2);
         if (g.per[2])
@@ -1569,7 +1569,7 @@ void launch_apply_A(hipStream_t s, const Geo &g, const Coef &c, const Box &pb, c
                                dot_mode == DOT_SELF ? src : w, part1, part2, active);
         return;
     }
-    const bool teams = tiles <= apply_team_tiles();
+    const bool teams = tiles <= apply_team_tiles(g.cus);
     const dim3 grid(xcd_grid(tiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
 #define IH_APPLY_AS(T, DMV, PZV)                                                                               \
     hipLaunchKernelGGL((k_apply<T, DMV, PZV>), grid, block, 0, s, g, c, r, nbx, nby, nbz, src, dst, w, part1, part2, \
@@ -1671,7 +1671,7 @@ static void launch_s_update(hipStream_t s, const Geo &g, const Range3 &r, int64_
 
 static void launch_x_update(hipStream_t s, const Geo &g, const Range3 &r, int64_t nb, const KrylovPtrs &k, bool pre) {
     const double *ra = pre ? k.z2 : k.rr, *pa = pre ? k.z1 : k.pk;
-    if (!x_split(nb)) {
+    if (!x_split(nb, g.cus)) {
         hipLaunchKernelGGL(k_x_update_omega, red_grid(r), dim3(RED_TX, RED_TY, 1), 0, s, g, r, k.phi, k.rr, ra, pa,
                            k.Ar, k.rh, k.part1, k.part2, nb, k.sc, k.fl, k.part3, k.part4);
         return;
@@ -1734,9 +1734,9 @@ void launch_krylov_part(hipStream_t s, const Geo &g, const Coef &c, const Box &b
 }
 
 void launch_apply_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, int form, bool pre,
-                        bool any_pz, bool any_nonpz) {
+                        bool any_pz, bool any_nonpz, int cus) {
     if (ntiles <= 0) return;
-    const bool teams = ntiles <= apply_team_tiles();
+    const bool teams = ntiles <= apply_team_tiles(cus);
     const dim3 grid(xcd_grid(ntiles)), block(RED_TX, RED_TY, teams ? 2 : 1);
 #define IH_APB_AS(T, DMV, PZV)                                                                                    \
     hipLaunchKernelGGL((k_apply_batch<T, DMV, PZV>), grid, block, 0, s, cases, tile_case, ntiles, form, (int)pre)
@@ -1793,9 +1793,10 @@ void launch_s_update_batch(hipStream_t s, const KBatchCase *cases, const int *ti
                            tile_case, ntiles, omega);
 }
 
-void launch_x_update_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, bool pre) {
+void launch_x_update_batch(hipStream_t s, const KBatchCase *cases, const int *tile_case, int ntiles, bool pre,
+                           int cus) {
     if (ntiles <= 0) return;
-    if (x_split(ntiles))
+    if (x_split(ntiles, cus))
         hipLaunchKernelGGL(k_x_update_batch<true>, dim3(xcd_grid(ntiles)), dim3(RED_TX, RED_TY, UPD_ZG), 0, s, cases,
                            tile_case, ntiles, (int)pre);
     else

@@ -1058,12 +1058,16 @@ __global__ __launch_bounds__(TPB) void k_lap_vec(Geo g, SweepCoef<T> c, Range3 r
 // Points outside the range enter the second sweep as zeros; their coefficients are
 // zero (the rule for taking this kernel checks it), as is what dead entries load.
 // A single sweep moves 24 (FP32: 12) bytes a point for 27 operations and runs at the
-// rate of the last-level cache or of the launches; a pair moves them once, and the
-// vector ALU bounds it (about 30 instructions a point and sweep, 13 of them the
-// IEEE division).  Measured, microseconds for two sweeps, two launches -> a pair:
+// rate of the last-level cache or of the launches; a pair moves them once.  The vector
+// ALU is then its busiest unit: 67 instructions a point and sweep in FP64, 51 in FP32 at
+// 257x129x129, of which a useful point takes 37 and 28 (13 of them the IEEE division) and
+// dead entries and overlapped planes the rest.  It is busy for 46 and 38 % of the cycles;
+// between two barriers the wavefronts of a block (four a SIMD in FP64, two in FP32) wait
+// for loads, LDS and each other.  Measured, microseconds for two sweeps, two launches -> a
+// pair:
 //               33x17x17    65^3       97^3       193x97x97  257x129x129 385x193x193
-//   FP64        7.0 ->  4.9 8.8 -> 7.7 12.6 -> 12.2 19.4 -> 16.5 38.4 -> 28.7 164 -> 93.5
-//   FP32        7.8 ->  5.2 8.4 -> 6.4 12.6 -> 10.6 14.4 -> 13.9 24.0 -> 22.4 55.2 -> 51.2
+//   FP64        5.7 ->  4.8 7.7 -> 7.4 11.7 -> 11.5 19.0 -> 15.2 37.7 -> 25.9 163 -> 90.8
+//   FP32        6.6 ->  5.2 7.4 -> 6.2 11.2 -> 10.4 13.3 -> 13.6 22.7 -> 21.6 53.8 -> 50.9
 // A reciprocal shared by the two sweeps with the quotient corrected to the IEEE
 // one costs, with the range checks, as many instructions as it saves.
 // Block function of stretch tw, z chunk bz (the single-case and the batched kernel;

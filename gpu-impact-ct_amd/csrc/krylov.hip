@@ -97,8 +97,8 @@ enum { DOT_NONE = 0, DOT_W = 1, DOT_SELF = 2, DOT_PAIR = 3 };
 //
 // What bounds them: where the tiles do not fill the compute units (65^3 has 75) the
 // chain of one plane, barrier to barrier, which the teams halve; beyond two tiles a
-// compute unit LDS and FP64 issue, each about 40 % busy at 257x129x129, which the
-// waves' waits keep from overlapping further, and there two teams (8 wavefronts, two
+// compute unit the waits of its wavefronts, with the vector ALU 34 to 40 % and LDS 33 to
+// 36 % busy at 257x129x129 (column form), and there two teams (8 wavefronts, two
 // blocks a compute unit) gain nothing over three blocks of 4 wavefronts.  Operator
 // with <Ap, w>, teams against column: 14.0 / 20.5 us at 33x17x17, 17.3 / 25.7 at
 // 65^3, 28.8 / 36.7 at 193x97x97; a whole BiCGstab iteration 108.7 / 122.2 us at

@@ -13,10 +13,13 @@ import oracle_lib as O
 pytestmark = pytest.mark.gpu
 
 W6, PX, PY, PXZ = (1,) * 6, (-1, -1, 1, 1, 1, 1), (1, 1, -1, -1, 1, 1), (-1, -1, 1, 1, -1, -1)
+PZ, PXYZ = (1, 1, 1, 1, -1, -1), (-1,) * 6
 THIN = [((9, 97, 97), PX),      # FP32: 5 x 49 x 49, four points of the range a row
         ((9, 193, 193), PX),    # FP64 too: 3 x 49 x 49, two points a row
         ((17, 129, 129), PXZ),  # 5 x 33 x 33
-        ((9, 129, 161), W6), ((9, 257, 129), PXZ), ((129, 9, 129), PY), ((129, 129, 9), W6)]
+        ((9, 129, 161), W6), ((9, 257, 129), PXZ), ((129, 9, 129), PY), ((129, 129, 9), W6),
+        ((257, 257, 9), PZ),    # 65 x 65 x 3, two planes
+        ((257, 9, 129), PXYZ), ((9, 129, 161), PXYZ)]
 
 
 @pytest.mark.parametrize("fp32", [False, True], ids=["fp64", "fp32"])
